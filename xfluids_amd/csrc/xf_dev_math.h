@@ -26,67 +26,98 @@ __device__ __forceinline__ double sconst(double c)
     return c;
 }
 
-__device__ __forceinline__ double dexp(double x)
+// a / b rounded as IEEE division for operands whose exponents stay clear of
+// the ends of the range: the hardware's own sequence (reciprocal estimate, two
+// Newton steps, quotient, one remainder correction) without the operand
+// scaling and the special-case fix-up around it, which do nothing there.  Eight
+// instructions instead of eleven, and no dependence through the carry register.
+// a = +0 gives +0; callers keep |b| and |a| within [2^-500, 2^500] otherwise.
+__device__ __forceinline__ double ddiv_core(double a, double b)
 {
-    // the reduction runs on x clamped to [-746, 710] (NaN goes to -746), so k
-    // stays in [-1076, 1024]; inputs outside the finite-result range are
-    // replaced at the end
-    const double xc = fmin(fmax(x, -746.0), 710.0);
-    const double kf = (xc * 0x1.71547652b82fep+0 + 0x1.8p52) - 0x1.8p52;
-    const int k = (int)kf;
-    // ln2 = LN2_HI + LN2_LO with LN2_HI the double nearest ln2: the first fma
-    // is exact (|result| < 1/2 and a multiple of 2^-54)
-    double r = fma(-kf, 0x1.62e42fefa39efp-1, xc);
-    r = fma(-kf, 0x1.abc9e3b39803fp-56, r);
+    double y = __builtin_amdgcn_rcp(b);
+    y = fma(y, fma(-b, y, 1.0), y);
+    y = fma(y, fma(-b, y, 1.0), y);
+    const double q = a * y;
+    return fma(fma(-b, q, a), y, q);
+}
+
+// RN(a / b) from y = RN(1 / b): Markstein's corrected quotient, with the same
+// bounds on the operands as ddiv_core
+__device__ __forceinline__ double dquot(double a, double b, double y)
+{
+    const double q = a * y;
+    return fma(fma(-b, q, a), y, q);
+}
+
+// exp of NX arguments at once.  The chains are independent, so their fused
+// steps fill each other's latency, and each coefficient is put into scalar
+// registers once for all of them.  Straight-line: rounding to an integer and
+// scaling by 2^k are one instruction each (v_rndne, v_ldexp, which rounds a
+// subnormal result once, as the two exact factors of the CPU restatement do),
+// and the clamp makes the results outside the finite range come out by
+// themselves (p 2^1024 overflows to +inf, p 2^-1076 rounds to 0).
+template <int NX> __device__ __forceinline__ void dexp_n(const double *x, double *out)
+{
+    double r[NX], p[NX];
+    int k[NX];
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+        const double xc = fmin(fmax(x[i], -746.0), 710.0);
+        const double kf = __builtin_rint(xc * 0x1.71547652b82fep+0);
+        k[i] = (int)kf;
+        // ln2 = LN2_HI + LN2_LO with LN2_HI the double nearest ln2: the first fma
+        // is exact (|result| < 1/2 and a multiple of 2^-54)
+        r[i] = fma(-kf, 0x1.62e42fefa39efp-1, xc);
+        r[i] = fma(-kf, 0x1.abc9e3b39803fp-56, r[i]);
+        p[i] = 0x1.6124613a86d09p-33;
+    }
     // the coefficients are forced into scalar registers right at their use:
     // the fma then reads them from there, where a literal in a vector
     // register per coefficient (hoisted out of loops) would cost two moves
     // and two vector registers each
-    double p = 0x1.6124613a86d09p-33;
-    p = fma(p, r, sconst(0x1.1eed8eff8d898p-29));
-    p = fma(p, r, sconst(0x1.ae64567f544e4p-26));
-    p = fma(p, r, sconst(0x1.27e4fb7789f5cp-22));
-    p = fma(p, r, sconst(0x1.71de3a556c734p-19));
-    p = fma(p, r, sconst(0x1.a01a01a01a01ap-16));
-    p = fma(p, r, sconst(0x1.a01a01a01a01ap-13));
-    p = fma(p, r, sconst(0x1.6c16c16c16c17p-10));
-    p = fma(p, r, sconst(0x1.1111111111111p-7));
-    p = fma(p, r, sconst(0x1.5555555555555p-5));
-    p = fma(p, r, sconst(0x1.5555555555555p-3));
-    p = fma(p, r, 0x1.0p-1);
-    p = fma(p, r, 1.0);
-    p = fma(p, r, 1.0);
-    // 2^k as 2^k1 * 2^k2, both factors normal: the first product is exact and
-    // the second rounds once, also for subnormal results
-    const int k1 = k >> 1, k2 = k - k1;
-    double e = (p * __longlong_as_double((long long)(k1 + 1023) << 52)) *
-               __longlong_as_double((long long)(k2 + 1023) << 52);
-    if (__builtin_expect(!(x >= -745.1332191019412 && x <= 709.782712893384), 0))
-        e = x != x ? x : (x > 0.0 ? __longlong_as_double(0x7ff0000000000000LL) : 0.0);
+    auto step = [&](double c) {
+#pragma unroll
+        for (int i = 0; i < NX; i++) p[i] = fma(p[i], r[i], c);
+    };
+    step(sconst(0x1.1eed8eff8d898p-29));
+    step(sconst(0x1.ae64567f544e4p-26));
+    step(sconst(0x1.27e4fb7789f5cp-22));
+    step(sconst(0x1.71de3a556c734p-19));
+    step(sconst(0x1.a01a01a01a01ap-16));
+    step(sconst(0x1.a01a01a01a01ap-13));
+    step(sconst(0x1.6c16c16c16c17p-10));
+    step(sconst(0x1.1111111111111p-7));
+    step(sconst(0x1.5555555555555p-5));
+    step(sconst(0x1.5555555555555p-3));
+    step(0x1.0p-1);
+    step(1.0);
+    step(1.0);
+#pragma unroll
+    for (int i = 0; i < NX; i++) {
+        const double e = __builtin_amdgcn_ldexp(p[i], k[i]);
+        out[i] = x[i] != x[i] ? x[i] : e;
+    }
+}
+
+__device__ __forceinline__ double dexp(double x)
+{
+    double e;
+    dexp_n<1>(&x, &e);
     return e;
 }
 
-__device__ __forceinline__ double dlog(double x)
+// log of a positive finite x: the hardware's exponent and mantissa split
+// (exact for subnormal x too) in place of the bit operations
+__device__ __forceinline__ double dlog_pos(double x)
 {
-    if (x != x) return x;
-    if (x < 0.0) return __longlong_as_double(0x7ff8000000000000LL);
-    if (x == 0.0) return -__longlong_as_double(0x7ff0000000000000LL);
-    unsigned long long b = (unsigned long long)__double_as_longlong(x);
-    if ((b >> 52) == 0x7ffULL) return x;
-    int e = 0;
-    if ((b >> 52) == 0ULL) {
-        x = x * 0x1.0p54;
-        b = (unsigned long long)__double_as_longlong(x);
-        e = -54;
-    }
-    e += (int)(b >> 52) - 1023;
-    double m = __longlong_as_double((long long)((b & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL));
-    if (m > 0x1.6a09e667f3bcdp+0) {
-        m = m * 0.5;
-        e += 1;
-    }
+    double m = __builtin_amdgcn_frexp_mant(x); // [1/2, 1)
+    int e = __builtin_amdgcn_frexp_exp(x);
+    // m in (sqrt(1/2), sqrt(2)]: doubled, exactly, when m <= sqrt(2) / 2
+    const int lo = m > 0x1.6a09e667f3bcdp-1 ? 0 : 1;
+    m = __builtin_amdgcn_ldexp(m, lo);
+    e -= lo;
     const double f = m - 1.0;
-    const double s = f / (2.0 + f);
+    const double s = ddiv_core(f, 2.0 + f); // 2 + f in [1.7, 2.5), f = 0 or |f| >= 2^-53
     const double z = s * s;
     double R = 0x1.642c8590b2164p-4;
     R = 0x1.8618618618618p-4 + z * R;
@@ -103,6 +134,18 @@ __device__ __forceinline__ double dlog(double x)
     const double t = f - s * (f - R);
     const double ed = (double)e;
     return ed * 0x1.62e42fee00000p-1 + (t + ed * 0x1.a39ef35793c76p-33);
+}
+
+__device__ __forceinline__ double dlog(double x)
+{
+    double v = dlog_pos(x);
+    if (__builtin_expect(!(x > 0.0 && x < __longlong_as_double(0x7ff0000000000000LL)), 0)) {
+        // NaN -> itself, negative -> NaN, zero -> -inf, +inf -> itself
+        v = x;
+        if (x < 0.0) v = __longlong_as_double(0x7ff8000000000000LL);
+        if (x == 0.0) v = -__longlong_as_double(0x7ff0000000000000LL);
+    }
+    return v;
 }
 
 // max/min with the reference's operand semantics on finite data

@@ -12,6 +12,7 @@
 //   UpdateURK3rdKernel         src/solver_UpdateStates/Update_kernels.hpp:64-94
 #pragma once
 #include "xf_thermo.h"
+#include <type_traits>
 
 namespace xf {
 
@@ -268,22 +269,32 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
             const double R_ = mix_R<NS>(th, yi);
             T = get_T<NS>(th, yi, tme, T);
             p = rho * R_ * T;
-            const TPre t = th->thermo ? tpre<true>(T, 1) : tpre<false>(T, 0);
-            // species Cp and h: with the fit range as a wave-uniform value when
-            // every lane shares it (scalar coefficient loads)
+            // species Cp and h at T
             double cpk[NS], hk[NS];
-            auto species = [&](const TPre &tt) {
+            auto species = [&](auto fam) {
+                constexpr bool NASA = decltype(fam)::value;
+                FastT<NASA> ft(th, th->fast, T);
+                cdouble *Rk = as_const(th->Ri);
+                if (ft.ok) {
+                    ft.each(NASA, [&](cdouble *cf) {
 #pragma unroll
-                for (int n = 0; n < NS; n++) cpk[n] = cp_k(th, tt, th->Ri[n], n), hk[n] = h_k(th, tt, th->Ri[n], n);
+                        for (int n = 0; n < NS; n++) {
+                            cpk[n] = cp_fast<NASA>(cf + 9 * n, T, ft.iT, Rk[n]);
+                            hk[n] = h_fast<NASA>(cf + 9 * n, T, ft.iT, ft.lT, Rk[n]);
+                        }
+                    });
+                } else {
+                    const TPre t = tpre<NASA>(T, NASA ? 1 : 0);
+#pragma unroll 1
+                    for (int n = 0; n < NS; n++) {
+                        const double cpn = cp_k(th, t, th->Ri[n], n), hn = h_k(th, t, th->Ri[n], n);
+#pragma unroll
+                        for (int q = 0; q < NS; q++) cpk[q] = q == n ? cpn : cpk[q], hk[q] = q == n ? hn : hk[q];
+                    }
+                }
             };
-            const int r0 = __builtin_amdgcn_readfirstlane(t.r);
-            if (__all(t.r == r0)) {
-                TPre tu = t;
-                tu.r = r0;
-                species(tu);
-            } else {
-                species(t);
-            }
+            if (th->thermo) species(std::true_type{});
+            else species(std::false_type{});
             double Cp = 0.0;
 #pragma unroll
             for (int n = 0; n < NS; n++) Cp += yi[n] * cpk[n];
