@@ -54,16 +54,17 @@ __device__ __forceinline__ double dquot(double a, double b, double y)
 // registers once for all of them.  Straight-line: rounding to an integer and
 // scaling by 2^k are one instruction each (v_rndne, v_ldexp, which rounds a
 // subnormal result once, as the two exact factors of the CPU restatement do),
-// and the clamp makes the results outside the finite range come out by
-// themselves (p 2^1024 overflows to +inf, p 2^-1076 rounds to 0).
+// and the results outside the finite range come out by themselves: below, x is
+// taken at -746, where p 2^-1076 rounds to 0; above, k stays at 1024 while r >= 0
+// grows, so p 2^1024 is +inf; a NaN goes through r.
 template <int NX> __device__ __forceinline__ void dexp_n(const double *x, double *out)
 {
     double r[NX], p[NX];
     int k[NX];
 #pragma unroll
     for (int i = 0; i < NX; i++) {
-        const double xc = fmin(fmax(x[i], -746.0), 710.0);
-        const double kf = __builtin_rint(xc * 0x1.71547652b82fep+0);
+        const double xc = x[i] < -746.0 ? -746.0 : x[i];
+        const double kf = __builtin_rint(fmin(xc, 710.0) * 0x1.71547652b82fep+0);
         k[i] = (int)kf;
         // ln2 = LN2_HI + LN2_LO with LN2_HI the double nearest ln2: the first fma
         // is exact (|result| < 1/2 and a multiple of 2^-54)
@@ -93,10 +94,7 @@ template <int NX> __device__ __forceinline__ void dexp_n(const double *x, double
     step(1.0);
     step(1.0);
 #pragma unroll
-    for (int i = 0; i < NX; i++) {
-        const double e = __builtin_amdgcn_ldexp(p[i], k[i]);
-        out[i] = x[i] != x[i] ? x[i] : e;
-    }
+    for (int i = 0; i < NX; i++) out[i] = __builtin_amdgcn_ldexp(p[i], k[i]);
 }
 
 __device__ __forceinline__ double dexp(double x)

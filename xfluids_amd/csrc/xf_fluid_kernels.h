@@ -50,16 +50,47 @@ __device__ __forceinline__ void xcd_tile(int &tx, int &ty, int &tz)
 }
 
 // ---------------------------------------------------------------------------
-// wave64 max reduction (butterfly over lane permutes) of non-negative doubles
+// wave64 reduction of several doubles at once
 // ---------------------------------------------------------------------------
-// maximum over the wave of magnitudes (>= +0, or NaN): fmax takes two
-// instructions per step where a compare and two selects took three, and it
-// drops a NaN, as the fold of the block maxima does (it keeps only values > 0)
-__device__ __forceinline__ double wave_max(double v)
+// the value of another lane of the same row of 16, by a DPP control code
+template <int CTRL> __device__ __forceinline__ double dpp_f64(double v)
 {
+    const int lo = __double2loint(v), hi = __double2hiint(v);
+    return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xf, 0xf, false),
+                            __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xf, 0xf, false));
+}
+// op(a, a of the other half) on lanes 0-31 and op(b, b of the other half) on
+// lanes 32-63 (HALF), or the same on the even and odd rows of 16: one swap
+// instruction per dword exchanges for both values
+template <bool HALF, class Op> __device__ __forceinline__ double swap_fold(double a, double b, Op op)
+{
+    const unsigned al = __double2loint(a), ah = __double2hiint(a), bl = __double2loint(b), bh = __double2hiint(b);
+    const auto lo = HALF ? __builtin_amdgcn_permlane32_swap(al, bl, false, false)
+                         : __builtin_amdgcn_permlane16_swap(al, bl, false, false);
+    const auto hi = HALF ? __builtin_amdgcn_permlane32_swap(ah, bh, false, false)
+                         : __builtin_amdgcn_permlane16_swap(ah, bh, false, false);
+    return op(__hiloint2double((int)hi[0], (int)lo[0]), __hiloint2double((int)hi[1], (int)lo[1]));
+}
+// op (a maximum or minimum: associative and idempotent) over the wave of each
+// of the N values in v, N a multiple of 4.  The first two steps halve the number
+// of values instead of reducing each on its own; the last four stay within rows
+// of 16.  12 values take 63 vector instructions and no LDS, where a butterfly of
+// lane permutes per value took 216 and 144 LDS permutes.  out[j] of row
+// q = lane / 16 holds the result of value wave_fold_index(j, q).
+__device__ __forceinline__ int wave_fold_index(int j, int row) { return 4 * j + ((row & 1) << 1) + (row >> 1); }
+template <int N, class Op> __device__ __forceinline__ void wave_fold(const double *v, double *out, Op op)
+{
+    static_assert(N % 4 == 0, "pad to a multiple of 4");
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmax(v, __shfl_xor(v, off, 64));
-    return v;
+    for (int j = 0; j < N / 4; j++) {
+        double m = swap_fold<false>(swap_fold<true>(v[4 * j], v[4 * j + 1], op),
+                                    swap_fold<true>(v[4 * j + 2], v[4 * j + 3], op), op);
+        m = op(m, dpp_f64<0xB1>(m));  // lane ^ 1
+        m = op(m, dpp_f64<0x4E>(m));  // lane ^ 2
+        m = op(m, dpp_f64<0x141>(m)); // mirror of 8 lanes: the other quad
+        m = op(m, dpp_f64<0x140>(m)); // mirror of the row: the other 8 lanes
+        out[j] = m;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -371,20 +402,18 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     if (threadIdx.x == 0) serr = 0;
     __syncthreads();
-    // the directions the case has (the others stay +0)
-    const int dimv[3] = {g.DimX, g.DimY, g.DimZ};
+    // maxima of magnitudes (>= +0, or NaN): fmax drops a NaN, as the fold of the
+    // block maxima does (it keeps only values > 0); directions the case does not
+    // have stay +0
+    double v12[12], m3[3];
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        if (!dimv[d]) continue;
+    for (int q = 0; q < 9; q++) v12[q] = glf[q];
 #pragma unroll
-        for (int q = 0; q < 3; q++) glf[3 * d + q] = wave_max(glf[3 * d + q]);
-        dtm[d] = wave_max(dtm[d]);
-    }
-    if (lane == 0) {
+    for (int q = 0; q < 3; q++) v12[9 + q] = dtm[q];
+    wave_fold<12>(v12, m3, [](double a, double b) { return fmax(a, b); });
+    if ((lane & 15) == 0) {
 #pragma unroll
-        for (int q = 0; q < 9; q++) sred[wv][q] = glf[q];
-#pragma unroll
-        for (int q = 0; q < 3; q++) sred[wv][9 + q] = dtm[q];
+        for (int j = 0; j < 3; j++) sred[wv][wave_fold_index(j, lane >> 4)] = m3[j];
     }
     if (ebits) {
         atomicOr(&serr, ebits);
