@@ -157,13 +157,157 @@ __device__ __forceinline__ void transport_mixed(const DevThermo *__restrict__ th
     }
 }
 
-// Waves per SIMD k_transport is compiled for (1: no bound).  Unbounded, the
-// FP64 form at nine species takes 194 registers and runs two waves per SIMD,
-// with the FP64 divisions, square roots and exponentials waiting on each
-// other; held to three waves (168 registers, 96 bytes per lane spilled) it
-// takes 15 % less time, and four waves (256 bytes spilled) gain nothing more.
-// At ten and eleven species a three-wave bound spills 272 and 432 bytes, and
-// the mixed form already runs five waves.
+// Fixes a value's place in program order (against the others so marked and the
+// exponentials' coefficient loads).  In one long basic block the compiler
+// otherwise starts every independent chain early and spills the results.
+__device__ __forceinline__ double in_order(double v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
+// exp of the cubic fits of NX rows at once (rows of 4 coefficients, stride st),
+// folding the largest |argument| into amax
+template <int NX> __device__ __forceinline__ void fit_exps(const double *a, int st, double lT, double *out, double &amax)
+{
+    double x[NX];
+    lT = in_order(lT);
+#pragma unroll
+    for (int i = 0; i < NX; i++) x[i] = fit4(a + st * i, lT), amax = fmax(amax, fabs(x[i]));
+    dexp_n<NX>(x, out);
+}
+
+// The FP64 transport coefficients of one cell: Wilke mixture viscosity and
+// conductivity (the conductivity uses the viscosity's denominators, as
+// Visc_device.h:121-134 does) and the mixture-averaged D_km.  FAST takes the
+// quotients and square roots in the forms that are IEEE's only away from the
+// ends of the exponent range, and returns false without storing anything when
+// some lane's fits, pressure or mole fractions are not well inside it; the
+// general form then computes the cell.  With |fit| <= 200 every exponential lies
+// within 2^+-289, and with |X|, p and rho within 2^+-300 no operand of a
+// shortcut leaves 2^+-700.  The launch is bound by FP64 issue: some 5000
+// instructions per cell at nine species where the range checks, the scaling around
+// each square root and quotient and the longer exponentials took 7000, in one
+// stretch of 52 KB of code (110 KB with 466 branches before, over the instruction
+// cache) and without scratch memory.  With k_vel_deriv, 783 -> 545 us on a 136^3
+// grid.
+template <int NS, bool FAST>
+__device__ __forceinline__ bool transport_fp64(const DevThermo *__restrict__ th, const DevTransport *__restrict__ tr,
+                                               Fields &f, long long id, long long N, const double *X, double C_total,
+                                               double rho, double rho1, double p, double lT, int heat, int diffu)
+{
+    constexpr int NG = NS % 3 == 0 ? 3 : (NS % 2 == 0 ? 2 : 1); // exponentials evaluated together
+    auto quot = [](double a, double b, double y) { return FAST ? dquot(a, b, y) : qdiv(a, b, y); };
+    double amax = 0.0, xmax = 0.0;
+    // 2 sqrt(2) and its reciprocal: (phi + 1)^2 0.5 / sqrt(2), the halving
+    // (exact) taken with the divisor; folded at compile time, and the corrected
+    // quotient is the IEEE one bit for bit
+    const double s2 = sqrt(2.0), rs2 = 1.0 / s2;
+    double mu[NS], rmu[NS];
+#pragma unroll
+    for (int k = 0; k < NS; k += NG) fit_exps<NG>(tr->fcv + 4 * k, 4, lT, mu + k, amax);
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+        rmu[k] = FAST ? ddiv_core(1.0, mu[k]) : 1.0 / mu[k];
+        xmax = fmax(xmax, fabs(X[k]));
+    }
+    if (FAST && !__all(amax <= 200.0 && xmax <= 0x1p300 && p >= 0x1p-300 && p <= 0x1p300 && rho >= 0x1p-300 &&
+                       rho <= 0x1p300))
+        return false;
+    double va = 0.0, tca = 0.0;
+#pragma unroll
+    for (int k0 = 0; k0 < NS; k0 += NG) {
+        double la[NG];
+        if (heat) fit_exps<NG>(tr->fct + 4 * k0, 4, lT, la, amax);
+#pragma unroll
+        for (int k = k0; k < k0 + NG; k++) {
+            double den = 0.0;
+            const double muk = in_order(mu[k]);
+#pragma unroll
+            for (int i = 0; i < NS; i++) {
+                double phi;
+                if (i == k) {
+                    // RN(mu_k / mu_k) = 1 wherever qdiv's correction holds (it
+                    // returns exactly 1 for a = b), and sqrt(1) = 1: the product
+                    // is phiA itself; elsewhere the IEEE quotient, as qdiv takes
+                    phi = tr->phiA[k * MAXNS + i];
+                    if (!FAST) {
+                        const double am = fabs(mu[k]);
+                        if (__builtin_expect(!(am >= 0x1p-500 && am <= 0x1p500), 0))
+                            phi = phi * sqrt(ieee_div(mu[k], mu[k]));
+                    }
+                } else {
+                    const double m = quot(muk, mu[i], rmu[i]);
+                    phi = tr->phiA[k * MAXNS + i] * (FAST ? dsqrt_core(m) : sqrt(m));
+                }
+                phi = FAST ? dquot((phi + 1.0) * (phi + 1.0), 2.0 * s2, 0.5 * rs2)
+                           : qdiv((phi + 1.0) * (phi + 1.0) * 0.5, s2, rs2);
+                phi = phi * tr->phiB[k * MAXNS + i];
+                den = den + X[i] * phi;
+            }
+            const double _den = 1.0 / den;
+            va = va + X[k] * mu[k] * _den;
+            if (heat) tca = tca + X[k] * la[k - k0] * _den;
+            va = in_order(va), tca = in_order(tca);
+        }
+    }
+    double D[NS];
+    if (diffu) {
+        // mixture-averaged D_km: temp2[k] = 1e-20 + sum_{i != k, i ascending}
+        // (X_i + 1e-40) / (D_ik + 1e-40), with D_ik = exp(fit(ln T)) / p.
+        // The fits are symmetric (Setup copies the lower triangle from the
+        // upper), so each pair's exponential serves both species.
+        double t2[NS];
+        const double rp = FAST ? ddiv_core(1.0, p) : 1.0 / p;
+#pragma unroll
+        for (int k = 0; k < NS; k++) t2[k] = 1.0e-20;
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            auto pair = [&](int i, double e) {
+                const double De = quot(e, p, rp) + 1.0e-40, rDe = FAST ? ddiv_core(1.0, De) : 1.0 / De;
+                t2[k] += quot(X[i] + 1.0e-40, De, rDe);
+                t2[i] += quot(X[k] + 1.0e-40, De, rDe);
+                t2[k] = in_order(t2[k]), t2[i] = in_order(t2[i]);
+            };
+#pragma unroll
+            for (int i = 0; i + 1 < k; i += 2) {
+                double e[2];
+                fit_exps<2>(tr->Dkj + 4 * (i * MAXNS + k), 4 * MAXNS, lT, e, amax);
+                pair(i, e[0]), pair(i + 1, e[1]);
+            }
+            if (k % 2 == 1) {
+                double e;
+                fit_exps<1>(tr->Dkj + 4 * ((k - 1) * MAXNS + k), 4 * MAXNS, lT, &e, amax);
+                pair(k - 1, e);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NS; k++) {
+            double t1 = 0.0;
+#pragma unroll
+            for (int i = 0; i < NS; i++)
+                if (i != k) t1 += (X[i] + 1.0e-40) * th->Wi[i];
+            if (t1 <= 0.0) // sycl::step(ceil(temp1), 0)
+                D[k] = dexp(fit4(tr->Dkj + 4 * (k * MAXNS + k), lT)) / p;
+            else
+                D[k] = qdiv(t1 / t2[k], rho, rho1) * C_total;
+            D[k] *= 1.0e-1;
+        }
+    }
+    if (FAST && !__all(amax <= 200.0)) return false;
+    f.mu[id] = va;
+    if (heat) f.kap[id] = tca;
+    if (diffu) {
+#pragma unroll
+        for (int k = 0; k < NS; k++) f.Dkm[k * N + id] = smax(D[k], 1.0e-10);
+    }
+    return true;
+}
+
+// Waves per SIMD k_transport is compiled for (1: no bound): the FP64 form at nine
+// species fits three (161 registers, nothing spilled) and is held there; with ten
+// and eleven it takes 186 and 216 and runs two, with fewer species and in the
+// mixed form five or more.
 template <int NS, int PREC> struct TransportOccupancy {
     static constexpr int waves = (PREC == 0 && NS == 9) ? 3 : 1;
 };
@@ -213,24 +357,30 @@ k_transport(Geom g, const DevThermo *__restrict__ th, const DevTransport *__rest
             for (int i = 0; i < NS; i++) X[i] = X[i] * _C_total;
         }
         if (diffu) {
-            // interior cells' min / max of each mass fraction: wave shuffles,
-            // then the block's four waves in LDS (other cells contribute 0.0,
-            // the value the reference's reduction combines with)
+            // interior cells' min / max of each mass fraction: within each
+            // wave, then the block's four waves in LDS (other cells contribute
+            // 0.0, the value the reference's reduction combines with)
             int i = 0, j = 0, kk = 0;
             if (live) cell_ijk(g, id, i, j, kk);
             const bool in = live && i >= g.Bx && i < g.Xmax - g.Bx && j >= g.By && j < g.Ymax - g.By &&
                             kk >= g.Bz && kk < g.Zmax - g.Bz;
-            __shared__ double sm[4][2 * NS];
-            const int wv = threadIdx.x >> 6;
+            // (a state whose fractions are NaN does not get here: UpdateStates
+            // halts the step); the maxima as minima of the negated values
+            constexpr int NV = (2 * NS + 3) / 4 * 4;
+            __shared__ double sm[4][NV];
+            double v[NV], m[NV / 4];
 #pragma unroll
-            for (int k = 0; k < NS; k++) {
-                double a = in ? yi[k] : 0.0, b = a;
+            for (int k = 0; k < NV; k++) v[k] = 0.0;
 #pragma unroll
-                for (int off = 32; off >= 1; off >>= 1) {
-                    a = smin(a, __shfl_xor(a, off, 64));
-                    b = smax(b, __shfl_xor(b, off, 64));
+            for (int k = 0; k < NS; k++) v[k] = in ? yi[k] : 0.0, v[NS + k] = -v[k];
+            wave_fold<NV>(v, m, [](double a, double b) { return fmin(a, b); });
+            const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+            if ((lane & 15) == 0) {
+#pragma unroll
+                for (int j = 0; j < NV / 4; j++) {
+                    const int q = wave_fold_index(j, lane >> 4);
+                    sm[wv][q] = q < NS ? m[j] : -m[j];
                 }
-                if ((threadIdx.x & 63) == 0) sm[wv][k] = a, sm[wv][NS + k] = b;
             }
             __syncthreads();
             if (threadIdx.x < 2 * NS) {
@@ -247,75 +397,11 @@ k_transport(Geom g, const DevThermo *__restrict__ th, const DevTransport *__rest
         transport_mixed<NS>(th, tr, f, id, N, X, C_total, rho, rho1, p, lT, heat, diffu);
         return;
     }
-    // Wilke mixture viscosity and conductivity (the conductivity uses the
-    // viscosity's denominators, as Visc_device.h:121-134 does)
-    double mu[NS], rmu[NS];
-#pragma unroll
-    for (int k = 0; k < NS; k++) mu[k] = dexp(fit4(tr->fcv + 4 * k, lT)), rmu[k] = 1.0 / mu[k];
-    double va = 0.0, tca = 0.0;
-    // the quotients by sqrt(2) take the corrected reciprocal of that constant
-    // (folded at compile time), which is the IEEE quotient bit for bit
-    const double s2 = sqrt(2.0), rs2 = 1.0 / s2;
-#pragma unroll
-    for (int k = 0; k < NS; k++) {
-        double den = 0.0;
-#pragma unroll
-        for (int i = 0; i < NS; i++) {
-            double phi;
-            if (i == k) {
-                // RN(mu_k / mu_k) = 1 wherever qdiv's correction holds (it
-                // returns exactly 1 for a = b), and sqrt(1) = 1: the product
-                // is phiA itself; elsewhere the IEEE quotient, as qdiv takes
-                const double am = fabs(mu[k]);
-                phi = tr->phiA[k * MAXNS + i];
-                if (__builtin_expect(!(am >= 0x1p-500 && am <= 0x1p500), 0)) phi = phi * sqrt(ieee_div(mu[k], mu[k]));
-            } else {
-                phi = tr->phiA[k * MAXNS + i] * sqrt(qdiv(mu[k], mu[i], rmu[i]));
-            }
-            phi = qdiv((phi + 1.0) * (phi + 1.0) * 0.5, s2, rs2);
-            phi = phi * tr->phiB[k * MAXNS + i];
-            den = den + X[i] * phi;
-        }
-        const double _den = 1.0 / den;
-        va = va + X[k] * mu[k] * _den;
-        if (heat) tca = tca + X[k] * dexp(fit4(tr->fct + 4 * k, lT)) * _den;
-    }
-    f.mu[id] = va;
-    if (heat) f.kap[id] = tca;
-    if (diffu) {
-        // mixture-averaged D_km: temp2[k] = 1e-20 + sum_{i != k, i ascending}
-        // (X_i + 1e-40) / (D_ik + 1e-40), with D_ik = exp(fit(ln T)) / p.
-        // The fits are symmetric (Setup copies the lower triangle from the
-        // upper), so each pair's exponential serves both species.
-        double t2[NS];
-        const double rp = 1.0 / p;
-#pragma unroll
-        for (int k = 0; k < NS; k++) t2[k] = 1.0e-20;
-#pragma unroll
-        for (int k = 0; k < NS; k++) {
-#pragma unroll
-            for (int i = 0; i < k; i++) {
-                const double D = qdiv(dexp(fit4(tr->Dkj + 4 * (i * MAXNS + k), lT)), p, rp);
-                const double De = D + 1.0e-40, rDe = 1.0 / De;
-                t2[k] += qdiv(X[i] + 1.0e-40, De, rDe);
-                t2[i] += qdiv(X[k] + 1.0e-40, De, rDe);
-            }
-        }
-#pragma unroll
-        for (int k = 0; k < NS; k++) {
-            double t1 = 0.0;
-#pragma unroll
-            for (int i = 0; i < NS; i++)
-                if (i != k) t1 += (X[i] + 1.0e-40) * th->Wi[i];
-            double D;
-            if (t1 <= 0.0) // sycl::step(ceil(temp1), 0)
-                D = dexp(fit4(tr->Dkj + 4 * (k * MAXNS + k), lT)) / p;
-            else
-                D = qdiv(t1 / t2[k], rho, rho1) * C_total;
-            D *= 1.0e-1;
-            f.Dkm[k * N + id] = smax(D, 1.0e-10);
-        }
-    }
+    if (transport_fp64<NS, true>(th, tr, f, id, N, X, C_total, rho, rho1, p, lT, heat, diffu)) return;
+    // a value of its own, so that nothing of the first attempt is kept for this one
+    double lT2 = lT;
+    asm volatile("" : "+v"(lT2));
+    transport_fp64<NS, false>(th, tr, f, id, N, X, C_total, rho, rho1, p, lT2, heat, diffu);
 }
 
 // the per-block partials of k_transport into red[RED_YMIN + k] (min) and
