@@ -29,6 +29,10 @@ HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-I", os.path.join(ROOT, "include")]
 HIP_SOURCES = ["csrc/xf_api.hip", "csrc/xf_ops_ns1.hip", "csrc/xf_ops_ns2.hip", "csrc/xf_ops_ns3.hip",
                "csrc/xf_ops_ns4.hip", "csrc/xf_ops_ns5.hip", "csrc/xf_ops_ns9.hip", "csrc/xf_ops_ns10.hip",
                "csrc/xf_ops_ns11.hip", "csrc/xf_dt_flow.hip"]
+# the sweeps, one object per species count and scheme, the longest first
+SWEEP_SOURCE = "csrc/xf_sweeps.hip"
+SWEEP_SPECIES = [11, 10, 9, 5, 4, 3, 2, 1]
+SWEEP_SCHEMES = [2, 1, 0]  # XF_WENOCU6, XF_WENO5Z, XF_WENO5JS
 HOST_SOURCES = ["host/xf_json.cpp", "host/xf_setup.cpp", "host/xf_initial.cpp", "host/xf_transport.cpp",
                 "host/xf_host.cpp"]
 
@@ -47,6 +51,11 @@ def build_library(verbose=False):
     gen_mech.generate()
     os.makedirs(OBJ, exist_ok=True)
     jobs = []
+    for ns in SWEEP_SPECIES:
+        for sch in SWEEP_SCHEMES:
+            o = os.path.join(OBJ, "xf_sweeps_ns%d_%d.o" % (ns, sch))
+            jobs.append([HIPCC] + HIP_FLAGS + ["-DXF_NS=%d" % ns, "-DXF_SCH=%d" % sch, "-c",
+                                               os.path.join(PKG, SWEEP_SOURCE), "-o", o])
     for s in HIP_SOURCES:
         o = os.path.join(OBJ, os.path.basename(s) + ".o")
         jobs.append([HIPCC] + HIP_FLAGS + ["-c", os.path.join(PKG, s), "-o", o])

@@ -419,7 +419,9 @@ int xf_set_thermo(xf_ctx *c, const double *Hia, const double *Hib, const double 
     c->h_th.thermo = c->d.thermo;
     // the range in which the kernels' corrected quotients are exact
     auto plain = [](double v) { return v == 0.0 || (std::fabs(v) >= 0x1p-300 && std::fabs(v) <= 0x1p300); };
-    c->h_th.fast = std::all_of(Hia, Hia + NS * 21, plain) && std::all_of(Hib, Hib + NS * 6, plain);
+    auto near1 = [](double v) { return v >= 0x1p-80 && v <= 0x1p80; };
+    c->h_th.fast = std::all_of(Hia, Hia + NS * 21, plain) && std::all_of(Hib, Hib + NS * 6, plain) &&
+                   std::all_of(Wi, Wi + NS, near1);
     XF_HIP(hipMemcpy(c->d_th, &c->h_th, sizeof(DevThermo), hipMemcpyHostToDevice));
     c->thermo_set = true;
     return XF_OK;

@@ -1,7 +1,8 @@
 // Context of one case and the per-species-count kernel dispatch table,
 // shared by the C-ABI translation unit (xf_api.hip) and the translation units
 // that instantiate the kernels for each compile-time species count
-// (xf_ops_ns*.hip), so that those compile in parallel.
+// (xf_ops_ns*.hip, and xf_sweeps.hip per count and scheme), so that those compile
+// in parallel.
 #pragma once
 #include "xf_sweep_kernels.h"
 #include "xf_chem_kernels.h"
@@ -162,6 +163,16 @@ struct ProfScope {
     }
 };
 
+// Launches of the sweeps of one species count and scheme (every direction,
+// precision form and tile shape): defined in xf_sweeps.hip, which the build
+// compiles once per pair, so that the many instances compile in parallel
+template <int NS, bool COP, int SCH> struct SweepLaunch {
+    static void sweep(xf_ctx *c, int dir, const double *Ug, int mode, int stage, const double *Ua, const double *Ub,
+                      double *Uo);
+    static void multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks, int dir,
+                      int shape, int mode, int stage, int sg, int sa, int sb, int so);
+};
+
 template <int NS, bool COP> struct Launch {
     static void states(xf_ctx *c, double *U, int full, int bcs, int where)
     {
@@ -176,55 +187,12 @@ template <int NS, bool COP> struct Launch {
         hipLaunchKernelGGL(k_states_fold, dim3(12), dim3(1024), 0, c->stream, c->f.spart, (int)nblk(c->N), c->f.red,
                            c->f.err);
     }
-    template <int DIR, int SCH, int PREC, int SHAPE>
-    static void sweep_t(xf_ctx *c, const double *Ug, int mode, int stage, const double *Ua, const double *Ub, double *Uo)
-    {
-        constexpr int E = COP ? NS + 4 : 5;
-        static_assert(SweepShape<DIR, E, SHAPE>::TS == (DIR == 0 ? (SHAPE == 0 ? 64 : 32)
-                                                                 : (SHAPE == 0 ? 16 : (SHAPE == 1 ? 32 : 8))),
-                      "sweep_grid's tile sizes");
-        unsigned gr[3];
-        sweep_grid(c->g, DIR, SHAPE, gr);
-        const dim3 grid(gr[0], gr[1], gr[2]);
-        static const char *names[3] = {"sweep_x", "sweep_y", "sweep_z"};
-        ProfScope ps(c, names[DIR]);
-        hipLaunchKernelGGL((k_sweep<NS, COP, DIR, SCH, PREC, SHAPE>), grid, dim3(256), 0, c->stream, c->g, c->d_th,
-                           Ug, c->f, c->d.ncop_gamma, mode, stage, Ua, Ub, Uo);
-    }
-    template <int DIR, int SCH, int PREC>
-    static void sweep_s_(xf_ctx *c, const double *Ug, int mode, int stage, const double *Ua, const double *Ub, double *Uo)
-    {
-        switch (c->shape[DIR]) {
-        case 1: sweep_t<DIR, SCH, PREC, 1>(c, Ug, mode, stage, Ua, Ub, Uo); break;
-        case 2:
-            if constexpr (SweepShapes<DIR>::count > 2) {
-                sweep_t<DIR, SCH, PREC, 2>(c, Ug, mode, stage, Ua, Ub, Uo);
-                break;
-            }
-            [[fallthrough]];
-        default: sweep_t<DIR, SCH, PREC, 0>(c, Ug, mode, stage, Ua, Ub, Uo);
-        }
-    }
-    template <int DIR, int PREC>
-    static void sweep_p(xf_ctx *c, const double *Ug, int mode, int stage, const double *Ua, const double *Ub, double *Uo)
-    {
-        if (c->d.scheme == XF_WENO5Z) sweep_s_<DIR, XF_WENO5Z, PREC>(c, Ug, mode, stage, Ua, Ub, Uo);
-        else if (c->d.scheme == XF_WENOCU6) sweep_s_<DIR, XF_WENOCU6, PREC>(c, Ug, mode, stage, Ua, Ub, Uo);
-        else sweep_s_<DIR, XF_WENO5JS, PREC>(c, Ug, mode, stage, Ua, Ub, Uo);
-    }
-    template <int DIR>
-    static void sweep_d(xf_ctx *c, const double *Ug, int mode, int stage, const double *Ua, const double *Ub, double *Uo)
-    {
-        if (c->d.precision == XF_MIXED) sweep_p<DIR, XF_MIXED>(c, Ug, mode, stage, Ua, Ub, Uo);
-        else if (c->d.precision == XF_FUSED_FP64) sweep_p<DIR, XF_FUSED_FP64>(c, Ug, mode, stage, Ua, Ub, Uo);
-        else sweep_p<DIR, XF_PLAIN_FP64>(c, Ug, mode, stage, Ua, Ub, Uo);
-    }
     static void sweep(xf_ctx *c, int dir, const double *Ug, int mode, int stage, const double *Ua, const double *Ub,
                       double *Uo)
     {
-        if (dir == 0) sweep_d<0>(c, Ug, mode, stage, Ua, Ub, Uo);
-        if (dir == 1) sweep_d<1>(c, Ug, mode, stage, Ua, Ub, Uo);
-        if (dir == 2) sweep_d<2>(c, Ug, mode, stage, Ua, Ub, Uo);
+        if (c->d.scheme == XF_WENO5Z) SweepLaunch<NS, COP, XF_WENO5Z>::sweep(c, dir, Ug, mode, stage, Ua, Ub, Uo);
+        else if (c->d.scheme == XF_WENOCU6) SweepLaunch<NS, COP, XF_WENOCU6>::sweep(c, dir, Ug, mode, stage, Ua, Ub, Uo);
+        else SweepLaunch<NS, COP, XF_WENO5JS>::sweep(c, dir, Ug, mode, stage, Ua, Ub, Uo);
     }
     // calls f(std::integral_constant<int, K>) for the compiled mechanism K
     // == spec if one exists for this species count, else with K = -1 (the
@@ -390,56 +358,15 @@ template <int NS, bool COP> struct Launch {
                            c0->d.ncop_gamma, full, fill, where, sel);
         hipLaunchKernelGGL(k_states_fold_multi, dim3((unsigned)(12 * ncases)), dim3(1024), 0, st, cases);
     }
-    template <int DIR, int SCH, int PREC, int SHAPE>
-    static void sweep_multi_t(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
-                              int mode, int stage, int sg, int sa, int sb, int so)
-    {
-        hipLaunchKernelGGL((k_sweep_multi<NS, COP, DIR, SCH, PREC, SHAPE>), dim3((unsigned)blocks), dim3(256), 0, st,
-                           cases, ncases, c0->d_th, c0->d.ncop_gamma, mode, stage, sg, sa, sb, so);
-    }
-    template <int DIR, int SCH, int PREC>
-    static void sweep_multi_s(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
-                              int shape, int mode, int stage, int sg, int sa, int sb, int so)
-    {
-        switch (shape) {
-        case 1: sweep_multi_t<DIR, SCH, PREC, 1>(c0, st, cases, ncases, blocks, mode, stage, sg, sa, sb, so); break;
-        case 2:
-            if constexpr (SweepShapes<DIR>::count > 2) {
-                sweep_multi_t<DIR, SCH, PREC, 2>(c0, st, cases, ncases, blocks, mode, stage, sg, sa, sb, so);
-                break;
-            }
-            [[fallthrough]];
-        default: sweep_multi_t<DIR, SCH, PREC, 0>(c0, st, cases, ncases, blocks, mode, stage, sg, sa, sb, so);
-        }
-    }
-    template <int DIR, int PREC>
-    static void sweep_multi_p(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
-                              int shape, int mode, int stage, int sg, int sa, int sb, int so)
-    {
-        if (c0->d.scheme == XF_WENO5Z)
-            sweep_multi_s<DIR, XF_WENO5Z, PREC>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        else if (c0->d.scheme == XF_WENOCU6)
-            sweep_multi_s<DIR, XF_WENOCU6, PREC>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        else
-            sweep_multi_s<DIR, XF_WENO5JS, PREC>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-    }
-    template <int DIR>
-    static void sweep_multi_d(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
-                              int shape, int mode, int stage, int sg, int sa, int sb, int so)
-    {
-        if (c0->d.precision == XF_MIXED)
-            sweep_multi_p<DIR, XF_MIXED>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        else if (c0->d.precision == XF_FUSED_FP64)
-            sweep_multi_p<DIR, XF_FUSED_FP64>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        else
-            sweep_multi_p<DIR, XF_PLAIN_FP64>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-    }
     static void sweep_multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
                             int dir, int shape, int mode, int stage, int sg, int sa, int sb, int so)
     {
-        if (dir == 0) sweep_multi_d<0>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        if (dir == 1) sweep_multi_d<1>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
-        if (dir == 2) sweep_multi_d<2>(c0, st, cases, ncases, blocks, shape, mode, stage, sg, sa, sb, so);
+        if (c0->d.scheme == XF_WENO5Z)
+            SweepLaunch<NS, COP, XF_WENO5Z>::multi(c0, st, cases, ncases, blocks, dir, shape, mode, stage, sg, sa, sb, so);
+        else if (c0->d.scheme == XF_WENOCU6)
+            SweepLaunch<NS, COP, XF_WENOCU6>::multi(c0, st, cases, ncases, blocks, dir, shape, mode, stage, sg, sa, sb, so);
+        else
+            SweepLaunch<NS, COP, XF_WENO5JS>::multi(c0, st, cases, ncases, blocks, dir, shape, mode, stage, sg, sa, sb, so);
     }
     static Ops ops()
     {

@@ -23,7 +23,7 @@ struct DevThermo {
     double Hc[3 * MAXNS * 9];
     double Wi[MAXNS], _Wi[MAXNS], Ri[MAXNS];
     int thermo; // 1 NASA-9, 0 JANAF
-    int fast;   // every coefficient is 0 or within [2^-300, 2^300] (xf_set_thermo)
+    int fast;   // every coefficient is 0 or within [2^-300, 2^300], every W within [2^-80, 2^80] (xf_set_thermo)
 };
 
 // One reaction as the rate kernel reads it: Arrhenius A, B and

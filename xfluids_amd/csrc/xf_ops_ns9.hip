@@ -1,7 +1,6 @@
-// Kernel instances for 9 species: sweeps (every direction, scheme,
-// precision form and tile shape), states and chemistry, and their dispatch
-// table.  One translation unit per species count so the build runs them in
-// parallel.
+// Kernel instances for 9 species other than the sweeps (xf_sweeps.hip): states,
+// viscous terms and chemistry, and the dispatch table.  One translation unit per
+// species count so the build runs them in parallel.
 #include "xf_context.h"
 
 namespace xf {

@@ -29,6 +29,14 @@
 //  * structurally-zero eigenvector entries are skipped: the reference adds
 //    +/-0 products to an accumulator that starts at +0.0 and is never -0.0
 //    afterwards, so skipping them leaves every sum bit-identical;
+//  * the rows of one face are straight-line code with the row's species, sign and
+//    flux component known at compile time, and rows u-c and u+c share their LDS
+//    reads and products.  What bounds it is FP64 issue (0.70-0.76 of the launch in
+//    x and y at nine species, two waves per SIMD) and, in z and the wall flux,
+//    memory latency; a runtime loop over the species rows spent a fifth of its
+//    instructions on selects.  At 128^3, nine species, WENO5-JS, viscous:
+//    709 / 687 / 766 us per launch (x, y, z) before, 544 / 541 / 637 now; three
+//    species, WENO5-Z, 1024 x 512: 93 / 97 before, 75 / 79 now;
 //  * the TS face fluxes go back to LDS and the TS-1 interior cells of the
 //    tile form LU = (F_{i-1/2} - F_{i+1/2}) / dx in the reference's direction
 //    order (x, then y, then z), optionally fused with the SSP-RK3 stage.
@@ -59,22 +67,26 @@ __device__ __forceinline__ int lds_ix(int ls, int tcol)
     return DIR == 0 ? tcol * (TS + 5) + ls : ls * TW + tcol;
 }
 
+// Products by 2 and 4 are exact, so the bodies below fuse them with the addition
+// that follows them: the reference's bits, eight multiplications less each.
+
 // WENO5-JS body (weno5old_BODY, USE_DOUBLE branch)
 __device__ __forceinline__ double weno5js_body(double v1, double v2, double v3, double v4, double v5)
 {
     double a1, a2, a3;
-    const double dtwo = 2.0, dtre = 3.0;
-    a1 = v1 - dtwo * v2 + v3;
+    const double dtre = 3.0;
+    const double t3 = dtre * v3;
+    a1 = fma(-2.0, v2, v1) + v3;
     double s1 = 13.0 * a1 * a1;
-    a1 = v1 - 4.0 * v2 + dtre * v3;
+    a1 = fma(-4.0, v2, v1) + t3;
     s1 += dtre * a1 * a1;
-    a1 = v2 - dtwo * v3 + v4;
+    a1 = fma(-2.0, v3, v2) + v4;
     double s2 = 13.0 * a1 * a1;
     a1 = v2 - v4;
     s2 += dtre * a1 * a1;
-    a1 = v3 - dtwo * v4 + v5;
+    a1 = fma(-2.0, v4, v3) + v5;
     double s3 = 13.0 * a1 * a1;
-    a1 = dtre * v3 - 4.0 * v4 + v5;
+    a1 = fma(-4.0, v4, t3) + v5;
     s3 += dtre * a1 * a1;
     const double tol = 1.0E-6;
     s1 += tol, s2 += tol, s3 += tol;
@@ -83,9 +95,9 @@ __device__ __forceinline__ double weno5js_body(double v1, double v2, double v3, 
     a3 = 0.3 * s1 * s1 * s2 * s2;
     const double tw1 = 1.0 / (a1 + a2 + a3);
     a1 = a1 * tw1, a2 = a2 * tw1, a3 = a3 * tw1;
-    s1 = a1 * (dtwo * v1 - 7.0 * v2 + 11.0 * v3);
-    s2 = a2 * (-v2 + 5.0 * v3 + dtwo * v4);
-    s3 = a3 * (dtwo * v3 + 5.0 * v4 - v5);
+    s1 = a1 * (fma(2.0, v1, -(7.0 * v2)) + 11.0 * v3);
+    s2 = a2 * fma(2.0, v4, 5.0 * v3 - v2);
+    s3 = a3 * (fma(2.0, v3, 5.0 * v4) - v5);
     return (s1 + s2 + s3);
 }
 
@@ -140,15 +152,16 @@ __device__ __forceinline__ double weno5z_body(double v1, double v2, double v3, d
         p2 = fma(2.0, v4, fma(5.0, v3, -v2));
         p3 = fma(5.0, v4, 2.0 * v3) - v5;
     } else {
-        const double d1 = v1 - 2.0 * v2 + v3, e1 = v1 - 4.0 * v2 + 3.0 * v3;
-        const double d2 = v2 - 2.0 * v3 + v4, e2 = v2 - v4;
-        const double d3 = v3 - 2.0 * v4 + v5, e3 = 3.0 * v3 - 4.0 * v4 + v5;
+        const double t3 = 3.0 * v3;
+        const double d1 = fma(-2.0, v2, v1) + v3, e1 = fma(-4.0, v2, v1) + t3;
+        const double d2 = fma(-2.0, v3, v2) + v4, e2 = v2 - v4;
+        const double d3 = fma(-2.0, v4, v3) + v5, e3 = fma(-4.0, v4, t3) + v5;
         s1 = 13.0 * d1 * d1 + 3.0 * e1 * e1;
         s2 = 13.0 * d2 * d2 + 3.0 * e2 * e2;
         s3 = 13.0 * d3 * d3 + 3.0 * e3 * e3;
-        p1 = 2.0 * v1 - 7.0 * v2 + 11.0 * v3;
-        p2 = -v2 + 5.0 * v3 + 2.0 * v4;
-        p3 = 2.0 * v3 + 5.0 * v4 - v5;
+        p1 = fma(2.0, v1, -(7.0 * v2)) + 11.0 * v3;
+        p2 = fma(2.0, v4, 5.0 * v3 - v2);
+        p3 = fma(2.0, v3, 5.0 * v4) - v5;
     }
     const double s5 = fabs(s1 - s3);
     const double a1 = 0.1 * (1.0 + s5 / (s1 + epsilon));
@@ -178,14 +191,15 @@ __device__ __forceinline__ double wenocu6_body(double v1, double v2, double v3, 
     const double six = 1.0 / 6.0;
     const double wa2a2 = 13.0 / 3.0, wa3a3 = 3129.0 / 80.0, wa4a4 = 87617.0 / 140.0, wa3a5 = 14127.0 / 224.0,
                  wa5a5 = 252337135.0 / 16128.0;
-    const double s11 = v1 - 2.0 * v2 + v3;
-    const double s12 = v1 - 4.0 * v2 + 3.0 * v3;
+    const double t3 = 3.0 * v3;
+    const double s11 = fma(-2.0, v2, v1) + v3;
+    const double s12 = fma(-4.0, v2, v1) + t3;
     const double s1 = 13.0 * s11 * s11 + 3.0 * s12 * s12;
-    const double s21 = v2 - 2.0 * v3 + v4;
+    const double s21 = fma(-2.0, v3, v2) + v4;
     const double s22 = v2 - v4;
     const double s2 = 13.0 * s21 * s21 + 3.0 * s22 * s22;
-    const double s31 = v3 - 2.0 * v4 + v5;
-    const double s32 = 3.0 * v3 - 4.0 * v4 + v5;
+    const double s31 = fma(-2.0, v4, v3) + v5;
+    const double s32 = fma(-4.0, v4, t3) + v5;
     const double s3 = 13.0 * s31 * s31 + 3.0 * s32 * s32;
     const double tau61 = (259.0 * v6 - 1895.0 * v5 + 6670.0 * v4 - 2590.0 * v3 - 2785.0 * v2 + 341.0 * v1) * ftss;
     const double tau62 = -(v5 - 12.0 * v4 + 22.0 * v3 - 12.0 * v2 + v1) * sxtn;
@@ -205,10 +219,10 @@ __device__ __forceinline__ double wenocu6_body(double v1, double v2, double v3, 
     const double tw1 = 1.0 / (a1 + a2 + a3 + a4);
     const double w1 = a1 * tw1, w2 = a2 * tw1, w3 = a3 * tw1, w4 = a4 * tw1;
     double temp = 0.0;
-    temp += w1 * (2.0 * v1 - 7.0 * v2 + 11.0 * v3);
-    temp += w2 * (-v2 + 5.0 * v3 + 2.0 * v4);
-    temp += w3 * (2.0 * v3 + 5.0 * v4 - v5);
-    temp += w4 * (11.0 * v4 - 7.0 * v5 + 2.0 * v6);
+    temp += w1 * (fma(2.0, v1, -(7.0 * v2)) + 11.0 * v3);
+    temp += w2 * fma(2.0, v4, 5.0 * v3 - v2);
+    temp += w3 * (fma(2.0, v3, 5.0 * v4) - v5);
+    temp += w4 * fma(2.0, v6, 11.0 * v4 - 7.0 * v5);
     return temp;
 }
 
@@ -217,16 +231,16 @@ __device__ __forceinline__ double wenocu6_body(double v1, double v2, double v3, 
 template <int SCHEME, bool FUSED>
 __device__ __forceinline__ double weno_face(const double *pp, const double *mm, double delta)
 {
+    const double six = 1.0 / 6.0;
     if (SCHEME == XF_WENOCU6) {
         const double epsilon = 1.e-8 * delta * delta;
         const double temf = wenocu6_body(pp[1], pp[2], pp[3], pp[4], pp[5], pp[6], epsilon);
         const double temm = wenocu6_body(mm[6], mm[5], mm[4], mm[3], mm[2], mm[1], epsilon);
-        return (temf + temm) * (1.0 / 6.0);
+        return (temf + temm) * six;
     }
     if (SCHEME == XF_WENO5Z)
         return weno5z_body<FUSED>(pp[1], pp[2], pp[3], pp[4], pp[5]) +
                weno5z_body<FUSED>(mm[6], mm[5], mm[4], mm[3], mm[2]);
-    const double six = 1.0 / 6.0;
     const double temf = weno5js_body(pp[1], pp[2], pp[3], pp[4], pp[5]);
     const double temm = weno5js_body(mm[6], mm[5], mm[4], mm[3], mm[2]);
     return (temf + temm) * six;
@@ -239,7 +253,12 @@ __device__ __forceinline__ double weno_face(const double *pp, const double *mm, 
 // weights are those of the FP64 definition up to FP32 rounding, with no
 // overflow for any data magnitude.  WENO5-JS weights are normalised through
 // the ratios (s_min / s_k)^2; WENO5-Z keeps tau5 = |beta_1 - beta_3|.  The
-// weights are normalised before they multiply the candidate values.
+// weights are normalised before they multiply the candidate values.  The split
+// values come in doubled, f +- a u for the reference's 0.5 (f +- a u): their
+// halving, exact until an FP32 value is subnormal, is folded into the constants
+// (four times the epsilons, half of the last factor), ten multiplications less per
+// field.  The FP64 forms halve each split value as the reference does, which
+// rounds where a tail of the field is subnormal.
 // Divisions use the hardware reciprocal (1 ulp).  A stencil below 1e-30 in
 // magnitude takes the ideal weights, as the FP64 form does when epsilon
 // dominates every indicator.
@@ -252,7 +271,7 @@ __device__ __forceinline__ float weno5_body_f32(float v1, float v2, float v3, fl
     const float q2 = -v2 + 5.0f * v3 + 2.0f * v4;
     const float q3 = 2.0f * v3 + 5.0f * v4 - v5;
     const float m = fmaxf(fmaxf(fmaxf(fabsf(v1), fabsf(v2)), fmaxf(fabsf(v3), fabsf(v4))), fabsf(v5));
-    if (!(m > 1e-30f)) return (0.1f * q1 + 0.6f * q2 + 0.3f * q3) * (1.0f / 6.0f);
+    if (!(m > 2e-30f)) return (0.1f * q1 + 0.6f * q2 + 0.3f * q3) * (0.5f * (1.0f / 6.0f));
     const float inv = rcp_f32(m);
     const float u1 = v1 * inv, u2 = v2 * inv, u3 = v3 * inv, u4 = v4 * inv, u5 = v5 * inv;
     float t = u1 - 2.0f * u2 + u3, r = u1 - 4.0f * u2 + 3.0f * u3;
@@ -261,7 +280,7 @@ __device__ __forceinline__ float weno5_body_f32(float v1, float v2, float v3, fl
     float s2 = 13.0f * t * t + 3.0f * r * r;
     t = u3 - 2.0f * u4 + u5, r = 3.0f * u3 - 4.0f * u4 + u5;
     float s3 = 13.0f * t * t + 3.0f * r * r;
-    const float eps = fmaxf(fminf(1e-6f * inv * inv, 1e30f), 1e-30f);
+    const float eps = fmaxf(fminf((4.0f * 1e-6f) * inv * inv, 1e30f), 1e-30f);
     float a1, a2, a3;
     if (SCHEME == XF_WENO5Z) {
         const float tau = fabsf(s1 - s3);
@@ -278,7 +297,7 @@ __device__ __forceinline__ float weno5_body_f32(float v1, float v2, float v3, fl
     // and epsilon is small, and a_k * q_k would overflow FP32 at the
     // magnitudes of strong shocks
     const float ia = rcp_f32(a1 + a2 + a3);
-    return ((a1 * ia) * q1 + (a2 * ia) * q2 + (a3 * ia) * q3) * (1.0f / 6.0f);
+    return ((a1 * ia) * q1 + (a2 * ia) * q2 + (a3 * ia) * q3) * (0.5f * (1.0f / 6.0f));
 }
 
 // WENO-CU6 in FP32 with the same rescaling: every indicator (s1..s3, s6)
@@ -291,7 +310,7 @@ __device__ __forceinline__ float wenocu6_body_f32(float v1, float v2, float v3, 
     const float c3 = 2.0f * v3 + 5.0f * v4 - v5;
     const float c4 = 11.0f * v4 - 7.0f * v5 + 2.0f * v6;
     const float m = fmaxf(fmaxf(fmaxf(fabsf(v1), fabsf(v2)), fmaxf(fabsf(v3), fabsf(v4))), fmaxf(fabsf(v5), fabsf(v6)));
-    if (!(m > 1e-30f)) return (0.05f * c1 + 0.45f * c2 + 0.45f * c3 + 0.05f * c4) * (1.0f / 6.0f);
+    if (!(m > 2e-30f)) return (0.05f * c1 + 0.45f * c2 + 0.45f * c3 + 0.05f * c4) * (0.5f * (1.0f / 6.0f));
     const float inv = rcp_f32(m);
     const float u1 = v1 * inv, u2 = v2 * inv, u3 = v3 * inv, u4 = v4 * inv, u5 = v5 * inv, u6 = v6 * inv;
     float t = u1 - 2.0f * u2 + u3, r = u1 - 4.0f * u2 + 3.0f * u3;
@@ -317,14 +336,14 @@ __device__ __forceinline__ float wenocu6_body_f32(float v1, float v2, float v3, 
     const float a4 = 0.05f * (20.0f + s5 * rcp_f32(s6 + eps));
     // normalised weights first (see weno5_body_f32): a_k up to ~1e34
     const float ia = rcp_f32(a1 + a2 + a3 + a4);
-    return ((a1 * ia) * c1 + (a2 * ia) * c2 + (a3 * ia) * c3 + (a4 * ia) * c4) * (1.0f / 6.0f);
+    return ((a1 * ia) * c1 + (a2 * ia) * c2 + (a3 * ia) * c3 + (a4 * ia) * c4) * (0.5f * (1.0f / 6.0f));
 }
 
 template <int SCHEME>
 __device__ __forceinline__ float weno_face_f32(const float *pp, const float *mm, float delta)
 {
     if (SCHEME == XF_WENOCU6) {
-        const float eps = 1.e-8f * delta * delta;
+        const float eps = 4.0f * (1.e-8f * delta * delta);
         return wenocu6_body_f32(pp[1], pp[2], pp[3], pp[4], pp[5], pp[6], eps) +
                wenocu6_body_f32(mm[6], mm[5], mm[4], mm[3], mm[2], mm[1], eps);
     }
@@ -332,18 +351,48 @@ __device__ __forceinline__ float weno_face_f32(const float *pp, const float *mm,
            weno5_body_f32<SCHEME>(mm[6], mm[5], mm[4], mm[3], mm[2]);
 }
 
-// get_DpDrho / get_DpDrhoi (Utils_device.hpp:14-35)
-__device__ __forceinline__ double dpdrho(double hN, double RN, double q2, double Cp, double R, double T, double gamma)
+// The Roe average and sound speed of a face divide some forty times at nine
+// species, most of them by the two cells' R and rho.  FAST (the wave's faces all
+// have rho, p, R, Cp and T within [2^-100, 2^100], face_fast) takes those from one
+// reciprocal per divisor by the corrected quotient and the others by the plain
+// division sequence, both the IEEE result there; otherwise IEEE division.
+template <bool FAST> __device__ __forceinline__ double face_quot(double a, double b, double y)
+{
+    return FAST ? dquot(a, b, y) : a / b;
+}
+template <bool FAST> __device__ __forceinline__ double face_div(double a, double b)
+{
+    return FAST ? ddiv_core(a, b) : a / b;
+}
+template <bool FAST> __device__ __forceinline__ double face_sqrt(double a) { return FAST ? dsqrt_core(a) : sqrt(a); }
+// every one of v[0..n) within [2^-100, 2^100] on every lane of the wave, from
+// the high words: ordered as unsigned integers, negative values and NaN on top
+template <int n> __device__ __forceinline__ bool face_fast(const double *v)
+{
+    unsigned lo = 0xffffffffu, hi = 0u;
+#pragma unroll
+    for (int k = 0; k < n; k++) {
+        const unsigned h = (unsigned)__double2hiint(v[k]);
+        lo = min(lo, h), hi = max(hi, h);
+    }
+    return __all(lo >= ((1023u - 100u) << 20) && hi < ((1023u + 100u) << 20));
+}
+
+// get_DpDrho / get_DpDrhoi (Utils_device.hpp:14-35); rR = RN(1 / R)
+template <bool FAST>
+__device__ __forceinline__ double dpdrho(double hN, double RN, double q2, double Cp, double R, double rR, double T,
+                                         double gamma)
 {
     const double RNT = RN * T;
-    return (gamma - 1.0) * (0.5 * q2 - hN + Cp * RNT / R);
+    return (gamma - 1.0) * (0.5 * q2 - hN + face_quot<FAST>(Cp * RNT, R, rR));
 }
+template <bool FAST>
 __device__ __forceinline__ double dpdrhoi(double hin, double Rin, double hiN, double RiN, double T, double Cp, double R,
-                                          double gamma)
+                                          double rR, double gamma)
 {
     const double hN_minus_hi = -hin + hiN;
     const double Ri_minus_RN = (Rin - RiN);
-    return (gamma - 1.0) * (hN_minus_hi + Cp * Ri_minus_RN * T / R);
+    return (gamma - 1.0) * (hN_minus_hi + face_quot<FAST>(Cp * Ri_minus_RN * T, R, rR));
 }
 
 // Face-local Roe state
@@ -354,12 +403,12 @@ template <int NS> struct RoeFace {
 };
 
 // ReconstructSoundSpeed + SoundSpeedMultiSpecies (Utils_device.hpp:42-140)
-// from the per-cell ingredients stored by the states pass.
-template <int NS>
+// from the per-cell ingredients stored by the states pass; r1l, r1r = RN(1 / rho)
+template <int NS, bool FAST>
 __device__ __forceinline__ void cop_c2(const DevThermo *__restrict__ th, RoeFace<NS> &rf, double D, double D1,
                                        const double *yl, const double *yr, const double *hl, const double *hr,
                                        double T_l, double T_r, double gamma_l, double gamma_r, double R_l, double R_r,
-                                       double Cp_l, double Cp_r, double rl, double rr, double ul, double vl, double wl,
+                                       double Cp_l, double Cp_r, double rl, double rr, double r1l, double r1r, double ul, double vl, double wl,
                                        double ur, double vr, double wr, double pl, double pr, double Hl, double Hr)
 {
     constexpr int NCOP = NS - 1;
@@ -368,19 +417,22 @@ __device__ __forceinline__ void cop_c2(const DevThermo *__restrict__ th, RoeFace
     const double Gamma = (gamma_l + D * gamma_r) * D1;
     const double q2_l = ul * ul + vl * vl + wl * wl;
     const double q2_r = ur * ur + vr * vr + wr * wr;
-    const double e_l = Hl - 0.5 * q2_l - pl / rl, e_r = Hr - 0.5 * q2_r - pr / rr;
-    const double RN = th->Ri[NCOP];
-    const double _dpdrho = (dpdrho(hl[NCOP], RN, q2_l, Cp_l, R_l, T_l, gamma_l) +
-                            D * dpdrho(hr[NCOP], RN, q2_r, Cp_r, R_r, T_r, gamma_r)) * D1;
+    const double prl = face_quot<FAST>(pl, rl, r1l), prr = face_quot<FAST>(pr, rr, r1r);
+    const double e_l = Hl - 0.5 * q2_l - prl, e_r = Hr - 0.5 * q2_r - prr;
+    const double rRl = FAST ? ddiv_core(1.0, R_l) : 0.0, rRr = FAST ? ddiv_core(1.0, R_r) : 0.0;
+    cdouble *Ri = as_const(th->Ri);
+    const double RN = Ri[NCOP];
+    const double _dpdrho = (dpdrho<FAST>(hl[NCOP], RN, q2_l, Cp_l, R_l, rRl, T_l, gamma_l) +
+                            D * dpdrho<FAST>(hr[NCOP], RN, q2_r, Cp_r, R_r, rRr, T_r, gamma_r)) * D1;
     double _dpdrhoi[NCOP > 0 ? NCOP : 1], drhoi[NCOP > 0 ? NCOP : 1];
 #pragma unroll
     for (int nn = 0; nn < NCOP; nn++) {
-        const double Rin = th->Ri[nn];
-        _dpdrhoi[nn] = (dpdrhoi(hl[nn], Rin, hl[NCOP], RN, T_l, Cp_l, R_l, gamma_l) +
-                        D * dpdrhoi(hr[nn], Rin, hr[NCOP], RN, T_r, Cp_r, R_r, gamma_r)) * D1;
+        const double Rin = Ri[nn];
+        _dpdrhoi[nn] = (dpdrhoi<FAST>(hl[nn], Rin, hl[NCOP], RN, T_l, Cp_l, R_l, rRl, gamma_l) +
+                        D * dpdrhoi<FAST>(hr[nn], Rin, hr[NCOP], RN, T_r, Cp_r, R_r, rRr, gamma_r)) * D1;
         drhoi[nn] = rr * yr[nn] - rl * yl[nn];
     }
-    const double _prho = (pl / rl + D * (pr / rr)) * D1 +
+    const double _prho = (prl + D * prr) * D1 +
                          0.5 * D * D1 * D1 * ((ur - ul) * (ur - ul) + (vr - vl) * (vr - vl) + (wr - wl) * (wr - wl));
     const double _dpdE = ((gamma_l - 1.0) + D * (gamma_r - 1.0)) * D1;
     const double _dpde = ((gamma_l - 1.0) * rl + D * ((gamma_r - 1.0) * rr)) * D1;
@@ -400,12 +452,21 @@ __device__ __forceinline__ void cop_c2(const DevThermo *__restrict__ th, RoeFace
     const double csqr = _dpdrho_new + _dpdE_new * _prho + Sum_Yidpdrhoi;
     rf.b1 = _dpdE_new / csqr;
     double b3 = 0.0;
+    // z_n = -nw_n / dpdE: one reciprocal while dpdE is well inside the range (a
+    // zero nw_n may come out as +0 for -0: z_n only multiplies sums that start at +0)
+    const double aE = fabs(_dpdE_new);
+    const bool shared = FAST && __all(aE >= 0x1p-300 && aE <= 0x1p300);
+    auto zs = [&](auto sh) {
+        const double y = 1.0 / _dpdE_new;
 #pragma unroll
-    for (int n = 0; n < NCOP; n++) {
-        const double nw = _dpdrhoi[n] + _dpdrhoi[n] * _dpdrhoi[n] * drhoi[n] * temp;
-        rf.z[n] = -nw / _dpdE_new;
-        b3 += rf._yi[n] * rf.z[n];
-    }
+        for (int n = 0; n < NCOP; n++) {
+            const double nw = _dpdrhoi[n] + _dpdrhoi[n] * _dpdrhoi[n] * drhoi[n] * temp;
+            rf.z[n] = decltype(sh)::value ? dquot(-nw, _dpdE_new, y) : -nw / _dpdE_new;
+            b3 += rf._yi[n] * rf.z[n];
+        }
+    };
+    if (shared) zs(std::true_type{});
+    else zs(std::false_type{});
     rf.b3 = b3 * rf.b1;
     double c2 = csqr;
     const double c2w = (c2 <= 0.0) ? 1.0 : 0.0;
@@ -430,6 +491,28 @@ __device__ __forceinline__ double glf_alpha(const double *red, int n)
     const int q = 3 * DIR + (n == 0 ? 0 : (n == E - 1 ? 2 : 1));
     const double a = red[RED_GLF + q], b = red[RED_GLFP + q];
     return b > a ? b : a;
+}
+
+// a value that is the same on every lane, on scalar registers
+__device__ __forceinline__ double uniform(double v)
+{
+    int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v)), lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+    asm volatile("" : "+s"(hi), "+s"(lo));
+    return __hiloint2double(hi, lo);
+}
+
+// the six sums are complete before any later LDS read of the face starts
+template <class T> __device__ __forceinline__ void projected(T *a)
+{
+    asm volatile("" : "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]) : : "memory");
+}
+
+// v is complete before any later LDS read of the face starts: without it the
+// compiler overlaps the unrolled rows and spills their partial sums
+__device__ __forceinline__ void row_done(double &v)
+{
+    asm volatile("" : "+v"(v) : : "memory");
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // PositivityPreservingKernel (positive-definite_eigen/PositivityPreserving_kernels.hpp:5-76)
@@ -669,27 +752,37 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
         const double ul = sU[NC + li_l] * r1l, vl = sU[2 * NC + li_l] * r1l, wl = sU[3 * NC + li_l] * r1l;
         const double ur = sU[NC + li_r] * r1r, vr = sU[2 * NC + li_r] * r1r, wr = sU[3 * NC + li_r] * r1r;
         const double Hl = (sU[4 * NC + li_l] + pl) * r1l, Hr = (sU[4 * NC + li_r] + pr) * r1r;
-        // MARCO_ROE
-        const double D = sqrt(rr / rl);
-        const double D1 = 1.0 / (D + 1.0);
+        // MARCO_ROE and the sound speed
         RoeFace<COP ? NS : 1> rf;
-        rf._u = (ul + D * ur) * D1;
-        rf._v = (vl + D * vr) * D1;
-        rf._w = (wl + D * wr) * D1;
-        rf._H = (Hl + D * Hr) * D1;
-        rf._P = (pl + D * pr) * D1;
-        rf._rho = sqrt(rr * rl);
-        if (COP) {
-            double yl[NT], yr[NT];
-            cell_y<NT>(g, f, id_l, r1l, [&](int k) { return sU[(5 + k) * NC + li_l]; }, yl);
-            cell_y<NT>(g, f, id_r, r1r, [&](int k) { return sU[(5 + k) * NC + li_r]; }, yr);
-            cop_c2<NT>(th, rf, D, D1, yl, yr, hl, hr, Tlr[0], Tlr[1], gcvlr[0], gcvlr[1], Rlr[0], Rlr[1], Cplr[0],
-                       Cplr[1], rl, rr, ul, vl, wl, ur, vr, wr, pl, pr, Hl, Hr);
+        auto roe = [&](auto fast) {
+            constexpr bool FAST = decltype(fast)::value;
+            const double D = face_sqrt<FAST>(face_quot<FAST>(rr, rl, r1l));
+            const double D1 = face_div<FAST>(1.0, D + 1.0);
+            rf._u = (ul + D * ur) * D1;
+            rf._v = (vl + D * vr) * D1;
+            rf._w = (wl + D * wr) * D1;
+            rf._H = (Hl + D * Hr) * D1;
+            rf._P = (pl + D * pr) * D1;
+            rf._rho = face_sqrt<FAST>(rr * rl);
+            if constexpr (COP) {
+                double yl[NT], yr[NT];
+                cell_y<NT>(g, f, id_l, r1l, [&](int k) { return sU[(5 + k) * NC + li_l]; }, yl);
+                cell_y<NT>(g, f, id_r, r1r, [&](int k) { return sU[(5 + k) * NC + li_r]; }, yr);
+                cop_c2<NT, FAST>(th, rf, D, D1, yl, yr, hl, hr, Tlr[0], Tlr[1], gcvlr[0], gcvlr[1], Rlr[0], Rlr[1],
+                                 Cplr[0], Cplr[1], rl, rr, r1l, r1r, ul, vl, wl, ur, vr, wr, pl, pr, Hl, Hr);
+            } else {
+                rf._yi[0] = 1.0;
+                rf.c2 = face_div<FAST>(ncop_gamma * rf._P, rf._rho);
+                rf.b1 = face_div<FAST>(ncop_gamma - 1.0, rf.c2);
+                rf.b3 = 0.0;
+            }
+        };
+        if constexpr (COP) {
+            const double v[10] = {rl, rr, pl, pr, Rlr[0], Rlr[1], Cplr[0], Cplr[1], Tlr[0], Tlr[1]};
+            if (face_fast<10>(v) && table_fast(th)) roe(std::true_type{});
+            else roe(std::false_type{});
         } else {
-            rf._yi[0] = 1.0;
-            rf.c2 = ncop_gamma * rf._P / rf._rho;
-            rf.b1 = (ncop_gamma - 1.0) / rf.c2;
-            rf.b3 = 0.0;
+            roe(std::false_type{}); // six divisions: the second copy's registers cost more
         }
         // MARCO_PREEIGEN (identical for every row, evaluated once)
         const double _u = rf._u, _v = rf._v, _w = rf._w, _H = rf._H, b1 = rf.b1, b3 = rf.b3;
@@ -716,93 +809,118 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
         auto split_weno_f32 = [&](float av, const float *uf, const float *ff) -> double {
             float pp[7], mm[7];
 #pragma unroll
-            for (int m = 1; m <= PHI; m++) pp[m] = 0.5f * fmaf(av, uf[m], ff[m]);
+            for (int m = 1; m <= PHI; m++) pp[m] = fmaf(av, uf[m], ff[m]);
 #pragma unroll
-            for (int m = PLO; m <= 6; m++) mm[m] = 0.5f * fmaf(-av, uf[m], ff[m]);
+            for (int m = PLO; m <= 6; m++) mm[m] = fmaf(-av, uf[m], ff[m]);
             return (double)weno_face_f32<SCHEME>(pp, mm, (float)dl);
         };
-        // dense rows: n = 0 (u-c), n = 1 + DIR (normal), n = E - 1 (u+c);
-        // called with literal n, so every branch on n folds at compile time
-        auto dense_row = [&](const int n) {
-            double L[E];
-            if (n == 0) {
-                L[0] = 0.5 * (b2 + un_c + b3);
+        // GLF dissipation of the three families of fields, on scalar registers
+        const double av_m = uniform(glf_alpha<DIR, E>(f.red, 0)), av_u = uniform(glf_alpha<DIR, E>(f.red, 1)),
+                     av_p = uniform(glf_alpha<DIR, E>(f.red, E - 1));
+        // LDS index of the first of the face's six points (the others follow at
+        // STEP), as a value of its own in every row: the compiler would keep the
+        // values that several rows read, and spill them
+        constexpr int STEP = DIR == 0 ? 1 : TW;
+        auto first_point = [&]() {
+            int li = lds_ix<DIR, TS, TW>(fidx, tcol);
+            asm volatile("" : "+v"(li));
+            return li;
+        };
+        // ---- dense rows: n = 0 (u-c), n = 1 + DIR (normal), n = E - 1 (u+c);
+        // called with literal n, so every branch on n folds at compile time.
+        // Projections component-outer: every accumulator still sums over n1
+        // in increasing order, product then sum (plain form) or one fused
+        // multiply-add per term (fused form).  The next component's values are
+        // read while the present one is accumulated, and no further ahead
+        // (projected): left alone the compiler reads all E components first and
+        // spills them.
+        double fl_m, fl_p;
+        auto acoustic = [&](auto zero, const auto *SU, const auto *SF, auto mad, auto face) {
+            typedef decltype(zero) T;
+            const int l0 = first_point();
+            T um[7], fm[7], up[7], fp[7], cu[7], cf[7], nu[7], nf[7];
+            auto read = [&](const int n1, T *u, T *q) {
 #pragma unroll
-                for (int k = 0; k < 3; k++)
-                    L[1 + k] = (k == DIR) ? -0.5 * (b1 * vr3[k] + _c1) : -0.5 * (b1 * vr3[k]);
-                L[4] = 0.5 * b1;
+                for (int m = 1; m <= 6; m++) u[m] = SU[n1 * NC + l0 + (m - 1) * STEP], q[m] = SF[n1 * NC + l0 + (m - 1) * STEP];
+            };
 #pragma unroll
-                for (int m = 0; m < NCOP; m++) L[5 + m] = -0.5 * b1 * rf.z[m];
-            } else if (n == E - 1) {
-                L[0] = 0.5 * (b2 - un_c + b3);
+            for (int m = 1; m <= 6; m++) um[m] = fm[m] = up[m] = fp[m] = zero;
+            read(0, cu, cf);
 #pragma unroll
-                for (int k = 0; k < 3; k++)
-                    L[1 + k] = (k == DIR) ? 0.5 * (-b1 * vr3[k] + _c1) : 0.5 * (-b1 * vr3[k]);
-                L[4] = 0.5 * b1;
+            for (int n1 = 0; n1 < E; n1++) {
+                const bool both = n1 != 0 && n1 != 1 + DIR;
+                double Lm, Lp;
+                if (n1 == 0) Lm = 0.5 * (b2 + un_c + b3), Lp = 0.5 * (b2 - un_c + b3);
+                else if (n1 == 1 + DIR) Lm = -0.5 * (b1 * vr3[DIR] + _c1), Lp = 0.5 * (-b1 * vr3[DIR] + _c1);
+                else if (n1 <= 3) Lm = Lp = -0.5 * (b1 * vr3[n1 - 1]);
+                else if (n1 == 4) Lm = Lp = 0.5 * b1;
+                else Lm = Lp = -0.5 * b1 * rf.z[n1 < 5 ? 0 : n1 - 5];
+                if (n1 + 1 < E) read(n1 + 1, nu, nf);
 #pragma unroll
-                for (int m = 0; m < NCOP; m++) L[5 + m] = -0.5 * b1 * rf.z[m];
-            } else {
-                L[0] = (1.0 - b2 - b3) / b1;
-                L[1] = _u;
-                L[2] = _v;
-                L[3] = _w;
-                L[4] = -1.0;
+                for (int m = 1; m <= 6; m++) {
+                    mad(cu[m], (T)Lm, um[m], (T)Lp, up[m], both);
+                    mad(cf[m], (T)Lm, fm[m], (T)Lp, fp[m], both);
+                }
+                projected(um), projected(fm), projected(up), projected(fp);
 #pragma unroll
-                for (int m = 0; m < NCOP; m++) L[5 + m] = rf.z[m];
+                for (int m = 1; m <= 6; m++) cu[m] = nu[m], cf[m] = nf[m];
             }
-            // projections, component-outer: every accumulator still sums
-            // over n1 in increasing order, product then sum (plain form) or
-            // one fused multiply-add per term (fused form); the empty asm is a compiler-only
-            // fence that keeps the LDS loads of one component from being
-            // hoisted above the previous one (register pressure)
-            double fl;
-            if (MIX) {
-                // FP32 projections (fused multiply-add) and FP32 WENO
-                float uf[7], ff[7];
+            fl_m = face((T)av_m, um, fm);
+            row_done(fl_m);
+            fl_p = face((T)av_p, up, fp);
+            row_done(fl_p);
+        };
+        auto normal = [&](auto zero, const auto *SU, const auto *SF, auto mad, auto face) -> double {
+            typedef decltype(zero) T;
+            const int l0 = first_point();
+            T uf[7], ff[7], cu[7], cf[7], nu[7], nf[7], dummy;
+            auto read = [&](const int n1, T *u, T *q) {
 #pragma unroll
-                for (int m = 1; m <= 6; m++) uf[m] = 0.0f, ff[m] = 0.0f;
+                for (int m = 1; m <= 6; m++) u[m] = SU[n1 * NC + l0 + (m - 1) * STEP], q[m] = SF[n1 * NC + l0 + (m - 1) * STEP];
+            };
 #pragma unroll
-                for (int n1 = 0; n1 < E; n1++) {
-                    const float Ln = (float)L[n1];
+            for (int m = 1; m <= 6; m++) uf[m] = ff[m] = zero;
+            read(0, cu, cf);
 #pragma unroll
-                    for (int m = 1; m <= 6; m++) {
-                        const int li = lds_ix<DIR, TS, TW>(fidx + m - 1, tcol);
-                        uf[m] = fmaf(sUf[n1 * NC + li], Ln, uf[m]);
-                        ff[m] = fmaf(sFf[n1 * NC + li], Ln, ff[m]);
-                    }
-                    asm volatile("" ::: "memory");
+            for (int n1 = 0; n1 < E; n1++) {
+                double L;
+                if (n1 == 0) L = (1.0 - b2 - b3) / b1;
+                else if (n1 <= 3) L = vr3[n1 - 1];
+                else if (n1 == 4) L = -1.0;
+                else L = rf.z[n1 < 5 ? 0 : n1 - 5];
+                if (n1 + 1 < E) read(n1 + 1, nu, nf);
+#pragma unroll
+                for (int m = 1; m <= 6; m++) {
+                    dummy = zero;
+                    mad(cu[m], (T)L, uf[m], (T)L, dummy, true), mad(cf[m], (T)L, ff[m], (T)L, dummy, true);
                 }
-                fl = split_weno_f32((float)glf_alpha<DIR, E>(f.red, n), uf, ff);
-            } else {
-                double uf[7], ff[7];
+                projected(uf), projected(ff);
 #pragma unroll
-                for (int m = 1; m <= 6; m++) uf[m] = 0.0, ff[m] = 0.0;
-#pragma unroll
-                for (int n1 = 0; n1 < E; n1++) {
-                    const double Ln = L[n1];
-#pragma unroll
-                    for (int m = 1; m <= 6; m++) {
-                        const int li = lds_ix<DIR, TS, TW>(fidx + m - 1, tcol);
-                        uf[m] = madd<FUSED>(sU[n1 * NC + li], Ln, uf[m]);
-                        ff[m] = madd<FUSED>(sF[n1 * NC + li], Ln, ff[m]);
-                    }
-                    asm volatile("" ::: "memory");
-                }
-                fl = split_weno(glf_alpha<DIR, E>(f.red, n), uf, ff);
+                for (int m = 1; m <= 6; m++) cu[m] = nu[m], cf[m] = nf[m];
             }
-            // right column n, accumulated in the reference's summation order
-            // (fluxl += f_flux * r per entry, fused in the fused form)
-            if (n == 0 || n == E - 1) {
-                flux[0] += fl;
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    const double Rk = (k == DIR) ? (n == 0 ? vr3[k] - _c : vr3[k] + _c) : vr3[k];
-                    flux[1 + k] = madd<FUSED>(fl, Rk, flux[1 + k]);
-                }
-                flux[4] = madd<FUSED>(fl, n == 0 ? _H - un * _c : _H + un * _c, flux[4]);
-#pragma unroll
-                for (int m = 0; m < NCOP; m++) flux[5 + m] = madd<FUSED>(fl, rf._yi[m], flux[5 + m]);
+            return face((T)av_u, uf, ff);
+        };
+        auto mad64 = [](double v, double la, double &aa, double lb, double &ab, bool both) {
+            if (FUSED) {
+                aa = fma(v, la, aa), ab = fma(v, lb, ab);
             } else {
+                const double pa = v * la, pb = both ? pa : v * lb;
+                aa += pa, ab += pb;
+            }
+        };
+        auto mad32 = [](float v, float la, float &aa, float lb, float &ab, bool) {
+            aa = fmaf(v, la, aa), ab = fmaf(v, lb, ab);
+        };
+        auto normal_row = [&]() -> double {
+            if constexpr (MIX) return normal(0.0f, sUf, sFf, mad32, split_weno_f32);
+            else return normal(0.0, sU, sF, mad64, split_weno);
+        };
+        if constexpr (MIX) acoustic(0.0f, sUf, sFf, mad32, split_weno_f32);
+        else acoustic(0.0, sU, sF, mad64, split_weno);
+        // ---- right columns, accumulated in the reference's summation order
+        // (field by field, fluxl += f_flux * r per entry, fused in the fused form)
+        auto column = [&](const int n, double fl) {
+            if (n == 1 + DIR) {
                 flux[0] = madd<FUSED>(fl, b1, flux[0]);
                 flux[1] = madd<FUSED>(fl, _u * b1, flux[1]);
                 flux[2] = madd<FUSED>(fl, _v * b1, flux[2]);
@@ -810,75 +928,85 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
                 flux[4] = madd<FUSED>(fl, _H * b1 - 1.0, flux[4]);
 #pragma unroll
                 for (int m = 0; m < NCOP; m++) flux[5 + m] = madd<FUSED>(fl, b1 * rf._yi[m], flux[5 + m]);
+                return;
+            }
+            flux[0] += fl;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const double Rk = (k == DIR) ? (n == 0 ? vr3[k] - _c : vr3[k] + _c) : vr3[k];
+                flux[1 + k] = madd<FUSED>(fl, Rk, flux[1 + k]);
+            }
+            flux[4] = madd<FUSED>(fl, n == 0 ? _H - un * _c : _H + un * _c, flux[4]);
+#pragma unroll
+            for (int m = 0; m < NCOP; m++) flux[5 + m] = madd<FUSED>(fl, rf._yi[m], flux[5 + m]);
+        };
+        column(0, fl_m);
+        // ---- the E-3 rows with two structural non-zeros (L[0] and +-1 at kk;
+        // the right column has +-1 at kk and an energy entry R4), unrolled: the
+        // row's species, its sign and the flux component it adds to are
+        // compile-time, where a runtime loop spent 68 of its instructions per
+        // row on selecting them.  A product by an exact 0 or +-1 rounds the same
+        // fused or unfused, so these rows equal the oracle's full dot products
+        // in either form.
+        auto sparse = [&](auto zero, const auto *SU, const auto *SF, auto face) {
+            typedef decltype(zero) T;
+            // rho and its flux, which every one of these rows reads, stay in
+            // registers where that costs no wave (with one species the four-wave
+            // bound has no room, with four and five it decides between two and
+            // three waves)
+            constexpr bool KEEP0 = NS != 1 && NS != 4 && NS != 5;
+            T u0[7], f0[7];
+            auto read0 = [&](int l0) {
+#pragma unroll
+                for (int m = 1; m <= 6; m++) u0[m] = SU[l0 + (m - 1) * STEP], f0[m] = SF[l0 + (m - 1) * STEP];
+            };
+            if (KEEP0) read0(first_point());
+#pragma unroll
+            for (int n = 1; n <= E - 2; n++) {
+                if (n == 1 + DIR) {
+                    column(n, normal_row());
+                    continue;
+                }
+                const int kk = n <= 3 ? n : n + 1;
+                double L0, R4;
+                bool neg = false;
+                if (n <= 3) {
+                    if (DIR == 0) { L0 = (n == 2) ? _v : -_w; neg = (n == 2); R4 = (n == 2) ? -_v : _w; }
+                    else if (DIR == 1) { L0 = (n == 1) ? -_u : _w; neg = (n == 3); R4 = (n == 1) ? _u : -_w; }
+                    else { L0 = (n == 1) ? _u : -_v; neg = (n == 1); R4 = (n == 1) ? -_u : _v; }
+                } else {
+                    L0 = -rf._yi[n - 4 < NCOP ? n - 4 : 0];
+                    R4 = rf.z[n - 4 < NCOP ? n - 4 : 0];
+                }
+                const T L = (T)L0;
+                const int l0 = first_point();
+                if (!KEEP0) read0(l0);
+                T uf[7], ff[7];
+#pragma unroll
+                for (int m = 1; m <= 6; m++) {
+                    const int li = l0 + (m - 1) * STEP;
+                    const T au = SU[kk * NC + li], bf = SF[kk * NC + li];
+                    if constexpr (MIX) {
+                        uf[m] = fmaf(u0[m], L, neg ? -au : au);
+                        ff[m] = fmaf(f0[m], L, neg ? -bf : bf);
+                    } else {
+                        // one fma for 0.0 + product: the product rounds once,
+                        // and a zero comes out +0 as the sum's does
+                        const double a0 = fma(u0[m], L, 0.0), b0 = fma(f0[m], L, 0.0);
+                        uf[m] = neg ? a0 - au : a0 + au;
+                        ff[m] = neg ? b0 - bf : b0 + bf;
+                    }
+                }
+                const double fl = face((T)av_u, uf, ff);
+                flux[kk] += neg ? -fl : fl;
+                flux[4] = madd<FUSED>(fl, R4, flux[4]);
+                row_done(flux[kk]);
+                row_done(flux[4]);
             }
         };
-
-        dense_row(0);
-        // the E-3 rows with two structural non-zeros (L[0] and +-1 at kk; the
-        // right column has +-1 at kk and an energy entry R4), in a runtime
-        // loop; contributions go to flux[kk] through a masked add (+0.0 on
-        // the other components is exact: no accumulator is ever -0.0).
-        // A product by an exact 0 or +-1 rounds the same fused or unfused,
-        // so these rows equal the oracle's full dot products in either form.
-#pragma unroll 1
-        for (int n = 1; n <= E - 2; n++) {
-            if (n == 1 + DIR) {
-                dense_row(1 + DIR);
-                continue;
-            }
-            double L0, R4;
-            int kk;
-            bool neg;
-            if (n <= 3) {
-                kk = n;
-                if (DIR == 0) { L0 = (n == 2) ? _v : -_w; neg = (n == 2); R4 = (n == 2) ? -_v : _w; }
-                else if (DIR == 1) { L0 = (n == 1) ? -_u : _w; neg = (n == 3); R4 = (n == 1) ? _u : -_w; }
-                else { L0 = (n == 1) ? _u : -_v; neg = (n == 1); R4 = (n == 1) ? -_u : _v; }
-            } else {
-                const int m = n - 4;
-                double ym = 0.0, zm = 0.0;
-#pragma unroll
-                for (int q = 0; q < NCOP; q++) {
-                    ym = (q == m) ? rf._yi[q] : ym;
-                    zm = (q == m) ? rf.z[q] : zm;
-                }
-                kk = 5 + m;
-                L0 = -ym;
-                R4 = zm;
-                neg = false;
-            }
-            double fl;
-            if (MIX) {
-                const float L0f = (float)L0;
-                float uf[7], ff[7];
-#pragma unroll
-                for (int m = 1; m <= 6; m++) {
-                    const int li = lds_ix<DIR, TS, TW>(fidx + m - 1, tcol);
-                    const float au = sUf[kk * NC + li], bf = sFf[kk * NC + li];
-                    uf[m] = fmaf(sUf[li], L0f, neg ? -au : au);
-                    ff[m] = fmaf(sFf[li], L0f, neg ? -bf : bf);
-                }
-                fl = split_weno_f32((float)glf_alpha<DIR, E>(f.red, n), uf, ff);
-            } else {
-                double uf[7], ff[7];
-#pragma unroll
-                for (int m = 1; m <= 6; m++) {
-                    const int li = lds_ix<DIR, TS, TW>(fidx + m - 1, tcol);
-                    const double a0 = 0.0 + sU[li] * L0;
-                    const double b0 = 0.0 + sF[li] * L0;
-                    const double au = sU[kk * NC + li], bf = sF[kk * NC + li];
-                    uf[m] = neg ? a0 + (-au) : a0 + au;
-                    ff[m] = neg ? b0 + (-bf) : b0 + bf;
-                }
-                fl = split_weno(glf_alpha<DIR, E>(f.red, n), uf, ff);
-            }
-            const double t = neg ? -fl : fl;
-#pragma unroll
-            for (int k = 1; k < E; k++)
-                if (k != 4) flux[k] += (k == kk) ? t : 0.0;
-            flux[4] = madd<FUSED>(fl, R4, flux[4]);
-        }
-        dense_row(E - 1);
+        if constexpr (MIX) sparse(0.0f, sUf, sFf, split_weno_f32);
+        else sparse(0.0, sU, sF, split_weno);
+        column(E - 1, fl_p);
         // positivity-preserving limiter on the faces right of interior cells
         if (g.positivity && sl >= B) {
             const double lambda_0 = f.red[RED_LAM + DIR];

@@ -132,6 +132,11 @@ __device__ __forceinline__ double s_k(const DevThermo *__restrict__ th, const TP
 // compiler drops that for an ordinary pointer once control flow diverges).
 typedef const double __attribute__((address_space(4))) cdouble;
 __device__ __forceinline__ cdouble *as_const(const double *p) { return (cdouble *)(unsigned long long)p; }
+// DevThermo::fast as a scalar load
+__device__ __forceinline__ bool table_fast(const DevThermo *__restrict__ th)
+{
+    return *(const int __attribute__((address_space(4))) *)(unsigned long long)&th->fast != 0;
+}
 
 // ---- the fits on a temperature every lane of the wave is known to share a
 // fit range at, 200 K <= T <= 1e5 K (FastT below): the same expressions with the
