@@ -74,6 +74,7 @@ struct xf_ctx {
     hipStream_t stream = nullptr;
     Fields f{};
     double *U2 = nullptr; // RK stage-2 output of the fused path
+    double *xbuf = nullptr; // cells in the host's order on their way in or out (xf_upload_state)
     DevThermo h_th{};
     DevThermo *d_th = nullptr;
     DevMech h_mc{};
