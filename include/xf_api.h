@@ -297,7 +297,8 @@ int xf_kernel_times(xf_ctx *ctx, const char **names, double *avg_ms, int *counts
 int xf_time_kernel(xf_ctx *ctx, const char *name, int reps, double *avg_ms);
 /* Sweep tile shape per direction (0 = x, 1 = y, 2 = z): x 0 = 64 faces x 4
    pencils, 1 = 32 x 8; y, z 0 = 16 x 16, 1 = 32 x 8, 2 = 8 x 32.  Every shape
-   computes the same bits.  Replaces the fixed work-group sizes of the
+   computes the same bits; a context starts with the shapes that need the fewest
+   blocks on its grid.  Replaces the fixed work-group sizes of the
    settings file (run.blockSize_x/y/z, src/read_ini/settings/read_json.cpp:112-114). */
 int xf_set_tile_shape(xf_ctx *ctx, int dir, int shape);
 int xf_get_tile_shape(const xf_ctx *ctx, int *shape3);

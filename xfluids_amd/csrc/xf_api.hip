@@ -344,6 +344,7 @@ int xf_create(const xf_case_desc *desc, xf_ctx **out)
     g.Yil_limiter = d.Yil_limiter;
     g.Dim_limiter = d.Dim_limiter;
     g.N = c->N;
+    for (int q = 0; q < 3; q++) c->shape[q] = default_tile_shape(g, q);
     auto fail = [&](int code) {
         xf_destroy(c);
         return code;
@@ -1345,9 +1346,9 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
             for (int q = 0; q < 6; q++) bcs |= (c->d.BC[q] & 15) << (4 * q);
             r.bcs = bcs | (1 << 28);
             for (int dd = 0; dd < 3; dd++) {
-                unsigned gr[3];
+                unsigned gr[5];
                 sweep_grid(c->g, dd, e->shape[dd], gr);
-                for (int q = 0; q < 3; q++) r.tiles[dd][q] = (int)gr[q];
+                for (int q = 0; q < 5; q++) r.tiles[dd][q] = (int)gr[q];
                 r.tile_off[dd] = tb[dd];
                 tb[dd] += (long long)gr[0] * gr[1] * gr[2];
             }

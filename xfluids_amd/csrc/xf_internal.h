@@ -94,7 +94,8 @@ struct Fields {
 
 // One case of an ensemble as the ensemble's launches see it: geometry,
 // fields, the stage-2 buffer, the case's first block in a states launch and
-// in a sweep launch of each direction, its tile grid per direction and its
+// in a sweep launch of each direction, its tile grid per direction with the cells
+// and columns a tile covers (sweep_grid), and its
 // packed ghost-fill codes (bit 28 set, as k_states takes them).
 struct EnsCase {
     Geom g;
@@ -102,7 +103,7 @@ struct EnsCase {
     double *U2;
     long long state_off;
     long long tile_off[3];
-    int tiles[3][3];
+    int tiles[3][5];
     int bcs;
     // 0 = U, 1 = U1, 2 = U2
     __device__ __forceinline__ double *buf(int sel) const { return sel == 0 ? f.U : (sel == 1 ? f.U1 : U2); }

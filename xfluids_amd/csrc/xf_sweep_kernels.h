@@ -583,12 +583,14 @@ template <int NS, int PREC> struct SweepOccupancy {
 template <int NS> constexpr bool visc_in_sweep() { return NS >= 4; }
 
 // One tile of TS faces x TW pencils of one direction: (tx, ty, tz) is the
-// tile, in units of tiles along x, the pencil rows and the third axis.
+// tile, in units of tiles along x, the pencil rows and the third axis; it covers
+// span cells along the sweep (at most TS - 1) and, in y and z, cols columns (at
+// most TW), as sweep_grid sets them.
 template <int NS, bool COP, int DIR, int SCHEME, int PREC, int SHAPE>
 __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__restrict__ th,
                                            const double *__restrict__ Ug, const Fields &f, double ncop_gamma,
                                            int mode, int stage, const double *Ua, const double *Ub, double *Uo,
-                                           int tx, int ty, int tz)
+                                           int tx, int ty, int tz, int span, int cols)
 {
     constexpr int E = COP ? NS + 4 : 5;
     constexpr int NCOP = COP ? NS - 1 : 0;
@@ -611,7 +613,9 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
     const int B = DIR == 0 ? g.Bx : (DIR == 1 ? g.By : g.Bz);
     const int inner = DIR == 0 ? g.X_inner : (DIR == 1 ? g.Y_inner : g.Z_inner);
     const int Lmax = DIR == 0 ? g.Xmax : (DIR == 1 ? g.Ymax : g.Zmax);
-    const int c0 = B + (TS - 1) * (DIR == 0 ? tx : ty);
+    const int c0 = B + span * (DIR == 0 ? tx : ty);
+    const int col_end = g.Bx + min((tx + 1) * cols, g.X_inner); // y, z: the tile's columns
+    const int face_end = min(c0 + span, B + inner);             // its faces: right of cells c0 - 1 .. face_end - 1
     const long long stride = DIR == 0 ? 1LL : (DIR == 1 ? (long long)g.Xmax : (long long)g.Xmax * g.Ymax);
     const double *vel_n = DIR == 0 ? f.u : (DIR == 1 ? f.v : f.w);
 
@@ -622,12 +626,12 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
             const int j = g.By + r % g.Y_inner, k = g.Bz + r / g.Y_inner;
             return (long long)g.Xmax * g.Ymax * k + (long long)g.Xmax * j;
         } else if (DIR == 1) {
-            const int i = g.Bx + tx * TW + q;
-            ok = i < g.Bx + g.X_inner;
+            const int i = g.Bx + tx * cols + q;
+            ok = i < col_end;
             return (long long)g.Xmax * g.Ymax * (g.Bz + tz) + i;
         } else {
-            const int i = g.Bx + tx * TW + q;
-            ok = i < g.Bx + g.X_inner;
+            const int i = g.Bx + tx * cols + q;
+            ok = i < col_end;
             return (long long)g.Xmax * (g.By + tz) + i;
         }
     };
@@ -717,7 +721,7 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
     bool okp;
     const long long pbase = pencil_base(tcol, okp);
     const int sl = c0 + fidx - 1;
-    const bool face_ok = okp && (sl <= B + inner - 1);
+    const bool face_ok = okp && sl < face_end;
     constexpr int NT = COP ? NS : 1;
     double hl[NT], hr[NT], Tlr[2], gcvlr[2], Rlr[2], Cplr[2];
     if (COP && face_ok) {
@@ -1072,7 +1076,7 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
     // loaded before the barriers: the loads are in flight while the tile's
     // other waves finish their faces.  Each cell is read and written only by
     // its own lane, and no tile stages from the arrays written here.
-    const bool cell_ok = fidx >= 1 && okp && sl <= B + inner - 1;
+    const bool cell_ok = fidx >= 1 && face_ok;
     double LUi[E], Ai[E], Bi[E];
 #pragma unroll
     for (int n = 0; n < E; n++) LUi[n] = 0.0, Ai[n] = 0.0, Bi[n] = 0.0;
@@ -1133,11 +1137,12 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
 template <int NS, bool COP, int DIR, int SCHEME, int PREC, int SHAPE>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SweepOccupancy<NS, PREC>::waves)))
 k_sweep(Geom g, const DevThermo *__restrict__ th, const double *__restrict__ Ug, Fields f, double ncop_gamma, int mode,
-        int stage, const double *Ua, const double *Ub, double *Uo)
+        int stage, const double *Ua, const double *Ub, double *Uo, int span, int cols)
 {
     int tx, ty, tz;
     xcd_tile(tx, ty, tz);
-    sweep_tile<NS, COP, DIR, SCHEME, PREC, SHAPE>(g, th, Ug, f, ncop_gamma, mode, stage, Ua, Ub, Uo, tx, ty, tz);
+    sweep_tile<NS, COP, DIR, SCHEME, PREC, SHAPE>(g, th, Ug, f, ncop_gamma, mode, stage, Ua, Ub, Uo, tx, ty, tz, span,
+                                                  cols);
 }
 
 // the tiles of every case of an ensemble in one launch: block b belongs to
@@ -1154,7 +1159,8 @@ k_sweep_multi(const EnsCase *__restrict__ cases, int ncases, const DevThermo *__
     const int l = (int)(b - c.tile_off[DIR]);
     const int gx = c.tiles[DIR][0], gy = c.tiles[DIR][1];
     sweep_tile<NS, COP, DIR, SCHEME, PREC, SHAPE>(c.g, th, c.buf(sel_g), c.f, ncop_gamma, mode, stage, c.buf(sel_a),
-                                                  c.buf(sel_b), c.buf(sel_o), l % gx, (l / gx) % gy, l / (gx * gy));
+                                                  c.buf(sel_b), c.buf(sel_o), l % gx, (l / gx) % gy, l / (gx * gy),
+                                                  c.tiles[DIR][3], c.tiles[DIR][4]);
 }
 
 } // namespace xf

@@ -13,12 +13,12 @@ template <int NS, bool COP, int SCH> struct SweepKernels {
         static_assert(SweepShape<DIR, E, SHAPE>::TS == (DIR == 0 ? (SHAPE == 0 ? 64 : 32)
                                                                  : (SHAPE == 0 ? 16 : (SHAPE == 1 ? 32 : 8))),
                       "sweep_grid's tile sizes");
-        unsigned gr[3];
+        unsigned gr[5];
         sweep_grid(c->g, DIR, SHAPE, gr);
         static const char *names[3] = {"sweep_x", "sweep_y", "sweep_z"};
         ProfScope ps(c, names[DIR]);
         hipLaunchKernelGGL((k_sweep<NS, COP, DIR, SCH, PREC, SHAPE>), dim3(gr[0], gr[1], gr[2]), dim3(256), 0, c->stream,
-                           c->g, c->d_th, Ug, c->f, c->d.ncop_gamma, mode, stage, Ua, Ub, Uo);
+                           c->g, c->d_th, Ug, c->f, c->d.ncop_gamma, mode, stage, Ua, Ub, Uo, (int)gr[3], (int)gr[4]);
     }
     template <int DIR, int PREC, int SHAPE>
     static void multi_t(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks, int mode,
