@@ -449,6 +449,15 @@ int xf_set_thermo(xf_ctx *c, const double *Hia, const double *Hib, const double 
             double *h = c->h_th.Hc + (r * MAXNS + n) * 9;
             for (int m = 0; m < 7; m++) h[m] = Hia[n * 21 + m * 3 + r];
             for (int m = 0; m < 2; m++) h[7 + m] = Hib[n * 6 + m * 3 + r];
+            double *f = c->h_th.Hf + (r * MAXNS + n) * FITC;
+            std::copy(h, h + 9, f);
+            if (c->d.thermo) {
+                f[9] = 0.5 * h[3], f[10] = h[4] * OT, f[11] = 0.25 * h[5], f[12] = 0.2 * h[6];
+                f[13] = -0.5 * h[0], f[14] = 0.5 * h[4], f[15] = h[5] * OT, f[16] = h[6] * 0.25;
+            } else {
+                f[9] = h[1] * 0.5, f[10] = h[2] * OT, f[11] = h[3] * 0.25;
+                f[14] = 0.5 * h[2], f[15] = h[3] * OT, f[16] = h[4] * 0.25;
+            }
         }
     for (int n = 0; n < NS; n++) {
         // src/read_ini/src/thermal.cpp:158-161

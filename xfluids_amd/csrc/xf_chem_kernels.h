@@ -261,12 +261,12 @@ __device__ __forceinline__ bool evalcv_fast(const DevThermo *__restrict__ th, co
         ft.each(true, [&](cdouble *cf) {
 #pragma unroll
             for (int n = 0; n < NS; n++) {
-                h1[n] = h_fast<NASA>(cf + 9 * n, m_tmp, ft.iT, ft.lT, 1.0);
+                h1[n] = h_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, ft.lT, 1.0);
                 double g = 0.0;
-                g += s_fast<NASA>(cf + 9 * n, m_tmp, ft.iT, ft.lT);
+                g += s_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, ft.lT);
                 g += dquot(-h1[n], m_tmp, ft.iT);
                 lg[n] = logP - g;
-                cv += y[1 + n] * cp_fast<NASA>(cf + 9 * n, m_tmp, ft.iT, Rk[n]);
+                cv += y[1 + n] * cp_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, Rk[n]);
             }
         });
         c.logT = ft.lT, c.rT = ft.iT;
@@ -637,7 +637,7 @@ __device__ __forceinline__ double mix_e(const DevThermo *__restrict__ th, const 
         if (ft.ok) {
             ft.each(NASA, [&](cdouble *c) {
 #pragma unroll
-                for (int n = 0; n < NS; n++) e += (h_fast<NASA>(c + 9 * n, T, ft.iT, ft.lT, 1.0) - T) * Rk[n] * yi[n];
+                for (int n = 0; n < NS; n++) e += (h_fast<NASA>(c + FITC * n, T, ft.iT, ft.lT, 1.0) - T) * Rk[n] * yi[n];
             });
             return;
         }

@@ -310,8 +310,8 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
                     ft.each(NASA, [&](cdouble *cf) {
 #pragma unroll
                         for (int n = 0; n < NS; n++) {
-                            cpk[n] = cp_fast<NASA>(cf + 9 * n, T, ft.iT, Rk[n]);
-                            hk[n] = h_fast<NASA>(cf + 9 * n, T, ft.iT, ft.lT, Rk[n]);
+                            cpk[n] = cp_fast<NASA>(cf + FITC * n, T, ft.iT, Rk[n]);
+                            hk[n] = h_fast<NASA>(cf + FITC * n, T, ft.iT, ft.lT, Rk[n]);
                         }
                     });
                 } else {

@@ -12,6 +12,8 @@ constexpr int MAXNS = XF_MAXNS;
 constexpr int MAXNR = XF_MAXNR;
 constexpr int MAXE = XF_MAXNS + 4;
 
+constexpr int FITC = 18; // doubles per row of DevThermo::Hf (17 used)
+
 // Thermal tables (reference layout, src/include/global_setup.h:202-208)
 struct DevThermo {
     double Hia[MAXNS * 21];
@@ -21,6 +23,10 @@ struct DevThermo {
     // one species is 72 contiguous bytes (two scalar loads when r is
     // wave-uniform, instead of nine strided ones)
     double Hc[3 * MAXNS * 9];
+    // the row of the straight-line fits (h_fast, s_fast): the nine coefficients, then
+    // the products with the fits' constants that do not depend on T, rounded as the
+    // kernels would (xf_set_thermo)
+    double Hf[3 * MAXNS * FITC];
     double Wi[MAXNS], _Wi[MAXNS], Ri[MAXNS];
     int thermo; // 1 NASA-9, 0 JANAF
     int fast;   // every coefficient is 0 or within [2^-300, 2^300], every W within [2^-80, 2^80] (xf_set_thermo)

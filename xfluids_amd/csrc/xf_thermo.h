@@ -157,22 +157,21 @@ template <bool NASA>
 __device__ __forceinline__ double h_fast(cdouble *c, double T, double iT, double lT, double Ri)
 {
     if (NASA)
-        return Ri * (dquot(-c[0], T, iT) + c[1] * lT +
-                     (c[2] + (0.5 * c[3] + (c[4] * OT + (0.25 * c[5] + 0.2 * c[6] * T) * T) * T) * T) * T + c[7]);
-    return Ri * (T * (c[0] + T * (c[1] * 0.5 + T * (c[2] * OT + T * (c[3] * 0.25 + c[4] * T * 0.2)))) + c[5]);
+        return Ri * (dquot(-c[0], T, iT) + c[1] * lT + (c[2] + (c[9] + (c[10] + (c[11] + c[12] * T) * T) * T) * T) * T +
+                     c[7]);
+    return Ri * (T * (c[0] + T * (c[9] + T * (c[10] + T * (c[11] + c[4] * T * 0.2)))) + c[5]);
 }
 template <bool NASA>
 __device__ __forceinline__ double s_fast(cdouble *c, double T, double iT, double lT)
 {
     if (NASA)
-        return ((-0.5 * c[0] * iT - c[1]) * iT + c[2] * lT +
-                (c[3] + (0.5 * c[4] + (c[5] * OT + c[6] * 0.25 * T) * T) * T) * T + c[8]);
-    return (c[0] * lT + (c[1] + (0.5 * c[2] + (c[3] * OT + c[4] * 0.25 * T) * T) * T) * T + c[6]);
+        return ((c[13] * iT - c[1]) * iT + c[2] * lT + (c[3] + (c[14] + (c[15] + c[16] * T) * T) * T) * T + c[8]);
+    return (c[0] * lT + (c[1] + (c[14] + (c[15] + c[16] * T) * T) * T) * T + c[6]);
 }
 
 // The per-temperature values of the fast fits.  ok: the table qualifies and
 // every active lane has 200 K <= T <= 1e5 K.  each(body) runs body(c) with the
-// coefficients of the lane's fit range at c + 9 * species, c the same on every
+// coefficients of the lane's fit range at c + FITC * species, c the same on every
 // lane that runs it together (scalar loads shared by the wave): once for a wave
 // in one range, once per range for a wave that straddles a limit.
 template <bool NASA> struct FastT {
@@ -196,7 +195,7 @@ template <bool NASA> struct FastT {
         for (int q = 0; q < (NASA ? 3 : 2); q++) {
             int ru = q; // hidden from the compiler, which would put r for q in the address
             asm volatile("" : "+s"(ru));
-            if (r == q) body(as_const(th->Hc + ru * (MAXNS * 9)));
+            if (r == q) body(as_const(th->Hf + ru * (MAXNS * FITC)));
         }
     }
 };
@@ -251,7 +250,9 @@ __device__ __forceinline__ double mix_gamma_cp(const DevThermo *__restrict__ th,
 // invariant and hoisted (same value every iteration).  A launch on few cells
 // lasts as long as its longest Newton chain (the step of T is limited, so a cell
 // behind a shock takes tens of iterations), a launch on many is bound by the
-// FP64 issue of the sums; the fast fits shorten both.
+// FP64 issue of the sums; the fast fits shorten both.  With the products of the
+// coefficients and the fits' constants in the table k_states takes 61 us instead of
+// 63 at 80 x 40 x 40 and five species.
 template <int NS, bool NASA>
 __device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, const double *yi, double e, double T0)
 {
@@ -268,8 +269,8 @@ __device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, co
 #pragma unroll
                 for (int n = 0; n < NS; n++) {
                     const double Ri = Rk[n];
-                    h += h_fast<NASA>(c + 9 * n, T, ft.iT, ft.lT, Ri) * yi[n];
-                    Cp += yi[n] * cp_fast<NASA>(c + 9 * n, T, ft.iT, Ri);
+                    h += h_fast<NASA>(c + FITC * n, T, ft.iT, ft.lT, Ri) * yi[n];
+                    Cp += yi[n] * cp_fast<NASA>(c + FITC * n, T, ft.iT, Ri);
                 }
             });
         } else {
