@@ -170,20 +170,20 @@ __device__ __forceinline__ double s_fast(cdouble *c, double T, double iT, double
 }
 
 // The per-temperature values of the fast fits.  ok: the table qualifies and
-// every active lane has 200 K <= T <= 1e5 K.  each(body) runs body(c) with the
-// coefficients of the lane's fit range at c + FITC * species, c the same on every
-// lane that runs it together (scalar loads shared by the wave): once for a wave
+// every active lane with run set has 200 K <= T <= 1e5 K.  each(body) runs body(c)
+// with the coefficients of the lane's fit range at c + FITC * species, c the same on
+// every lane that runs it together (scalar loads shared by the wave): once for a wave
 // in one range, once per range for a wave that straddles a limit.
 template <bool NASA> struct FastT {
     double T, iT, lT;
     const DevThermo *__restrict__ th;
     bool ok;
     // fast_: th_->fast, read once by the caller
-    __device__ __forceinline__ FastT(const DevThermo *__restrict__ th_, int fast_, double T_)
+    __device__ __forceinline__ FastT(const DevThermo *__restrict__ th_, int fast_, double T_, bool run = true)
     {
         th = th_;
         T = T_;
-        ok = fast_ && __all(T >= 200.0 && T <= 1.0e5);
+        ok = fast_ && __all(!run || (T >= 200.0 && T <= 1.0e5));
     }
     template <class F> __device__ __forceinline__ void each(bool need_log, F body)
     {
@@ -252,18 +252,23 @@ __device__ __forceinline__ double mix_gamma_cp(const DevThermo *__restrict__ th,
 // behind a shock takes tens of iterations), a launch on many is bound by the
 // FP64 issue of the sums; the fast fits shorten both.  With the products of the
 // coefficients and the fits' constants in the table k_states takes 61 us instead of
-// 63 at 80 x 40 x 40 and five species.
+// 63 at 80 x 40 x 40 and five species, and with converged lanes kept on 54; at
+// 60 x 40 x 36 52 instead of 63.
 template <int NS, bool NASA>
 __device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, const double *yi, double e, double T0)
 {
-    double T = T0;
+    double T = T0, root = T0;
     const double R = mix_R<NS>(th, yi);
     const int fast = th->fast;
     cdouble *Rk = as_const(th->Ri);
+    bool run = true;
     for (int it = 1; it < 101; it++) {
         double h = 0.0;
         double Cp = 0.0;
-        FastT<NASA> ft(th, fast, T);
+        // a lane that has converged goes on about its root, past the result: with the
+        // last few cells alone active a wave runs at half speed on an otherwise idle
+        // chip
+        FastT<NASA> ft(th, fast, T, run);
         if (ft.ok) {
             ft.each(NASA, [&](cdouble *c) {
 #pragma unroll
@@ -289,9 +294,11 @@ __device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, co
         double df = dmin(func_T / (dfunc_T + 1.0e-30), 1e-3 * T);
         df = dmax(df, -1e-2 * T);
         T = T - df;
-        if (fabs(df) <= 1.0e-6) break;
+        root = run ? T : root;
+        run = run && !(fabs(df) <= 1.0e-6);
+        if (!__any(run)) break;
     }
-    return T;
+    return root;
 }
 template <int NS>
 __device__ __forceinline__ double get_T(const DevThermo *__restrict__ th, const double *yi, double e, double T0)
