@@ -233,12 +233,11 @@ void lu_async(xf_ctx *c, const double *Ug, int rk_stage, const double *Ua, const
 
 void reaction_prep_async(xf_ctx *c);
 
-// XFLUIDS::Reaction before its chemistry launch: UpdateStates(U) and the
-// device-side chemistry step (dt/2 for Strang)
+// XFLUIDS::Reaction before its chemistry launch: UpdateStates(U) (the step's
+// k_dt has set the chemistry step)
 void reaction_prep_async(xf_ctx *c)
 {
     states_async(c, c->f.U, 0, 0, 4);
-    hipLaunchKernelGGL(k_dt_chem, dim3(1), dim3(64), 0, c->stream, c->f.dt, c->d.strang, c->f.err);
 }
 
 // A step is: dt; [Strang: Reaction]; three RK stages; [Reaction].  The parts
@@ -246,7 +245,7 @@ void reaction_prep_async(xf_ctx *c)
 // can launch one chemistry kernel for all its cases at each Reaction.
 void step_pre_async(xf_ctx *c)
 {
-    hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, c->stream, c->g, c->f.red, c->f.dt, c->f.err, 1);
+    hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, c->stream, c->g, c->f, 1, c->d.strang);
     if (c->d.react && c->d.strang) reaction_prep_async(c);
 }
 
@@ -369,6 +368,7 @@ int xf_create(const xf_case_desc *desc, xf_ctx **out)
     for (auto pp : dbl)
         if (hipMemset(*pp, 0, n1)) return fail(XF_EHIP);
     if (hipMemset(f.hi, 0, (size_t)d.NS * n1) || hipMemset(f.red, 0, RED_SIZE * sizeof(double)) ||
+        hipMemset(f.spart, 0, (size_t)nblk(c->N) * 12 * sizeof(double)) ||
         hipMemset(f.substeps, 0, (size_t)c->Ninner * sizeof(int)))
         return fail(XF_EHIP);
     if (hipDeviceSynchronize()) return fail(XF_EHIP);
@@ -726,6 +726,11 @@ int xf_download_maxima(xf_ctx *c, double *eigen_block, double *uvw_c_max)
 {
     if (!c) return XF_EINVAL;
     double red[RED_SIZE];
+    // the CFL maxima of the last pass, which a step's own kernels may have folded
+    // for themselves
+    hipLaunchKernelGGL(k_states_fold, dim3(12), dim3(1024), 0, c->stream, c->f.spart, state_blocks(c->g), c->f.red,
+                       c->f.err);
+    if (int e = check_launch()) return e;
     XF_HIP(hipStreamSynchronize(c->stream));
     XF_HIP(hipMemcpy(red, c->f.red, sizeof(red), hipMemcpyDeviceToHost));
     const int E = c->E;
@@ -783,7 +788,7 @@ int xf_rk3_stage(xf_ctx *c, int stage, double dt)
 int xf_get_dt(xf_ctx *c, double *dt_out)
 {
     if (!c || !dt_out) return XF_EINVAL;
-    hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, c->stream, c->g, c->f.red, c->f.dt, c->f.err, 0);
+    hipLaunchKernelGGL(k_dt, dim3(1), dim3(64), 0, c->stream, c->g, c->f, 0, 0);
     if (int e = check_launch()) return e;
     XF_HIP(hipMemcpyAsync(dt_out, c->f.dt, sizeof(double), hipMemcpyDeviceToHost, c->stream));
     XF_HIP(hipStreamSynchronize(c->stream));
@@ -950,21 +955,26 @@ int xf_set_profiling(xf_ctx *c, int on)
 }
 
 namespace {
-// the GLF/CFL reduction slots, saved around measurement launches so that a
-// timing or tuning run leaves the running GLF maxima exactly as it found them
+// the GLF/CFL reduction slots and the last pass's partial maxima, saved around
+// measurement launches so that a timing or tuning run leaves the running GLF maxima
+// and the next dt exactly as it found them
 struct RedGuard {
     xf_ctx *c;
     double h[RED_SIZE];
+    std::vector<double> part;
     bool ok;
-    explicit RedGuard(xf_ctx *c_) : c(c_)
+    explicit RedGuard(xf_ctx *c_) : c(c_), part((size_t)state_blocks(c_->g) * 12)
     {
         ok = hipMemcpyAsync(h, c->f.red, sizeof(h), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
+             hipMemcpyAsync(part.data(), c->f.spart, part.size() * sizeof(double), hipMemcpyDeviceToHost,
+                            c->stream) == hipSuccess &&
              hipStreamSynchronize(c->stream) == hipSuccess;
     }
     ~RedGuard()
     {
         if (ok) {
             (void)hipMemcpyAsync(c->f.red, h, sizeof(h), hipMemcpyHostToDevice, c->stream);
+            (void)hipMemcpyAsync(c->f.spart, part.data(), part.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
             (void)hipStreamSynchronize(c->stream);
         }
     }
@@ -1183,6 +1193,7 @@ struct xf_ensemble {
     void *spill = nullptr; // hand-over list of the shared chemistry queue
     int spill_cap = 0;
     long long state_blocks = 0, tiles[3] = {0, 0, 0};
+    bool fold = false; // some case has more than FOLD_BLOCKS blocks
     int shape[3] = {0, 0, 0};
 };
 
@@ -1218,10 +1229,9 @@ void ens_step_multi(xf_ensemble *e)
     xf_ctx *c0 = e->cases[0];
     const int n = (int)e->cases.size();
     hipStream_t st = e->stream;
-    hipLaunchKernelGGL(k_dt_multi, dim3(1), dim3(64), 0, st, e->d_ens, n);
+    hipLaunchKernelGGL(k_dt_multi, dim3((unsigned)n), dim3(64), 0, st, e->d_ens, c0->d.strang);
     auto reaction = [&]() {
-        c0->ops.states_multi(c0, st, e->d_ens, n, e->state_blocks, 0, 0, 4, 0);
-        hipLaunchKernelGGL(k_dt_chem_multi, dim3(1), dim3(64), 0, st, e->d_ens, n, c0->d.strang);
+        c0->ops.states_multi(c0, st, e->d_ens, n, e->state_blocks, 0, 0, 4, 0, e->fold);
         ens_chem(e);
     };
     if (e->react && e->strang) reaction();
@@ -1233,7 +1243,7 @@ void ens_step_multi(xf_ensemble *e)
     // step_mid_async; at stage 1 the sweep's Ub is U2 (the NaN check's U1)
     const int in_sel[3] = {0, 1, 2}, out_sel[3] = {1, 2, 0};
     for (int s = 1; s <= 3; s++) {
-        c0->ops.states_multi(c0, st, e->d_ens, n, e->state_blocks, 0, 1, s, in_sel[s - 1]);
+        c0->ops.states_multi(c0, st, e->d_ens, n, e->state_blocks, 0, 1, s, in_sel[s - 1], e->fold);
         for (int q = 0; q < nd; q++) {
             int mode = (q > 0) ? 1 : 0;
             if (q == nd - 1) mode |= 2;
@@ -1351,6 +1361,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
             r.U2 = c->U2;
             r.state_off = sb;
             sb += nblk(c->N);
+            e->fold = e->fold || state_blocks(c->g) > FOLD_BLOCKS;
             int bcs = 0;
             for (int q = 0; q < 6; q++) bcs |= (c->d.BC[q] & 15) << (4 * q);
             r.bcs = bcs | (1 << 28);

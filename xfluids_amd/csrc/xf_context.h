@@ -46,8 +46,9 @@ struct Ops {
     // one launch over every case of an ensemble (case table on the device;
     // sel codes pick U, U1 or U2 per case; the scheme, precision and tile
     // shape are those of the template case c0)
+    // fold: some case's blocks are too many for the sweeps to fold
     void (*states_multi)(const xf_ctx *c0, hipStream_t, const EnsCase *, int ncases, long long blocks, int full,
-                         int fill, int where, int sel);
+                         int fill, int where, int sel, bool fold);
     void (*sweep_multi)(const xf_ctx *c0, hipStream_t, const EnsCase *, int ncases, long long blocks, int dir, int shape,
                         int mode, int stage, int sel_g, int sel_a, int sel_b, int sel_o);
     // the sweeps compute the wall flux themselves when Geom::visc_fused is set
@@ -212,8 +213,9 @@ template <int NS, bool COP> struct Launch {
                 hipLaunchKernelGGL((k_rhoyi_writeback<NS>), dim3(nblk(c->N)), dim3(256), 0, c->stream, c->g, U,
                                    c->f);
         }
-        hipLaunchKernelGGL(k_states_fold, dim3(12), dim3(1024), 0, c->stream, c->f.spart, (int)nblk(c->N), c->f.red,
-                           c->f.err);
+        if (state_blocks(c->g) > FOLD_BLOCKS)
+            hipLaunchKernelGGL(k_states_fold, dim3(12), dim3(1024), 0, c->stream, c->f.spart, state_blocks(c->g),
+                               c->f.red, c->f.err);
     }
     static void sweep(xf_ctx *c, int dir, const double *Ug, int mode, int stage, const double *Ua, const double *Ub,
                       double *Uo)
@@ -337,23 +339,20 @@ template <int NS, bool COP> struct Launch {
             else
                 hipLaunchKernelGGL((k_transport<NS, 0>), dim3(nblk(c->N)), dim3(256), 0, c->stream, g, c->d_th,
                                    c->d_tr, Ug, c->f, c->d.visc_heat, c->d.visc_diffu);
-            if (c->d.visc_diffu)
-                hipLaunchKernelGGL((k_yreduce<NS>), dim3(2 * NS), dim3(1024), 0, c->stream, c->f.ypart,
-                                   (int)nblk(c->N), c->f.red);
             const int i0 = g.DimX ? g.Bx - 2 : 0, nx = g.DimX ? g.X_inner + 4 : 1;
             const int j0 = g.DimY ? g.By - 2 : 0, ny = g.DimY ? g.Y_inner + 4 : 1;
             const int k0 = g.DimZ ? g.Bz - 2 : 0, nz = g.DimZ ? g.Z_inner + 4 : 1;
             const int *bc = c->d.BC;
             // the mixed form stores the gradients (and the transport
             // coefficients) as FP32 planes
-            if (c->d.precision == XF_MIXED)
-                hipLaunchKernelGGL((k_vel_deriv<XF_MIXED>), dim3(nblk((long long)nx * ny * nz)), dim3(256), 0,
-                                   c->stream, g, c->f, i0, nx, j0, ny, k0, nz, bc[0], bc[1], bc[2], bc[3], bc[4],
-                                   bc[5]);
-            else
-                hipLaunchKernelGGL((k_vel_deriv<XF_PLAIN_FP64>), dim3(nblk((long long)nx * ny * nz)), dim3(256), 0,
-                                   c->stream, g, c->f, i0, nx, j0, ny, k0, nz, bc[0], bc[1], bc[2], bc[3], bc[4],
-                                   bc[5]);
+            const int ns = c->d.visc_diffu ? NS : 0;
+            const unsigned blocks = nblk((long long)nx * ny * nz) + 2u * ns;
+            auto deriv = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, c->stream, g, c->f, i0, nx, j0, ny, k0, nz, bc[0],
+                                   bc[1], bc[2], bc[3], bc[4], bc[5], ns, (int)nblk(c->N));
+            };
+            if (c->d.precision == XF_MIXED) deriv(k_vel_deriv<XF_MIXED>);
+            else deriv(k_vel_deriv<XF_PLAIN_FP64>);
         }
     }
     template <int DIR> static void visc_flux_d(xf_ctx *c, const double *Ug)
@@ -380,11 +379,11 @@ template <int NS, bool COP> struct Launch {
         }
     }
     static void states_multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
-                             int full, int fill, int where, int sel)
+                             int full, int fill, int where, int sel, bool fold)
     {
         hipLaunchKernelGGL((k_states_multi<NS, COP>), dim3((unsigned)blocks), dim3(256), 0, st, cases, ncases, c0->d_th,
                            c0->d.ncop_gamma, full, fill, where, sel);
-        hipLaunchKernelGGL(k_states_fold_multi, dim3((unsigned)(12 * ncases)), dim3(1024), 0, st, cases);
+        if (fold) hipLaunchKernelGGL(k_states_fold_multi, dim3((unsigned)(12 * ncases)), dim3(1024), 0, st, cases);
     }
     static void sweep_multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
                             int dir, int shape, int mode, int stage, int sg, int sa, int sb, int so)

@@ -219,6 +219,82 @@ static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__r
 }
 
 // ---------------------------------------------------------------------------
+// the GLF and CFL maxima of an UpdateStates pass
+// ---------------------------------------------------------------------------
+// Each block of k_states leaves its maxima in spart, one plane per slot (9 GLF, 3
+// CFL).  A slot's value is the maximum of +0 and every positive block value (the
+// pass's maxima, combined with the 0 the pass starts from).
+//
+// Up to FOLD_BLOCKS blocks the kernels that use the values (the sweeps, k_dt) fold
+// the planes themselves, each wave on its own while its first loads are in flight;
+// k_states_fold then runs only where the host reads the slots.  A launch costs 4.5 us
+// here however little it does: a 64 x 64 vortex step takes 72.2 us
+// instead of 76.6, 253 x 190 (202 blocks) 74.5 instead of 79.8.  At 468 blocks a sweep
+// takes 1.3 us longer for it, which is where the line lies: a step 106.7 instead of
+// 107.5.
+constexpr int FOLD_BLOCKS = 512;
+__host__ __device__ inline int state_blocks(const Geom &g) { return (int)((g.N + 255) / 256); }
+
+// slots q, q + 1, q + 2, the same on every lane; run by whole waves
+__device__ __forceinline__ void pass_maxima(const double *__restrict__ spart, int nb, int q, double *out)
+{
+    double m[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x & 63; b < nb; b += 256) {
+        double x[3][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) x[k][u] = spart[(q + k) * nb + (b + 64 * u < nb ? b + 64 * u : b)];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int k = 0; k < 3; k++) m[k] = fmax(m[k], x[k][u]);
+    }
+    double r;
+    wave_fold<4>(m, &r, [](double a, double b) { return fmax(a, b); });
+#pragma unroll
+    for (int k = 0; k < 3; k++) { // value k is on row wave_fold_index's k
+        const int lane = 16 * (((k & 1) << 1) + (k >> 1));
+        out[k] = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(r), lane),
+                                  __builtin_amdgcn_readlane(__double2loint(r), lane));
+    }
+}
+
+// The fold as a launch: one block per slot (12)
+__device__ __forceinline__ void states_fold(const double *__restrict__ spart, int nblocks, double *red, int *err, int q)
+{
+    __shared__ unsigned long long s[1024];
+    // latch a failure of the UpdateStates pass (or of any earlier one)
+    if (q == 0 && threadIdx.x == 0 && err[ERR_BITS]) err[ERR_HALT] = 1;
+    unsigned long long v = 0ULL; // +0.0
+    for (int b = threadIdx.x; b < nblocks; b += 1024) {
+        const double x = spart[(long long)q * nblocks + b];
+        const unsigned long long bx = (unsigned long long)__double_as_longlong(x);
+        if (x > 0.0 && bx > v) v = bx;
+    }
+    s[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = 512; w >= 1; w >>= 1) {
+        if (threadIdx.x < w && s[threadIdx.x + w] > s[threadIdx.x]) s[threadIdx.x] = s[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) red[q < 9 ? RED_GLFP + q : RED_DT + q - 9] = __longlong_as_double((long long)s[0]);
+}
+
+static __global__ void __launch_bounds__(1024) k_states_fold(const double *__restrict__ spart, int nblocks, double *red,
+                                                             int *err)
+{
+    states_fold(spart, nblocks, red, err, blockIdx.x);
+}
+
+// the folds of every case: 12 blocks per case
+static __global__ void __launch_bounds__(1024) k_states_fold_multi(const EnsCase *__restrict__ cases)
+{
+    const EnsCase &c = cases[blockIdx.x / 12];
+    states_fold(c.f.spart, state_blocks(c.g), c.f.red, c.f.err, blockIdx.x % 12);
+}
+
+// ---------------------------------------------------------------------------
 // conservative -> primitive over all padded cells
 // ---------------------------------------------------------------------------
 // bcs: 0 = the ghost cells already hold their values; otherwise the six BC
@@ -421,13 +497,13 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
         if (ebits & EBIT_PRIM) report_cell(f.err, EBIT_PRIM, id);
     }
     __syncthreads();
-    // the block's maxima go to spart; k_states_fold combines the blocks (one
-    // pass over the partials instead of same-address atomics from every block)
+    // the block's maxima (pass_maxima or k_states_fold combines the blocks, instead
+    // of same-address atomics from every block)
     if (threadIdx.x < 12) {
         double m = sred[0][threadIdx.x];
         const int nw = (blockDim.x + 63) >> 6;
         for (int q = 1; q < nw; q++) m = sred[q][threadIdx.x] > m ? sred[q][threadIdx.x] : m;
-        f.spart[bid * 12 + threadIdx.x] = m;
+        f.spart[(long long)threadIdx.x * state_blocks(g) + bid] = m;
     }
     if (threadIdx.x == 0 && serr) report_pass(f.err, serr, where);
 }
@@ -443,7 +519,7 @@ __global__ void __launch_bounds__(256) k_states(Geom g, const DevThermo *__restr
 // padded cell: U_{5+k} = rho * Y_k with the fractions k_states stored.  A
 // launch of its own after k_states, whose ghost fill reads interior cells as
 // its sources; it runs exactly when k_states did (the same entry test, and
-// before k_states_fold latches this pass's failures).
+// before a later kernel latches this pass's failures).
 template <int NS>
 __global__ void __launch_bounds__(256) k_rhoyi_writeback(Geom g, double *Ug, Fields f)
 {
@@ -468,42 +544,6 @@ __global__ void __launch_bounds__(256) k_states_multi(const EnsCase *__restrict_
     states_block<NS, COP>(c.g, th, c.buf(sel), c.f, ncop_gamma, full, fill ? c.bcs : 0, where, b - c.state_off);
 }
 
-// the per-block GLF and CFL maxima of k_states into the reduction slots: one
-// block per slot (12), each the maximum of +0 and every positive block value
-// (the pass's maxima, combined with the 0 the pass starts from)
-__device__ __forceinline__ void states_fold(const double *__restrict__ spart, int nblocks, double *red, int *err, int q)
-{
-    __shared__ unsigned long long s[1024];
-    // latch a failure of the UpdateStates pass (or of any earlier one)
-    if (q == 0 && threadIdx.x == 0 && err[ERR_BITS]) err[ERR_HALT] = 1;
-    unsigned long long v = 0ULL; // +0.0
-    for (int b = threadIdx.x; b < nblocks; b += 1024) {
-        const double x = spart[(long long)b * 12 + q];
-        const unsigned long long bx = (unsigned long long)__double_as_longlong(x);
-        if (x > 0.0 && bx > v) v = bx;
-    }
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = 512; w >= 1; w >>= 1) {
-        if (threadIdx.x < w && s[threadIdx.x + w] > s[threadIdx.x]) s[threadIdx.x] = s[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) red[q < 9 ? RED_GLFP + q : RED_DT + q - 9] = __longlong_as_double((long long)s[0]);
-}
-
-static __global__ void __launch_bounds__(1024) k_states_fold(const double *__restrict__ spart, int nblocks, double *red,
-                                                             int *err)
-{
-    states_fold(spart, nblocks, red, err, blockIdx.x);
-}
-
-// the folds of every case: 12 blocks per case
-static __global__ void __launch_bounds__(1024) k_states_fold_multi(const EnsCase *__restrict__ cases)
-{
-    const EnsCase &c = cases[blockIdx.x / 12];
-    states_fold(c.f.spart, (int)((c.g.N + 255) / 256), c.f.red, c.f.err, blockIdx.x % 12);
-}
-
 // ---------------------------------------------------------------------------
 // small control kernels
 // ---------------------------------------------------------------------------
@@ -514,9 +554,17 @@ static __global__ void __launch_bounds__(1024) k_states_fold_multi(const EnsCase
 // target_t); otherwise the step is counted (Iteration++), dt is clamped so
 // that the clock lands on the target (physicalTime + dt > target_t ->
 // dt = target_t - physicalTime) and the clock advances.  It also latches a
-// failure of the previous pass into ERR_HALT.  step = 0 is GetDt alone.
-__device__ __forceinline__ void dt_case(const Geom &g, double *red, double *dt, int *err, int step)
+// failure of the previous pass into ERR_HALT, and sets the chemistry step of the
+// step's Reactions, dt / 2 or (Lie) dt.  step = 0 is GetDt alone.
+// One wave.
+__device__ __forceinline__ void dt_case(const Geom &g, const Fields &f, int step, int strang)
 {
+    double *red = f.red, *dt = f.dt;
+    int *err = f.err;
+    double cfl[3];
+    if (state_blocks(g) <= FOLD_BLOCKS) pass_maxima(f.spart, state_blocks(g), 9, cfl);
+    else cfl[0] = red[RED_DT + 0], cfl[1] = red[RED_DT + 1], cfl[2] = red[RED_DT + 2];
+    if (threadIdx.x != 0) return;
     if (step) {
         if (err[ERR_BITS]) err[ERR_HALT] = 1;
         if (err[ERR_HALT]) return;
@@ -528,43 +576,31 @@ __device__ __forceinline__ void dt_case(const Geom &g, double *red, double *dt, 
         }
         err[ERR_COUNT] = err[ERR_COUNT] + 1;
     }
-    const double mx = g.DimX ? red[RED_DT + 0] : 0.0;
-    const double my = g.DimY ? red[RED_DT + 1] : 0.0;
-    const double mz = g.DimZ ? red[RED_DT + 2] : 0.0;
+    const double mx = g.DimX ? cfl[0] : 0.0;
+    const double my = g.DimY ? cfl[1] : 0.0;
+    const double mz = g.DimZ ? cfl[2] : 0.0;
     const double dtref = mx * g._dx + my * g._dy + mz * g._dz;
     double d = g.CFL / dtref;
     if (step) {
         const double t = dt[DT_TIME], te = dt[DT_TARGET];
         if (t + d > te) d = te - t;
         dt[DT_TIME] = t + d;
+        dt[DT_CHEM] = strang ? d * 0.5 : d;
     }
     dt[DT_STEP] = d;
     // uvw_c_max as GetDt leaves it (the positivity limiter's lambda_0)
     red[RED_LAM + 0] = mx, red[RED_LAM + 1] = my, red[RED_LAM + 2] = mz;
 }
 
-static __global__ void k_dt(Geom g, double *red, double *dt, int *err, int step)
+static __global__ void __launch_bounds__(64) k_dt(Geom g, Fields f, int step, int strang)
 {
-    if (threadIdx.x == 0) dt_case(g, red, dt, err, step);
+    dt_case(g, f, step, strang);
 }
 
-// Strang half step on device: dt[1] = dt[0] * 0.5 (or dt[0] for Lie)
-static __global__ void k_dt_chem(double *dt, int strang, const int *err)
+// the head of a step of every case of an ensemble, one block per case
+static __global__ void __launch_bounds__(64) k_dt_multi(const EnsCase *__restrict__ cases, int strang)
 {
-    if (threadIdx.x == 0 && !step_halted(err, ~0)) dt[DT_CHEM] = strang ? dt[DT_STEP] * 0.5 : dt[DT_STEP];
-}
-
-// the same two for every case of an ensemble, one lane per case
-static __global__ void k_dt_multi(const EnsCase *__restrict__ cases, int ncases)
-{
-    for (int k = threadIdx.x; k < ncases; k += blockDim.x) dt_case(cases[k].g, cases[k].f.red, cases[k].f.dt, cases[k].f.err, 1);
-}
-static __global__ void k_dt_chem_multi(const EnsCase *__restrict__ cases, int ncases, int strang)
-{
-    for (int k = threadIdx.x; k < ncases; k += blockDim.x) {
-        const Fields &f = cases[k].f;
-        if (!step_halted(f.err, ~0)) f.dt[DT_CHEM] = strang ? f.dt[DT_STEP] * 0.5 : f.dt[DT_STEP];
-    }
+    dt_case(cases[blockIdx.x].g, cases[blockIdx.x].f, 1, strang);
 }
 
 // ---------------------------------------------------------------------------

@@ -95,7 +95,7 @@ struct Fields {
     // first NS - 1 species (NS - 1 planes) as the last UpdateStates formed
     // them; the ghost species' own is 0
     double *y;
-    double *spart; // per-block GLF and CFL maxima of k_states (12 per block)
+    double *spart; // per-block GLF and CFL maxima of k_states (12 planes)
 };
 
 // One case of an ensemble as the ensemble's launches see it: geometry,
@@ -201,10 +201,14 @@ __device__ __forceinline__ void cell_y(const Geom &g, const Fields &f, long long
 }
 
 // the step kernels' entry test: a halted step, or a failure recorded by an
-// earlier launch (bits in mask are those the calling kernel never sets)
-__device__ __forceinline__ bool step_halted(const int *err, int mask)
+// earlier launch (bits in mask are those the calling kernel never sets), which it
+// latches for the later kernels that do not test its bit
+__device__ __forceinline__ bool step_halted(int *err, int mask)
 {
-    return err[ERR_HALT] != 0 || (err[ERR_BITS] & mask) != 0;
+    if (err[ERR_HALT] != 0) return true;
+    if ((err[ERR_BITS] & mask) == 0) return false;
+    err[ERR_HALT] = 1;
+    return true;
 }
 
 // record a failing cell: the bit, the lowest id per bit, the step and stage

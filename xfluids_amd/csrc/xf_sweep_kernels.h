@@ -482,14 +482,14 @@ namespace xf {
 // GLF dissipation of characteristic field n (Artificial_type 3): the running
 // maximum of |eigen_local[n]|; fields 1..E-2 share the |u_n| maximum.
 // GetLU's GLF reduction happens here: the running maximum is folded with
-// the maximum of the last UpdateStates pass.  Every block computes the same
-// max(running, pass) and block 0 stores it back; readers before or after the
-// store see the same value (max is idempotent).
+// the maximum of the last UpdateStates pass (pass, the direction's three).  Every
+// block computes the same max(running, pass) and block 0 stores it back; readers
+// before or after the store see the same value (max is idempotent).
 template <int DIR, int E>
-__device__ __forceinline__ double glf_alpha(const double *red, int n)
+__device__ __forceinline__ double glf_alpha(const double *red, const double *pass, int n)
 {
-    const int q = 3 * DIR + (n == 0 ? 0 : (n == E - 1 ? 2 : 1));
-    const double a = red[RED_GLF + q], b = red[RED_GLFP + q];
+    const int q = n == 0 ? 0 : (n == E - 1 ? 2 : 1);
+    const double a = red[RED_GLF + 3 * DIR + q], b = pass[q];
     return b > a ? b : a;
 }
 
@@ -666,6 +666,12 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
             }
         }
     }
+    // the direction's GLF maxima of the pass, folded while the cells arrive
+    double pass[3];
+    if (state_blocks(g) <= FOLD_BLOCKS) pass_maxima(f.spart, state_blocks(g), 3 * DIR, pass);
+    else
+#pragma unroll
+        for (int k = 0; k < 3; k++) pass[k] = f.red[RED_GLFP + 3 * DIR + k];
 #pragma unroll
     for (int it = 0; it < NIT; it++) {
         if (tid + 256 * it >= NC) continue;
@@ -736,7 +742,7 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
     __syncthreads();
 
     if (tx == 0 && ty == 0 && tz == 0 && tid < 3) {
-        const double a = f.red[RED_GLF + 3 * DIR + tid], b = f.red[RED_GLFP + 3 * DIR + tid];
+        const double a = f.red[RED_GLF + 3 * DIR + tid], b = tid == 0 ? pass[0] : (tid == 1 ? pass[1] : pass[2]);
         f.red[RED_GLF + 3 * DIR + tid] = b > a ? b : a;
     }
 
@@ -819,8 +825,9 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
             return (double)weno_face_f32<SCHEME>(pp, mm, (float)dl);
         };
         // GLF dissipation of the three families of fields, on scalar registers
-        const double av_m = uniform(glf_alpha<DIR, E>(f.red, 0)), av_u = uniform(glf_alpha<DIR, E>(f.red, 1)),
-                     av_p = uniform(glf_alpha<DIR, E>(f.red, E - 1));
+        const double av_m = uniform(glf_alpha<DIR, E>(f.red, pass, 0)),
+                     av_u = uniform(glf_alpha<DIR, E>(f.red, pass, 1)),
+                     av_p = uniform(glf_alpha<DIR, E>(f.red, pass, E - 1));
         // LDS index of the first of the face's six points (the others follow at
         // STEP), as a value of its own in every row: the compiler would keep the
         // values that several rows read, and spill them

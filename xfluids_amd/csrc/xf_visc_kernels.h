@@ -7,9 +7,9 @@
 //   k_transport<NS,PREC> every padded cell: u, v, w, Wilke mu and lambda, D_km
 //                     (PREC 1: the mixed form's FP32 exponentials and factors);
 //                     per-block min/max of each interior mass fraction
-//   k_yreduce<NS>     one block: those partials into the reduction slots
-//   k_vel_deriv<PREC> fourth-order centre derivatives of u, v, w, with the
-//                     ghost-cell rules for the values each wall flux reads
+//   k_vel_deriv<PREC> those partials into the reduction slots; fourth-order
+//                     centre derivatives of u, v, w, with the ghost-cell rules
+//                     for the values each wall flux reads
 //   visc_face<NS,DIR,PREC> per face of one direction, inside the sweep of
 //                     that direction (NS >= 4), or k_visc_flux<NS,DIR,PREC>
 //                     writing the flux planes the sweep subtracts
@@ -407,25 +407,26 @@ k_transport(Geom g, const DevThermo *__restrict__ th, const DevTransport *__rest
 // the per-block partials of k_transport into red[RED_YMIN + k] (min) and
 // red[RED_YMAX + k] (max), each combined with 0.0 as the reference's
 // sycl::reduction combines with the stored yi_min = yi_max = 0; one block per
-// quantity (2 NS blocks)
-template <int NS>
-__global__ void __launch_bounds__(1024) k_yreduce(const double *__restrict__ ypart, int nblocks, double *red)
+// quantity q (the minima, then the maxima, of ns species)
+__device__ __forceinline__ void y_fold(const double *__restrict__ ypart, int nblocks, int ns, int q, double *red)
 {
-    __shared__ double s[1024];
-    const int q = blockIdx.x;
-    const bool mx = q >= NS;
+    __shared__ double s[256];
+    const bool mx = q >= ns;
     double v = 0.0;
-    for (int b = threadIdx.x; b < nblocks; b += 1024) {
-        const double x = ypart[(long long)b * 2 * NS + q];
-        v = mx ? smax(v, x) : smin(v, x);
+    for (int b = threadIdx.x; b < nblocks; b += 256 * 8) {
+        double x[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) x[u] = ypart[(long long)(b + 256 * u < nblocks ? b + 256 * u : b) * 2 * ns + q];
+#pragma unroll
+        for (int u = 0; u < 8; u++) v = mx ? smax(v, x[u]) : smin(v, x[u]);
     }
     s[threadIdx.x] = v;
     __syncthreads();
-    for (int w = 512; w >= 1; w >>= 1) {
+    for (int w = 128; w >= 1; w >>= 1) {
         if (threadIdx.x < w) s[threadIdx.x] = mx ? smax(s[threadIdx.x], s[threadIdx.x + w]) : smin(s[threadIdx.x], s[threadIdx.x + w]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) red[mx ? RED_YMAX + q - NS : RED_YMIN + q] = s[0];
+    if (threadIdx.x == 0) red[mx ? RED_YMAX + q - ns : RED_YMIN + q] = s[0];
 }
 
 // fourth-order centre derivatives of u, v, w along direction a at cell id
@@ -462,9 +463,16 @@ __device__ __forceinline__ void centre_deriv(const Geom &g, const Fields &f, lon
 // x and y kernels (the reference's k - offset indexes outside the array).
 template <int PREC>
 __global__ void __launch_bounds__(256) k_vel_deriv(Geom g, Fields f, int i0, int nx, int j0, int ny, int k0,
-                                                          int nz, int bc0, int bc1, int bc2, int bc3, int bc4, int bc5)
+                                                          int nz, int bc0, int bc1, int bc2, int bc3, int bc4, int bc5,
+                                                          int ns, int ny_fold)
 {
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    // the first 2 ns blocks (0 without diffusion) fold the mass-fraction limits,
+    // which the gradients do not need: a launch of their own costs 4.8 us
+    if ((int)blockIdx.x < 2 * ns) {
+        y_fold(f.ypart, ny_fold, ns, (int)blockIdx.x, f.red);
+        return;
+    }
+    const long long t = ((long long)blockIdx.x - 2 * ns) * blockDim.x + threadIdx.x;
     if (t >= (long long)nx * ny * nz) return;
     if (step_halted(f.err, ~0)) return;
     const int c[3] = {i0 + (int)(t % nx), j0 + (int)((t / nx) % ny), k0 + (int)(t / ((long long)nx * ny))};
