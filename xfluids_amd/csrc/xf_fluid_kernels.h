@@ -235,20 +235,32 @@ static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__r
 constexpr int FOLD_BLOCKS = 512;
 __host__ __device__ inline int state_blocks(const Geom &g) { return (int)((g.N + 255) / 256); }
 
-// slots q, q + 1, q + 2, the same on every lane; run by whole waves
-__device__ __forceinline__ void pass_maxima(const double *__restrict__ spart, int nb, int q, double *out)
+// slots q, q + 1, q + 2, the same on every lane; run by whole waves.  The loads of
+// the first 256 blocks and the fold are apart, for a caller's own loads between.
+struct PassPart {
+    double x[3][4];
+};
+__device__ __forceinline__ PassPart pass_load(const double *__restrict__ spart, int nb, int q, int b0)
+{
+    PassPart l;
+    const int b = b0 + (threadIdx.x & 63);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) l.x[k][u] = spart[(q + k) * nb + min(b + 64 * u, nb - 1)];
+    return l;
+}
+__device__ __forceinline__ void pass_maxima(const double *__restrict__ spart, int nb, int q, PassPart l, double *out)
 {
     double m[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x & 63; b < nb; b += 256) {
-        double x[3][4];
+    for (int b0 = 0;;) {
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
-            for (int k = 0; k < 3; k++) x[k][u] = spart[(q + k) * nb + (b + 64 * u < nb ? b + 64 * u : b)];
-#pragma unroll
-        for (int u = 0; u < 4; u++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) m[k] = fmax(m[k], x[k][u]);
+            for (int k = 0; k < 3; k++) m[k] = fmax(m[k], l.x[k][u]);
+        b0 += 256;
+        if (b0 >= nb) break;
+        l = pass_load(spart, nb, q, b0);
     }
     double r;
     wave_fold<4>(m, &r, [](double a, double b) { return fmax(a, b); });
@@ -310,8 +322,8 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
 {
     constexpr int E = COP ? NS + 4 : 5;
     constexpr int NCOP = COP ? NS - 1 : 0;
-    // block-uniform: the words tested are not written by this launch
-    if (step_halted(f.err, ~(EBIT_RHO_Y | EBIT_PRIM))) return;
+    // tested once the first loads are on their way
+    const StepState step(f.err);
     const long long N = g.N;
     const long long id = bid * blockDim.x + threadIdx.x;
     const bool live = id < N;
@@ -321,12 +333,15 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
 #pragma unroll
     for (int q = 0; q < 3; q++) dtm[q] = 0.0;
     int ebits = 0;
+    int i = 0, j = 0, k = 0;
+    bool wb = false;
+    double U[E];
+#pragma unroll
+    for (int n = 0; n < E; n++) U[n] = 0.0;
     if (live) {
-        int i, j, k;
         cell_ijk(g, id, i, j, k);
         long long src = id;
         int flip = 0;
-        bool wb = false;
         if (bcs) {
             int si = i, sj = j, sk = k;
             auto bc = [&](int q) { return (bcs >> (4 * q)) & 15; };
@@ -338,12 +353,15 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
                 wb = true;
             }
         }
-        double U[E];
 #pragma unroll
         for (int n = 0; n < E; n++) {
             const double v = Ug[n * N + src];
             U[n] = ((flip >> n) & 1) ? -v : v;
         }
+    }
+    // block-uniform: the words tested are not written by this launch
+    if (step.halted(~(EBIT_RHO_Y | EBIT_PRIM))) return;
+    if (live) {
         if (wb) {
 #pragma unroll
             for (int n = 0; n < E; n++) Ug[n * N + id] = U[n];
@@ -512,6 +530,7 @@ template <int NS, bool COP>
 __global__ void __launch_bounds__(256) k_states(Geom g, const DevThermo *__restrict__ th, double *Ug, Fields f,
                                                 double ncop_gamma, int full, int bcs, int where)
 {
+    touch_args<sizeof(Geom) + sizeof(Fields) + 32>();
     states_block<NS, COP>(g, th, Ug, f, ncop_gamma, full, bcs, where, (long long)blockIdx.x);
 }
 
@@ -562,7 +581,8 @@ __device__ __forceinline__ void dt_case(const Geom &g, const Fields &f, int step
     double *red = f.red, *dt = f.dt;
     int *err = f.err;
     double cfl[3];
-    if (state_blocks(g) <= FOLD_BLOCKS) pass_maxima(f.spart, state_blocks(g), 9, cfl);
+    const int nb = state_blocks(g);
+    if (nb <= FOLD_BLOCKS) pass_maxima(f.spart, nb, 9, pass_load(f.spart, nb, 9, 0), cfl);
     else cfl[0] = red[RED_DT + 0], cfl[1] = red[RED_DT + 1], cfl[2] = red[RED_DT + 2];
     if (threadIdx.x != 0) return;
     if (step) {
@@ -594,6 +614,7 @@ __device__ __forceinline__ void dt_case(const Geom &g, const Fields &f, int step
 
 static __global__ void __launch_bounds__(64) k_dt(Geom g, Fields f, int step, int strang)
 {
+    touch_args<sizeof(Geom) + sizeof(Fields)>();
     dt_case(g, f, step, strang);
 }
 

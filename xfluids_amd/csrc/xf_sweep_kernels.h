@@ -603,8 +603,8 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
     __shared__ float sUf[MIX ? E * NC : 1];   // FP32 copies: mixed form only
     __shared__ float sFf[MIX ? E * NC : 1];
     __shared__ double sP[NC], sR1[NC];
-    // block-uniform: the words tested are not written by this launch
-    if (step_halted(f.err, ~EBIT_NAN)) return;
+    // tested once the first loads are on their way
+    const StepState step(f.err);
 
     const long long N = g.N;
     const int tid = threadIdx.x;
@@ -636,6 +636,11 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
         }
     };
 
+    const int nsb = state_blocks(g);
+    const bool own_fold = nsb <= FOLD_BLOCKS;
+    PassPart part;
+    if (own_fold) part = pass_load(f.spart, nsb, 3 * DIR, 0);
+
     // ---- stage U and the physical flux F of TS+5 cells per pencil ----------
     // A lane stages at most NIT cells; every cell's loads are issued before
     // any of them is used, so the second cell's loads overlap the first's
@@ -666,9 +671,11 @@ __device__ __forceinline__ void sweep_tile(const Geom &g, const DevThermo *__res
             }
         }
     }
+    // block-uniform: the words tested are not written by this launch
+    if (step.halted(~EBIT_NAN)) return;
     // the direction's GLF maxima of the pass, folded while the cells arrive
     double pass[3];
-    if (state_blocks(g) <= FOLD_BLOCKS) pass_maxima(f.spart, state_blocks(g), 3 * DIR, pass);
+    if (own_fold) pass_maxima(f.spart, nsb, 3 * DIR, part, pass);
     else
 #pragma unroll
         for (int k = 0; k < 3; k++) pass[k] = f.red[RED_GLFP + 3 * DIR + k];
@@ -1146,6 +1153,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SweepO
 k_sweep(Geom g, const DevThermo *__restrict__ th, const double *__restrict__ Ug, Fields f, double ncop_gamma, int mode,
         int stage, const double *Ua, const double *Ub, double *Uo, int span, int cols)
 {
+    touch_args<sizeof(Geom) + sizeof(Fields) + 64>();
     int tx, ty, tz;
     xcd_tile(tx, ty, tz);
     sweep_tile<NS, COP, DIR, SCHEME, PREC, SHAPE>(g, th, Ug, f, ncop_gamma, mode, stage, Ua, Ub, Uo, tx, ty, tz, span,

@@ -324,12 +324,14 @@ k_transport(Geom g, const DevThermo *__restrict__ th, const DevTransport *__rest
 {
     constexpr int E = NS + 4;
     constexpr int NCOP = NS - 1;
-    if (step_halted(f.err, ~0)) return; // block-uniform (no bit is set here)
+    touch_args<sizeof(Geom) + sizeof(Fields) + 40>();
+    const StepState step(f.err); // tested once the first loads are on their way
     const long long N = g.N;
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = id < N;
     // T and p, loaded ahead of the block's reduction barrier
     const double T = live ? f.T[id] : 0.0, p = live ? f.p[id] : 0.0;
+    if (step.halted(~0)) return; // block-uniform (no bit is set here)
     // mass fractions (Getrhoyi), velocities (GetStates) and mole fractions
     // (get_xi); the mass fractions feed the min / max and are then dropped
     double X[NS], C_total = 0.0, rho = 1.0, rho1 = 1.0;
