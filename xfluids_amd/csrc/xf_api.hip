@@ -538,7 +538,31 @@ static int build_mech(DevMech &m, int NS, int NR, const int *Nu_f, const int *Nu
             if (m.third[r * NS + j] != 0.0) x.mt |= 1u << j;
             if (nf != 0) x.mf |= 1u << j, x.pf |= (unsigned long long)nf << (4 * j);
             if (nb != 0) x.mb |= 1u << j, x.pb |= (unsigned long long)nb << (4 * j);
+            m.wacc[j * (MAXNR / 4) + r / 4] |= (unsigned)(nf | nb << 4) << (8 * (r % 4));
         }
+    }
+    m.wave_ok = NS < 15;
+    for (int r = 0; r < NR; r++) {
+        const DevRxn &x = m.rx[r];
+        DevWaveRxn &w = m.wr[r];
+        w.A = x.A, w.B = x.B, w.EaR = x.EaR, w.third = x.third_ind;
+        const double aE = std::fabs(x.EaR);
+        if (!(x.EaR == 0.0 || (aE >= 0x1p-500 && aE <= 0x1p500))) m.wave_ok = 0;
+        for (int j = 0; j < NS; j++) {
+            w.nu |= (unsigned long long)(m.Nu_d[r * NS + j] + 8) << (4 * j);
+            w.dn += m.Nu_d[r * NS + j];
+        }
+        auto factors = [&](const int *nu, unsigned &out) {
+            int k = 0;
+            for (int j = 0; j < NS; j++) {
+                if (nu[j] == 0) continue;
+                if (nu[j] > 2 || k == 3) m.wave_ok = 0;
+                else out |= (unsigned)(j | (nu[j] == 2 ? 16 : 0)) << (5 * k++);
+            }
+            for (; k < 3; k++) out |= 15u << (5 * k);
+        };
+        factors(m.Nu_f + r * NS, w.ff);
+        factors(m.Nu_b + r * NS, w.fb);
     }
     return XF_OK;
 }

@@ -1013,6 +1013,12 @@ __global__ void __launch_bounds__(64) k_chem_coop_multi(const ChemCase *__restri
 // the error norm) runs as an ordered chain over the lanes' values, so each
 // value is rounded exactly as in ChemLane / evalcv_dev and the results are the
 // per-cell driver's bits.  Requires NS + 1 <= 64 and NR <= 64.
+//
+// Bound by the latency of a pass's chains.  With the reactions' loops as branches on
+// their records, a table walk at the start of every cell and 239 registers a lane, 8192
+// cells (one pass each but for a few) took 98 us; as straight-line steps over packed
+// records, with the lane's tables in LDS, 57, and 2000 cells (as long as the stiffest
+// cell's passes) 37 instead of 56.
 // ---------------------------------------------------------------------------
 
 // Cross-lane exchanges of the cell's wave go through LDS: the lanes that own
@@ -1020,13 +1026,19 @@ __global__ void __launch_bounds__(64) k_chem_coop_multi(const ChemCase *__restri
 // every lane reads them back at the same addresses (LDS broadcasts).  Sums are
 // then formed on every lane in the reference's order.
 template <int NS> struct WaveShared {
-    double K[2 * MAXNR];    // Kf, Kck of each reaction
-    double S[2 * MAXNS];    // Gibbs energy and concentration of each species
-    double V[4 * 64];       // per-lane operands of the ordered sums
-    // species lane ln's nu_f | nu_b << 4 in reaction r at nu[64 * r + ln]
-    // (filled once per cell; each lane reads only its own entries)
-    unsigned char nu[64 * MAXNR];
+    double K[2 * MAXNR]; // Kf, Kck of each reaction, side by side; 0 beyond the last
+    double S[2 * MAXNS]; // log p less the Gibbs energy (general path: the energy) and concentration of each species
+    double V[4 * 64];    // per-lane operands of the ordered sums
+    double hc[FITC - 1][16];  // species n's fit coefficients of the current range at [.][1 + n]
+    double eff[NS][MAXNR];    // reaction r's third-body efficiencies
 };
+
+// lane k's value on every lane
+__device__ __forceinline__ double wave_lane(double v, int k)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), k),
+                            __builtin_amdgcn_readlane(__double2loint(v), k));
+}
 
 // ((init + v[lo]) + v[lo+1]) + ... of a lane-indexed LDS array with stride st
 __device__ __forceinline__ double lds_sum(const double *v, int st, int lo, int hi, double init)
@@ -1043,109 +1055,213 @@ __device__ __forceinline__ double lds_sub(const double *v, int st, int lo, int h
     return s;
 }
 
+// a lane's column of coefficients in LDS
+struct FitCol {
+    const double *c;
+    __device__ __forceinline__ double operator[](int m) const { return c[16 * m]; }
+};
+
 // What a lane reads on every pass, loaded once per cell: species lane 1 + n
-// keeps W, 1/W and R of species n and the fit coefficients of the current
-// range (reloaded when T crosses into another range); reaction lane r keeps
-// its record and third-body efficiencies.
+// keeps W, 1/W and R of species n and its orders in the reactions, and in LDS the fit
+// coefficients of the current range (reloaded when T crosses into another range);
+// reaction lane r keeps its record, and its third-body efficiencies in LDS.
 template <int NS> struct WaveLane {
     double Wi = 0.0, iWi = 0.0, Ri = 0.0;
-    int rc = -2; // range the coefficients hc belong to
-    double hc[9];
-    DevRxn R{};
-    double eff[NS];
+    int rc = -1; // range the coefficients hc belong to
+    double *hc; // the lane's coefficients: m at hc[16 * m] (FitCol)
+    DevWaveRxn R{};
+    unsigned acc[MAXNR / 4];
+    bool fast; // the tables qualify for the straight-line path
 
-    __device__ __forceinline__ void load(const DevThermo *__restrict__ th, const DevMech *__restrict__ mc, int NR)
+    __device__ __forceinline__ void load(const DevThermo *__restrict__ th, const DevMech *__restrict__ mc,
+                                         WaveShared<NS> &sh, int NR, double m_p)
     {
         const int ln = threadIdx.x & 63;
+        const bool sp = ln >= 1 && ln <= NS;
+        hc = &sh.hc[0][ln & 15];
+        if (ln < 16) {
 #pragma unroll
-        for (int m = 0; m < 9; m++) hc[m] = 0.0;
-        if (ln >= 1 && ln <= NS) Wi = th->Wi[ln - 1], iWi = th->_Wi[ln - 1], Ri = th->Ri[ln - 1];
-#pragma unroll
-        for (int it = 0; it < NS; it++) eff[it] = 0.0;
-        if (ln < NR) {
-            R = mc->rx[ln];
-#pragma unroll
-            for (int it = 0; it < NS; it++) eff[it] = mc->third[ln * NS + it];
+            for (int m = 0; m < FITC - 1; m++) hc[16 * m] = 0.0;
         }
+        if (sp) Wi = th->Wi[ln - 1], iWi = th->_Wi[ln - 1], Ri = th->Ri[ln - 1];
+#pragma unroll
+        for (int w = 0; w < MAXNR / 4; w++) acc[w] = sp ? mc->wacc[(ln - 1) * (MAXNR / 4) + w] : 0u;
+        // an idle lane's record: every order 0, no factors
+        R.nu = 0x8888888888888888ull, R.ff = R.fb = 15u | 15u << 5 | 15u << 10;
+        if (ln < NR) {
+            R = mc->wr[ln];
+#pragma unroll
+            for (int it = 0; it < NS; it++) sh.eff[it][ln] = mc->third[ln * NS + it];
+        }
+        fast = th->fast && mc->wave_ok && m_p >= 0x1p-300 && m_p <= 0x1p300;
     }
     // the fit coefficients of range r (the same on every lane: T is the cell's)
     __device__ __forceinline__ void range(const DevThermo *__restrict__ th, int r)
     {
+        r = r < 0 ? 0 : r;
         if (r != rc) {
             const int ln = threadIdx.x & 63;
             if (ln >= 1 && ln <= NS) {
-                const double *c = fit_coeffs(th, r, ln - 1);
+                const double *c = th->Hf + (r * MAXNS + ln - 1) * FITC;
 #pragma unroll
-                for (int m = 0; m < 9; m++) hc[m] = c[m];
+                for (int m = 0; m < FITC - 1; m++) hc[16 * m] = c[m];
             }
             rc = r;
         }
     }
 };
 
-// evalcv (ProductionRates.h:459-479) at the distributed state: yv is
-// component ln, m_tmp = T; returns the component's q and d
+// the lane's Kf and Kck and the species lane's sums over the reactions, for T where
+// the fast fits and quotients are exact; false, with nothing of use, when a value is
+// not finite.  Every lane runs every step: terms of a zero order add a zero, factors
+// that a reaction lacks are 1.  No branch and no table read is
+// left between the barriers, the two logarithms run on different lanes, and the two
+// exponentials together.
 template <int NS, int THERMO>
-__device__ __forceinline__ void evalcv_wave(const DevThermo *__restrict__ th, const DevMech *__restrict__ mc,
-                                            WaveLane<NS> &W, WaveShared<NS> &sh, int NR, double yv, double m_tmp,
-                                            double &qv, double &dv, double m_dens, double m_p, double _dens,
-                                            double logP)
+__device__ __forceinline__ bool wave_rates(const DevThermo *__restrict__ th, WaveLane<NS> &W, WaveShared<NS> &sh,
+                                           int NR, double yv, double T, double m_dens, double m_p, double logP,
+                                           double &h1, double &ycp, double &qi, double &pi)
+{
+    const double inf = __longlong_as_double(0x7ff0000000000000LL);
+    const int ln = threadIdx.x & 63;
+    const bool sp = ln >= 1 && ln <= NS;
+    const double iT = ddiv_core(1.0, T);
+    const double lx = dlog_pos(ln < 32 ? T : ddiv_core(m_p, R0 * T));
+    const double lT = wave_lane(lx, 0), logStandConc = wave_lane(lx, 32);
+    W.range(th, THERMO ? (T >= 6000.0 ? 2 : (T >= 1000.0 ? 1 : 0)) : (T > 1000.0 ? 0 : 1));
+    const FitCol hc{W.hc};
+    h1 = h_fast<THERMO != 0>(hc, T, iT, lT, 1.0);
+    double g = 0.0;
+    g += s_fast<THERMO != 0>(hc, T, iT, lT);
+    g += dquot(-h1, T, iT);
+    const double lg = logP - g, conc = yv * W.iWi * m_dens * 1.0E-3;
+    if (sp) sh.S[ln - 1] = lg, sh.S[MAXNS + ln - 1] = conc;
+    if (ln == 0) sh.S[MAXNS + 15] = 1.0;
+    ycp = yv * cp_fast<THERMO != 0>(hc, T, iT, W.Ri);
+    __syncthreads();
+    // the packed orders as values of their own on every pass: the compiler would keep
+    // each, unpacked, in registers for the whole cell
+    auto packed = [](unsigned v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    const unsigned nu[2] = {packed((unsigned)W.R.nu), packed((unsigned)(W.R.nu >> 32))};
+    double DG = 0.0;
+#pragma unroll
+    for (int n = 0; n < NS; n++) DG += ((int)((nu[n / 8] >> (4 * (n % 8))) & 15u) - 8) * sh.S[n];
+    double arg[2] = {W.R.B * lT - dquot(W.R.EaR, T, iT), DG - W.R.dn * logStandConc}, e[2];
+    dexp_n<2>(arg, e);
+    double Kf = W.R.A * e[0], Kck = dmin(e[1], 1.0E+40);
+    double tb = 0.0;
+#pragma unroll
+    for (int n = 0; n < NS; n++) tb += sh.eff[n][ln < MAXNR ? ln : 0] * sh.S[MAXNS + n];
+    Kf *= W.R.third ? tb : 1.0;
+    Kck *= Kf;
+    const unsigned ff = packed(W.R.ff), fb = packed(W.R.fb);
+    auto factor = [&](unsigned f) {
+        const double x = sh.S[MAXNS + (f & 15u)];
+        return f & 16u ? x * x : x;
+    };
+#pragma unroll
+    for (int k = 0; k < 3; k++) Kf *= factor(ff >> (5 * k));
+#pragma unroll
+    for (int k = 0; k < 3; k++) Kck *= factor(fb >> (5 * k));
+    if (!__all((ln >= NR || (fabs(Kf) < inf && fabs(Kck) < inf)) && (!sp || (fabs(lg) < inf && fabs(conc) < inf))))
+        return false;
+    if (ln < MAXNR) sh.K[2 * ln] = ln < NR ? Kf : 0.0, sh.K[2 * ln + 1] = ln < NR ? Kck : 0.0;
+    __syncthreads();
+    qi = 0.0, pi = 0.0;
+#pragma unroll
+    for (int w = 0; w < MAXNR; w += 8) {
+        if (w >= NR) break;
+        const unsigned a[2] = {packed(W.acc[w / 4]), packed(W.acc[w / 4 + 1])};
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+            const unsigned b = a[r / 4] >> (8 * (r % 4));
+            const int nf = (int)(b & 15u), nb = (int)((b >> 4) & 15u);
+            const double kf = sh.K[2 * (w + r)], kc = sh.K[2 * (w + r) + 1];
+            qi += nb * kf + nf * kc;
+            pi += nf * kf + nb * kc;
+        }
+    }
+    return true;
+}
+
+// the same for every T and value, with the tests of rxn_rates on the record
+template <int NS, int THERMO>
+__device__ __forceinline__ void wave_rates_general(const DevThermo *__restrict__ th, const DevMech *__restrict__ mc,
+                                                   WaveLane<NS> &W, WaveShared<NS> &sh, int NR, double yv, double T,
+                                                   double m_dens, double m_p, double logP, double &h1, double &ycp,
+                                                   double &qi, double &pi)
 {
     const int ln = threadIdx.x & 63;
-    const int n = ln - 1;
     const bool sp = ln >= 1 && ln <= NS;
-    // THERMO: the fit family (1 NASA-9, 0 JANAF) as a constant, so that each
-    // formula reads the coefficients at fixed positions (kept in registers)
-    constexpr int thermo = THERMO;
-    const TPre t = tpre<true>(m_tmp, thermo);
+    const TPre t = tpre<true>(T, THERMO);
     W.range(th, t.r);
-    double h1 = 0.0;
+    h1 = 0.0, ycp = 0.0;
     if (sp) {
-        // h_k and s_k with Ri = 1
-        h1 = h_fit(W.hc, thermo, t, 1.0);
-        if (t.TT < 200.0) h1 += cp200_k(th, 1.0, n) * (t.TT - 200.0);
-        double temp = 0.0;
-        temp += s_fit(W.hc, thermo, t, 1.0);
-        temp += (-h1 / m_tmp);
-        sh.S[n] = temp;
-        sh.S[MAXNS + n] = yv * W.iWi * m_dens * 1.0E-3;
-    }
-    const double logStandConc = dlog(m_p / (R0 * m_tmp));
-    // log T: the fit's log max(T, 200) when T >= 200 (the same call on the same value)
-    const double logT = m_tmp >= 200.0 ? t.lT : dlog(m_tmp);
-    __syncthreads();
-    double Kf = 0.0, Kck = 0.0;
-    if (ln < NR) {
-        double gka[NS], mca[NS];
+        double hc[9];
 #pragma unroll
-        for (int k = 0; k < NS; k++) gka[k] = sh.S[k], mca[k] = sh.S[MAXNS + k];
+        for (int m = 0; m < 9; m++) hc[m] = W.hc[16 * m];
+        // h_k and s_k with Ri = 1
+        h1 = h_fit(hc, THERMO, t, 1.0);
+        if (t.TT < 200.0) h1 += cp200_k(th, 1.0, ln - 1) * (t.TT - 200.0);
+        double temp = 0.0;
+        temp += s_fit(hc, THERMO, t, 1.0);
+        temp += (-h1 / T);
+        sh.S[ln - 1] = temp;
+        sh.S[MAXNS + ln - 1] = yv * W.iWi * m_dens * 1.0E-3;
+        ycp = yv * cp_fit(hc, THERMO, t, W.Ri);
+    }
+    const double logStandConc = dlog(m_p / (R0 * T));
+    // log T: the fit's log max(T, 200) when T >= 200 (the same call on the same value)
+    const double logT = T >= 200.0 ? t.lT : dlog(T);
+    __syncthreads();
+    if (ln < NR) {
         RxnCtx c;
-        c.m_tmp = m_tmp, c.logT = logT, c.logP = logP, c.logStandConc = logStandConc;
-        c.rT = m_tmp >= 200.0 ? t.iT : 1.0 / m_tmp; // the fit's 1 / max(T, 200) when T >= 200
-        c.t_ok = m_tmp >= 0x1p-500 && m_tmp <= 0x1p500;
-        rxn_rates<NS>(W.R, [&W](int it) { return W.eff[it]; }, c, gka, mca, Kf, Kck);
-        sh.K[ln] = Kf, sh.K[MAXNR + ln] = Kck;
+        c.m_tmp = T, c.logT = logT, c.logP = logP, c.logStandConc = logStandConc;
+        c.rT = T >= 200.0 ? t.iT : 1.0 / T; // the fit's 1 / max(T, 200) when T >= 200
+        c.t_ok = T >= 0x1p-500 && T <= 0x1p500;
+        double Kf, Kck;
+        rxn_rates<NS>(mc->rx[ln], [mc, ln](int it) { return mc->third[ln * NS + it]; }, c, sh.S, sh.S + MAXNS, Kf, Kck);
+        sh.K[2 * ln] = Kf, sh.K[2 * ln + 1] = Kck;
     }
     __syncthreads();
-    // species n's sums over the reactions, in increasing order (rxn_accum)
-    double qi = 0.0, pi = 0.0;
+    qi = 0.0, pi = 0.0;
     if (sp) {
         // a reaction adds to species n exactly when its nu_f or nu_b is non-zero
         for (int r = 0; r < NR; r++) {
-            const unsigned b = sh.nu[64 * r + ln];
+            const unsigned b = (mc->wacc[(ln - 1) * (MAXNR / 4) + r / 4] >> (8 * (r % 4))) & 255u;
             if (b) {
                 const int nf = (int)(b & 15u), nb = (int)(b >> 4);
-                const double kf = sh.K[r], kc = sh.K[MAXNR + r];
+                const double kf = sh.K[2 * r], kc = sh.K[2 * r + 1];
                 qi += nb * kf + nf * kc;
                 pi += nf * kf + nb * kc;
             }
         }
+    }
+}
+
+// evalcv (ProductionRates.h:459-479) at the distributed state: yv is
+// component ln, T the cell's; returns the component's q and d
+template <int NS, int THERMO>
+__device__ __forceinline__ void evalcv_wave(const DevThermo *__restrict__ th, const DevMech *__restrict__ mc,
+                                            WaveLane<NS> &W, WaveShared<NS> &sh, int NR, double yv, double T,
+                                            double &qv, double &dv, double m_dens, double m_p, double _dens,
+                                            double logP)
+{
+    const int ln = threadIdx.x & 63;
+    double h1, ycp, qi, pi;
+    if (!(W.fast && T >= 200.0 && T <= 1.0e5 &&
+          wave_rates<NS, THERMO>(th, W, sh, NR, yv, T, m_dens, m_p, logP, h1, ycp, qi, pi)))
+        wave_rates_general<NS, THERMO>(th, mc, W, sh, NR, yv, T, m_dens, m_p, logP, h1, ycp, qi, pi);
+    if (ln >= 1 && ln <= NS) {
         qi *= W.Wi * _dens;
         pi *= W.Wi * _dens;
-        const double ei = (h1 - m_tmp) * W.Ri;
+        const double ei = (h1 - T) * W.Ri;
         sh.V[4 * ln + 0] = qi * ei;
         sh.V[4 * ln + 1] = pi * ei;
-        sh.V[4 * ln + 2] = yv * cp_fit(W.hc, thermo, t, W.Ri);
+        sh.V[4 * ln + 2] = ycp;
         sh.V[4 * ln + 3] = yv * W.iWi;
     }
     __syncthreads();
@@ -1163,28 +1279,23 @@ __device__ __forceinline__ void evalcv_wave(const DevThermo *__restrict__ th, co
 
 // get_Cope at the distributed state (mix_e's order)
 template <int NS, int THERMO>
-__device__ __forceinline__ double mix_e_wave(const DevThermo *__restrict__ th, WaveShared<NS> &sh, double yv, double T)
+__device__ __forceinline__ double mix_e_wave(const DevThermo *__restrict__ th, WaveLane<NS> &W, WaveShared<NS> &sh,
+                                             double yv, double T)
 {
     const int ln = threadIdx.x & 63;
-    if (ln >= 1 && ln <= NS) {
+    double h;
+    if (W.fast && T >= 200.0 && T <= 1.0e5) {
+        W.range(th, THERMO ? (T >= 6000.0 ? 2 : (T >= 1000.0 ? 1 : 0)) : (T > 1000.0 ? 0 : 1));
+        h = h_fast<THERMO != 0>(FitCol{W.hc}, T, ddiv_core(1.0, T), THERMO ? dlog_pos(T) : 0.0, 1.0);
+    } else {
         const TPre t = THERMO ? tpre<true>(T, 1) : tpre<false>(T, 0);
-        const double ei = (h_k(th, t, 1.0, ln - 1) - T) * th->Ri[ln - 1];
-        sh.V[ln] = ei * yv;
+        h = ln >= 1 && ln <= NS ? h_k(th, t, 1.0, ln - 1) : 0.0;
     }
+    if (ln >= 1 && ln <= NS) sh.V[ln] = (h - T) * W.Ri * yv;
     __syncthreads();
     const double e = lds_sum(sh.V, 1, 1, NS + 1, 0.0);
     __syncthreads();
     return e;
-}
-
-// T, held by lane 0, to every lane
-template <int NS> __device__ __forceinline__ double wave_T(WaveShared<NS> &sh, double yv)
-{
-    if ((threadIdx.x & 63) == 0) sh.V[0] = yv;
-    __syncthreads();
-    const double T = sh.V[0];
-    __syncthreads();
-    return T;
 }
 
 // ChemeODEQ2SolverKernel1 + Chemeq2 for interior cell tl of case cc on one
@@ -1219,17 +1330,9 @@ __device__ __forceinline__ void chem_wave_cell(const DevThermo *__restrict__ th,
         __syncthreads();
         if (ln == NS) yv = rem;
     }
-    const double e0 = mix_e_wave<NS, THERMO>(th, sh, yv, wave_T<NS>(sh, yv));
     WaveLane<NS> W;
-    W.load(th, mc, NR);
-    for (int r = 0; r < NR; r++) {
-        unsigned v = 0;
-        if (ln >= 1 && ln <= NS) {
-            const unsigned long long pf = mc->rx[r].pf, pb = mc->rx[r].pb;
-            v = (unsigned)((pf >> (4 * (ln - 1))) & 15ull) | ((unsigned)((pb >> (4 * (ln - 1))) & 15ull) << 4);
-        }
-        sh.nu[64 * r + ln] = (unsigned char)v;
-    }
+    W.load(th, mc, sh, NR, m_p);
+    const double e0 = mix_e_wave<NS, THERMO>(th, W, sh, yv, wave_lane(yv, 0));
     // Chemeq2 (ProductionRates.h:488-638), the steps of ChemLane
     const double ymin = 1.0e-20, tfd = 1.0 + 1.0e-10, epscl = 1.0e4;
     const double dtg = cc.dt[DT_CHEM];
@@ -1260,7 +1363,7 @@ __device__ __forceinline__ void chem_wave_cell(const DevThermo *__restrict__ th,
             }
             tn = ts + dt;
         }
-        evalcv_wave<NS, THERMO>(th, mc, W, sh, NR, yv, wave_T<NS>(sh, yv), qv, dv, rho, m_p, _dens, logP);
+        evalcv_wave<NS, THERMO>(th, mc, W, sh, NR, yv, wave_lane(yv, 0), qv, dv, rho, m_p, _dens, logP);
         if (!started) {
             const double epsmin = 1.0e-4, sqreps = 0.05;
             if (comp) {
@@ -1330,8 +1433,7 @@ __device__ __forceinline__ void chem_wave_cell(const DevThermo *__restrict__ th,
         ys = yv, qs = qv, ds = dv;
     }
     // write-back (ChemeODEQ2SolverKernel1's tail), the pass count, the checks
-    const double T1 = wave_T<NS>(sh, yv);
-    const double e1 = mix_e_wave<NS, THERMO>(th, sh, yv, T1);
+    const double e1 = mix_e_wave<NS, THERMO>(th, W, sh, yv, wave_lane(yv, 0));
     bool bad = false;
     if (ln >= 1 && ln < NS) {
         const double v = yv * rho;
@@ -1358,10 +1460,12 @@ __device__ __forceinline__ void chem_wave_cell(const DevThermo *__restrict__ th,
     }
 }
 
-// one interior cell per one-wave block; THERMO = the context's fit family
+// one interior cell per one-wave block; THERMO = the context's fit family.  Three
+// waves per SIMD: at 8192 cells and nine species 57 us, two waves 60, four (which
+// spill 192 bytes a lane) 67.
 template <int NS, int THERMO>
-__global__ void __launch_bounds__(64) k_chem_wave(Geom g, const DevThermo *__restrict__ th,
-                                                  const DevMech *__restrict__ mc, Fields f, int record, int check)
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+k_chem_wave(Geom g, const DevThermo *__restrict__ th, const DevMech *__restrict__ mc, Fields f, int record, int check)
 {
     const long long tl = blockIdx.x;
     if (tl >= (long long)g.X_inner * g.Y_inner * g.Z_inner) return;

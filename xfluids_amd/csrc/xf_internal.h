@@ -44,6 +44,16 @@ struct DevRxn {
     int third_ind, pad;
 };
 
+// What one lane of k_chem_wave reads of its reaction: the net orders nu + 8 in 4 bits
+// per species and their sum dn, and up to three factors of each direction's rate
+// (5 bits each: species, 16 for its square; species 15 stands for a factor of 1)
+struct DevWaveRxn {
+    double A, B, EaR, dn;
+    unsigned long long nu;
+    unsigned ff, fb;
+    int third, pad;
+};
+
 // Reaction tables (reference layout, src/include/global_setup.h:210-215)
 // plus the per-reaction records built from them
 struct DevMech {
@@ -53,6 +63,9 @@ struct DevMech {
     int third_ind[MAXNR];
     int NR;
     DevRxn rx[MAXNR];
+    DevWaveRxn wr[MAXNR];
+    unsigned wacc[MAXNS * (MAXNR / 4)]; // species n: nu_f | nu_b << 4 of each reaction, a byte each
+    int wave_ok; // every reaction fits its DevWaveRxn, and EaR is 0 or within [2^-500, 2^500]
 };
 
 // Geometry passed by value to every kernel

@@ -148,21 +148,21 @@ __device__ __forceinline__ bool table_fast(const DevThermo *__restrict__ th)
 // Newton iteration at nine species is one basic block instead of some thirty,
 // and k_states<9> at 8192 cells (a launch as long as its longest Newton chain)
 // went from 44.7 to 24.5 us, on a 128^3 mixing layer from 223 to 181 us.
-template <bool NASA> __device__ __forceinline__ double cp_fast(cdouble *c, double T, double iT, double Ri)
+template <bool NASA, class P> __device__ __forceinline__ double cp_fast(P c, double T, double iT, double Ri)
 {
     if (NASA) return Ri * ((c[0] * iT + c[1]) * iT + c[2] + (c[3] + (c[4] + (c[5] + c[6] * T) * T) * T) * T);
     return Ri * (c[0] + (c[1] + (c[2] + (c[3] + c[4] * T) * T) * T) * T);
 }
-template <bool NASA>
-__device__ __forceinline__ double h_fast(cdouble *c, double T, double iT, double lT, double Ri)
+template <bool NASA, class P>
+__device__ __forceinline__ double h_fast(P c, double T, double iT, double lT, double Ri)
 {
     if (NASA)
         return Ri * (dquot(-c[0], T, iT) + c[1] * lT + (c[2] + (c[9] + (c[10] + (c[11] + c[12] * T) * T) * T) * T) * T +
                      c[7]);
     return Ri * (T * (c[0] + T * (c[9] + T * (c[10] + T * (c[11] + c[4] * T * 0.2)))) + c[5]);
 }
-template <bool NASA>
-__device__ __forceinline__ double s_fast(cdouble *c, double T, double iT, double lT)
+template <bool NASA, class P>
+__device__ __forceinline__ double s_fast(P c, double T, double iT, double lT)
 {
     if (NASA)
         return ((c[13] * iT - c[1]) * iT + c[2] * lT + (c[3] + (c[14] + (c[15] + c[16] * T) * T) * T) * T + c[8]);
