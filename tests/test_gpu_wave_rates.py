@@ -1,7 +1,8 @@
-"""The wave driver's straight-line rates and what they leave to the general path, bit
-for bit: temperatures around the fit ranges and below 200 K against the oracle, and
-mechanisms whose reactions do and do not fit the packed records against one lane per
-cell."""
+"""The chemistry drivers' straight-line paths and what they leave to the general ones,
+bit for bit: temperatures around the fit ranges and below 200 K against the oracle, and
+the wave driver against one lane per cell for mechanisms whose reactions do and do not
+fit the packed records, and for negative rates (which one lane per cell divides as
+IEEE, like the wave driver)."""
 import numpy as np
 import pytest
 
@@ -47,9 +48,9 @@ def test_ranges_match_oracle(thermo, lo, hi):
 # orders written over reaction r's, the same on both sides so that it is in balance:
 # squares of two species, a cube, four species, none
 @pytest.mark.parametrize("nu", [{0: 2, 3: 2}, {1: 3}, {0: 1, 1: 1, 2: 1, 4: 1}, {}])
-@pytest.mark.parametrize("r", [0, -1])
-def test_mechanisms_match_per_cell(nu, r):
-    announce("wave rates mechanism %s %d" % (nu, r))
+@pytest.mark.parametrize("r,sign", [(0, 1.0), (-1, 1.0), (0, -1.0)])
+def test_mechanisms_match_per_cell(nu, r, sign):
+    announce("wave rates mechanism %s %d %g" % (nu, r, sign))
     s, U, T = case(1, 900.0, 1300.0)
     d = s.desc
     Nu_f, Nu_b, third, Rargus = s.mechanism()
@@ -59,6 +60,7 @@ def test_mechanisms_match_per_cell(nu, r):
         for n, v in nu.items():
             row[n] = v
     Rargus.reshape(d.NR, 6)[r, 2] = 0.0
+    Rargus.reshape(d.NR, 6)[r, 0] *= sign
     i32 = lambda a: a.ctypes.data_as(xf.C.POINTER(xf.C.c_int))
     f64 = lambda a: a.ctypes.data_as(xf.C.POINTER(xf.C.c_double))
     out = []

@@ -136,8 +136,8 @@ __device__ __forceinline__ void rxn_step(const DevRxn R, Eff eff, const RxnCtx &
 // cell, ~4250 instructions per pass and cell before, 97 KB of code against the 64
 // KB instruction cache): the fast path below drops what a compiled mechanism and
 // an ordinary state make exact no-ops, and needs no scratch memory.  k_chem at
-// 128^3 went from 1417 to 1219 us, k_chem_queue on a 256^2 channel from 149 to
-// 130 us.
+// 128^3 went from 1417 to 997 us, k_chem_queue on a 256^2 channel from 149 to
+// 106 us.
 //
 // Reaction r of compiled mechanism K on the fast path of evalcv_dev: rxn_step's
 // values with every test on the record resolved at compile time.  lg = log p - g
@@ -411,6 +411,35 @@ __device__ __forceinline__ double alpha_of(double r)
     return (180.0 + r * (60.0 + r * (11.0 + r))) / (360.0 + r * (60.0 + r * (12.0 + r)));
 }
 
+// The predictor and corrector divide seven times per component, which as IEEE
+// divisions were 770 of a pass's 3460 vector instructions, chained through the carry
+// register, with a branch per component around the error norm.  For the species they
+// take the unscaled sequence, all components in one block.  Its quotient is the
+// IEEE-rounded one while divisor and dividend stay clear of the ends of the range:
+// the divisors are at least ymin, 1 or 1e-30 where the ratios r and the rates are not
+// negative, and in_range bounds all of them.  A dividend so small that the remainder
+// underflows leaves a quotient below 2^-890, whose last bits reach nothing: it is only
+// ever added to ymin or more, or competes with eps >= 1e-10.  The temperature's rates
+// may have either sign, and it keeps the IEEE division.  k_chem at 128^3 and one pass
+// per cell went from 997 to 947 us, k_chem_queue on a 256^2 channel from 106 to 102.
+//
+// a non-negative number up to 2^160: its upper word is at most this one
+constexpr unsigned CHEM_IN_RANGE = (1023u + 160u) << 20;
+__device__ __forceinline__ void in_range(unsigned &top, double a)
+{
+    const unsigned h = (unsigned)__double2hiint(a); // negative, infinite and NaN: larger
+    top = h > top ? h : top;
+}
+// a / b: FAST by ddiv_core
+template <bool FAST> __device__ __forceinline__ double chem_div(double a, double b)
+{
+    return FAST ? ddiv_core(a, b) : a / b;
+}
+template <bool FAST> __device__ __forceinline__ double chem_alpha(double r)
+{
+    return chem_div<FAST>(180.0 + r * (60.0 + r * (11.0 + r)), 360.0 + r * (60.0 + r * (12.0 + r)));
+}
+
 // Chemeq2 state of one cell, advanced one rate evaluation at a time so that
 // a lane can also work through a queue of cells (k_chem_queue).  Every
 // advance is: before() -> evalcv_dev(y) -> after().  The first advance of a
@@ -469,23 +498,60 @@ template <int NS, class St = ChemRegs<NS + 1>, int SPEC = -1> struct ChemLane {
             return 0;
         }
         if (++passes > CHEM_MAXSUB) return -1;
-        // predictor
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const double rt = dt * ds(i) / ys(i);
-            rtau(i) = rt;
-            const double alpha = alpha_of(rt);
-            const double scr = dt * (qs(i) - ds(i)) / (1.0 + alpha * rt);
-            y[i] = dmax(ys(i) + scr, ymin);
-        }
+        unsigned top = 0;
+        predict<false>(0, 1, top);
+        predict<true>(1, NL, top);
+        if (__any(top > CHEM_IN_RANGE)) predict<false>(1, NL, top);
         tn = ts + dt;
         return 0;
+    }
+
+    // components lo .. hi - 1; FAST: top collects the words that in_range bounds
+    template <bool FAST> __device__ __forceinline__ void predict(int lo, int hi, unsigned &top)
+    {
+        const double ymin = 1.0e-20;
+#pragma unroll
+        for (int i = lo; i < hi; i++) {
+            const double rt = chem_div<FAST>(dt * ds(i), ys(i));
+            rtau(i) = rt;
+            const double alpha = chem_alpha<FAST>(rt);
+            const double scr = chem_div<FAST>(dt * (qs(i) - ds(i)), 1.0 + alpha * rt);
+            if (FAST) in_range(top, rt), in_range(top, ys(i)), in_range(top, qs(i));
+            y[i] = dmax(ys(i) + scr, ymin);
+        }
+    }
+    // the corrector with the convergence test: the new values, and eps raised to the
+    // components' errors
+    template <bool FAST>
+    __device__ __forceinline__ void correct(int lo, int hi, double *yn, double &eps, unsigned &top)
+    {
+        const double ymin = 1.0e-20;
+#pragma unroll
+        for (int i = lo; i < hi; i++) {
+            const double yp = y[i];
+            const double rtaub = 0.5 * (rtau(i) + chem_div<FAST>(dt * d[i], yp));
+            const double alpha = chem_alpha<FAST>(rtaub);
+            const double ysi = ys(i);
+            const double qt = (1.0 - alpha) * qs(i) + alpha * q[i];
+            const double scr = chem_div<FAST>(qt * dt - rtaub * ysi, 1.0 + alpha * rtaub);
+            const double scr2 = dmax(ysi + scr, 0.0);
+            double scr1 = fabs(scr2 - yp);
+            yn[i] = dmax(scr2, ymin);
+            scr1 = chem_div<FAST>(scr1, yn[i]);
+            const double err =
+                0.5 * (scr1 + dmin(chem_div<FAST>(fabs(q[i] - d[i]), q[i] + d[i] + 1.0e-30), scr1));
+            eps = (0.25 * (ysi + yn[i])) > ymin ? dmax(err, eps) : eps;
+            if (FAST) {
+                in_range(top, yp), in_range(top, rtaub), in_range(top, yn[i]);
+                in_range(top, q[i]), in_range(top, d[i]);
+            }
+        }
     }
 
     // after the rate evaluation at y: 1 = reached dtg, 0 = continue
     __device__ __forceinline__ int after()
     {
-        const double ymin = 1.0e-20, tfd = 1.0 + 1.0e-10, epscl = 1.0e4;
+        const double tfd = 1.0 + 1.0e-10, epscl = 1.0e4;
         if (!started) {
             const double epsmin = 1.0e-4, sqreps = 0.05;
             double scrtch = 1e-25;
@@ -505,24 +571,17 @@ template <int NS, class St = ChemRegs<NS + 1>, int SPEC = -1> struct ChemLane {
             started = true;
             return 0;
         }
-        // corrector fused with the convergence test
-        double eps = 1e-10;
-#pragma unroll
-        for (int i = 0; i < NL; i++) {
-            const double yp = y[i];
-            const double rtaub = 0.5 * (rtau(i) + dt * d[i] / yp);
-            const double alpha = alpha_of(rtaub);
-            const double ysi = ys(i);
-            const double qt = (1.0 - alpha) * qs(i) + alpha * q[i];
-            const double scr = (qt * dt - rtaub * ysi) / (1.0 + alpha * rtaub);
-            const double scr2 = dmax(ysi + scr, 0.0);
-            double scr1 = fabs(scr2 - yp);
-            y[i] = dmax(scr2, ymin);
-            if ((0.25 * (ysi + y[i])) > ymin) {
-                scr1 = scr1 / y[i];
-                eps = dmax(0.5 * (scr1 + dmin(fabs(q[i] - d[i]) / (q[i] + d[i] + 1.0e-30), scr1)), eps);
-            }
+        double eps0 = 1e-10, yn[NL];
+        unsigned top = 0;
+        correct<false>(0, 1, yn, eps0, top);
+        double eps = eps0;
+        correct<true>(1, NL, yn, eps, top);
+        if (__any(top > CHEM_IN_RANGE)) {
+            eps = eps0;
+            correct<false>(1, NL, yn, eps, top);
         }
+#pragma unroll
+        for (int i = 0; i < NL; i++) y[i] = yn[i];
         eps = eps * epscl;
         if (eps < epsmax) {
             if (dtg <= (tn * tfd)) return 1;
