@@ -206,8 +206,12 @@ template <int NS, bool COP> struct Launch {
     static void states(xf_ctx *c, double *U, int full, int bcs, int where)
     {
         ProfScope ps(c, "states");
-        hipLaunchKernelGGL((k_states<NS, COP>), dim3(nblk(c->N)), dim3(256), 0, c->stream, c->g, c->d_th, U, c->f,
-                           c->d.ncop_gamma, full, bcs, where);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(nblk(c->N)), dim3(256), 0, c->stream, c->g, c->d_th, U, c->f,
+                               c->d.ncop_gamma, full, bcs, where);
+        };
+        if (COP && nblk(c->N) <= STATES_TAIL) launch(k_states<NS, COP, COP>);
+        else launch(k_states<NS, COP, false>);
         if constexpr (COP) {
             if (c->g.ghost)
                 hipLaunchKernelGGL((k_rhoyi_writeback<NS>), dim3(nblk(c->N)), dim3(256), 0, c->stream, c->g, U,
@@ -381,8 +385,12 @@ template <int NS, bool COP> struct Launch {
     static void states_multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,
                              int full, int fill, int where, int sel, bool fold)
     {
-        hipLaunchKernelGGL((k_states_multi<NS, COP>), dim3((unsigned)blocks), dim3(256), 0, st, cases, ncases, c0->d_th,
-                           c0->d.ncop_gamma, full, fill, where, sel);
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, st, cases, ncases, c0->d_th,
+                               c0->d.ncop_gamma, full, fill, where, sel);
+        };
+        if (COP && blocks <= STATES_TAIL) launch(k_states_multi<NS, COP, COP>);
+        else launch(k_states_multi<NS, COP, false>);
         if (fold) hipLaunchKernelGGL(k_states_fold_multi, dim3((unsigned)(12 * ncases)), dim3(1024), 0, st, cases);
     }
     static void sweep_multi(const xf_ctx *c0, hipStream_t st, const EnsCase *cases, int ncases, long long blocks,

@@ -233,6 +233,12 @@ static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__r
 // takes 1.3 us longer for it, which is where the line lies: a step 106.7 instead of
 // 107.5.
 constexpr int FOLD_BLOCKS = 512;
+// Up to this many blocks (four on each CU) a states launch is resident at once and
+// lasts as long as its longest Newton chain; above it the registers of newton_tail
+// cost a wave per SIMD and its shorter chains gain nothing (three species at 2096
+// blocks 31.8 us with it, 29.0 without; at 711 blocks and five species 45.5 instead
+// of 54.3, at 33 and nine 16.7 instead of 20.0).
+constexpr long long STATES_TAIL = 1024;
 __host__ __device__ inline int state_blocks(const Geom &g) { return (int)((g.N + 255) / 256); }
 
 // slots q, q + 1, q + 2, the same on every lane; run by whole waves.  The loads of
@@ -314,8 +320,9 @@ static __global__ void __launch_bounds__(1024) k_states_fold_multi(const EnsCase
 // bit 28, and every ghost cell first takes its value from its source cell as
 // k_boundary_all forms it (FluidBoundaryCondition, fused into UpdateStates:
 // the sources are interior cells or Inflow ghosts, which no thread writes)
-// the 256 cells of block bid of one case
-template <int NS, bool COP>
+// the 256 cells of block bid of one case; TAIL: the last chains of the Newton solves on
+// groups of lanes (newton_tail), for launches of at most STATES_TAIL blocks
+template <int NS, bool COP, bool TAIL>
 __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__restrict__ th, double *Ug,
                                              const Fields &f, double ncop_gamma, int full, int bcs, int where,
                                              long long bid)
@@ -392,7 +399,7 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
         double T = f.T[id], p, gamma;
         if (COP) {
             const double R_ = mix_R<NS>(th, yi);
-            T = get_T<NS>(th, yi, tme, T);
+            T = get_T<NS, TAIL>(th, yi, tme, T);
             p = rho * R_ * T;
             // species Cp and h at T
             double cpk[NS], hk[NS];
@@ -526,12 +533,12 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
     if (threadIdx.x == 0 && serr) report_pass(f.err, serr, where);
 }
 
-template <int NS, bool COP>
+template <int NS, bool COP, bool TAIL>
 __global__ void __launch_bounds__(256) k_states(Geom g, const DevThermo *__restrict__ th, double *Ug, Fields f,
                                                 double ncop_gamma, int full, int bcs, int where)
 {
     touch_args<sizeof(Geom) + sizeof(Fields) + 32>();
-    states_block<NS, COP>(g, th, Ug, f, ncop_gamma, full, bcs, where, (long long)blockIdx.x);
+    states_block<NS, COP, TAIL>(g, th, Ug, f, ncop_gamma, full, bcs, where, (long long)blockIdx.x);
 }
 
 // GhostSpecies write-back of Getrhoyi (Update_device.hpp:20-21) on every
@@ -552,7 +559,7 @@ __global__ void __launch_bounds__(256) k_rhoyi_writeback(Geom g, double *Ug, Fie
 
 // UpdateStates of every case of an ensemble in one launch (fill = 1: with
 // each case's ghost fill); sel picks the state (0 U, 1 U1, 2 U2)
-template <int NS, bool COP>
+template <int NS, bool COP, bool TAIL>
 __global__ void __launch_bounds__(256) k_states_multi(const EnsCase *__restrict__ cases, int ncases,
                                                       const DevThermo *__restrict__ th, double ncop_gamma, int full,
                                                       int fill, int where, int sel)
@@ -560,7 +567,7 @@ __global__ void __launch_bounds__(256) k_states_multi(const EnsCase *__restrict_
     const long long b = blockIdx.x;
     const int k = ens_find(cases, ncases, b, 3);
     const EnsCase &c = cases[k];
-    states_block<NS, COP>(c.g, th, c.buf(sel), c.f, ncop_gamma, full, fill ? c.bcs : 0, where, b - c.state_off);
+    states_block<NS, COP, TAIL>(c.g, th, c.buf(sel), c.f, ncop_gamma, full, fill ? c.bcs : 0, where, b - c.state_off);
 }
 
 // ---------------------------------------------------------------------------
