@@ -70,3 +70,34 @@ def test_ensemble_on_either_side():
     ens.close()
     for c in alone + together:
         c.close()
+
+
+@pytest.mark.parametrize("stops", [0, 1, 2])
+def test_ensemble_case_that_has_stopped(stops):
+    """A case that has reached its target time neither holds back the chemistry of the
+    cells that share a wave with its own, nor goes on itself."""
+    announce("ensemble with a stopped case %d" % stops)
+    setups = [xf.Setup(xf.case_path("reactive-channel"), nx=n, ny=11) for n in (13, 9, 15)]
+    states = [s.initial("reactive-channel", seed=7 + k) for k, s in enumerate(setups)]
+
+    def started():
+        out = [s.context() for s in setups]
+        for c, (U, T) in zip(out, states):
+            c.upload(U, T)
+            c.initialize()
+        out[stops].set_target_time(1.5 * out[stops].get_dt())
+        return out
+
+    alone, together = started(), started()
+    for c in alone:
+        c.steps(4)
+    ens = xf.Ensemble(together)
+    assert ens.one_launch
+    ens.steps(4)
+    ens.synchronize()
+    for a, b in zip(alone, together):
+        for x, y in zip(a.download(), b.download()):
+            assert np.array_equal(x.view(np.uint64), y.view(np.uint64))
+    ens.close()
+    for c in alone + together:
+        c.close()

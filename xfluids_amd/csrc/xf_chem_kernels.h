@@ -917,7 +917,7 @@ __device__ __forceinline__ void chem_queue_run(const Cases &cases, long long tot
                     cc = cases.get(ck);
                 }
                 // the cells of a case whose step has halted are skipped
-                if (t < total && !step_halted(cc.err, ~EBIT_CHEM)) {
+                if (t < total && !lane_halted(cc.err, ~EBIT_CHEM)) {
                     tl = t - cc.off;
                     const long long N = cc.g.N;
                     id = chem_cell_id(cc.g, tl);

@@ -65,7 +65,7 @@ struct DevMech {
     DevRxn rx[MAXNR];
     DevWaveRxn wr[MAXNR];
     unsigned wacc[MAXNS * (MAXNR / 4)]; // species n: nu_f | nu_b << 4 of each reaction, a byte each
-    int wave_ok; // every reaction fits its DevWaveRxn, and EaR is 0 or within [2^-500, 2^500]
+    int wave_ok, pad; // wave_ok: every reaction fits its DevWaveRxn, EaR is 0 or within [2^-500, 2^500]
 };
 
 // Geometry passed by value to every kernel
@@ -235,7 +235,15 @@ struct StepState {
         return (b | h) != 0;
     }
 };
+// the same test where it stands; err the same on every lane of the wave
 __device__ __forceinline__ bool step_halted(int *err, int mask) { return StepState(err).halted(mask); }
+// err of the lane's own case
+__device__ __forceinline__ bool lane_halted(int *err, int mask)
+{
+    const int h = err[ERR_HALT], b = err[ERR_BITS] & mask;
+    if (b != 0 && h == 0) err[ERR_HALT] = 1;
+    return (b | h) != 0;
+}
 
 // One scalar load per cache line of a kernel's arguments (or of an ensemble's case),
 // all in flight together.  The compiler loads the arguments where they are first used,

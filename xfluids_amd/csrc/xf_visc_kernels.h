@@ -324,7 +324,7 @@ k_transport(Geom g, const DevThermo *__restrict__ th, const DevTransport *__rest
 {
     constexpr int E = NS + 4;
     constexpr int NCOP = NS - 1;
-    touch_args<sizeof(Geom) + sizeof(Fields) + 40>();
+    touch_args<sizeof(Geom) + sizeof(Fields) + 32>();
     const StepState step(f.err); // tested once the first loads are on their way
     const long long N = g.N;
     const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
