@@ -900,15 +900,15 @@ __device__ __forceinline__ void chem_queue_run(const Cases &cases, long long tot
     double e0 = 0.0;
     bool active = false, done = false, can_spill = sp.cap > 0;
     for (;;) {
-        const bool need = !active && !done;
-        const unsigned long long want = __ballot(need);
-        if (want) {
+        // every lane without a cell draws until it has one or the queue is empty; the
+        // cells of a case whose step has halted are passed over
+        while (const unsigned long long want = __ballot(!active && !done)) {
             const int cnt = __popcll(want);
             const int leader = __ffsll((long long)want) - 1;
             unsigned long long base = 0;
             if (lane == leader) base = atomicAdd(queue, (unsigned long long)cnt);
             base = __shfl(base, leader);
-            if (need) {
+            if (!active && !done) {
                 const int rank = __popcll(want & ((1ull << lane) - 1ull));
                 const long long t = (long long)(base + (unsigned long long)rank);
                 ChemCase cc{};
@@ -916,7 +916,6 @@ __device__ __forceinline__ void chem_queue_run(const Cases &cases, long long tot
                     ck = cases.find_k(t);
                     cc = cases.get(ck);
                 }
-                // the cells of a case whose step has halted are skipped
                 if (t < total && !lane_halted(cc.err, ~EBIT_CHEM)) {
                     tl = t - cc.off;
                     const long long N = cc.g.N;
@@ -930,6 +929,10 @@ __device__ __forceinline__ void chem_queue_run(const Cases &cases, long long tot
                     active = true;
                 } else if (t >= total) {
                     done = true;
+                } else if (rank == cnt - 1) {
+                    // the wave's last index lies in a halted case: the counter goes on
+                    // behind it (every index up to there is one of that case's cells)
+                    atomicMax(queue, (unsigned long long)(cc.off + (long long)cc.g.X_inner * cc.g.Y_inner * cc.g.Z_inner));
                 }
             }
         }
