@@ -25,6 +25,10 @@
 namespace xf {
 
 constexpr int CHEM_MAXSUB = 200000;
+// the bits a chemistry launch may set, which it therefore does not test: the pass bound,
+// and the NaN check of the cells it has written (a NaN of an earlier launch has been
+// latched by the Reaction's UpdateStates, which runs in between)
+constexpr int CHEM_BITS = EBIT_CHEM | EBIT_NAN;
 
 __device__ __forceinline__ double pown_i(double x, int n)
 {
@@ -798,7 +802,7 @@ k_chem(Geom g, const DevThermo *__restrict__ th, const DevMech *__restrict__ mc,
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long total = (long long)g.X_inner * g.Y_inner * g.Z_inner;
     if (t >= total) return;
-    if (step_halted(f.err, ~EBIT_CHEM)) return;
+    if (step_halted(f.err, ~CHEM_BITS)) return;
     const int i = g.Bx + (int)(t % g.X_inner);
     const int j = g.By + (int)((t / g.X_inner) % g.Y_inner);
     const int k = g.Bz + (int)(t / ((long long)g.X_inner * g.Y_inner));
@@ -916,7 +920,7 @@ __device__ __forceinline__ void chem_queue_run(const Cases &cases, long long tot
                     ck = cases.find_k(t);
                     cc = cases.get(ck);
                 }
-                if (t < total && !lane_halted(cc.err, ~EBIT_CHEM)) {
+                if (t < total && !lane_halted(cc.err, ~CHEM_BITS)) {
                     tl = t - cc.off;
                     const long long N = cc.g.N;
                     id = chem_cell_id(cc.g, tl);
@@ -1531,7 +1535,7 @@ k_chem_wave(Geom g, const DevThermo *__restrict__ th, const DevMech *__restrict_
 {
     const long long tl = blockIdx.x;
     if (tl >= (long long)g.X_inner * g.Y_inner * g.Z_inner) return;
-    if (step_halted(f.err, ~EBIT_CHEM)) return;
+    if (step_halted(f.err, ~CHEM_BITS)) return;
     __shared__ WaveShared<NS> sh;
     chem_wave_cell<NS, THERMO>(th, mc, one_case(g, f).c, tl, record, check, sh);
 }

@@ -171,11 +171,13 @@ constexpr int EBIT_CHEM = 8;
 // bit in ERR_BITS, the lowest failing cell id of that bit in ERR_ID + b
 // (b = 0 rho/Y, 1 primitives, 2 NaN check, 3 chemistry), and the step and
 // stage it ran in.  Every kernel of a step returns at entry once an earlier
-// launch has failed (ERR_HALT, latched by the one-lane and fold kernels
-// between passes, or a bit that the kernel itself never sets), so the state
-// stays as the failing pass left it, as the reference stops its time loop
-// there (src/XFLUIDS.cpp:211-225, 285-287).  A kernel never consults bits its
-// own launch may set, so the recorded cell does not depend on block order.
+// launch has failed: ERR_HALT, or a bit that the kernel itself never sets, so the
+// state stays as the failing pass left it, as the reference stops its time loop
+// there (src/XFLUIDS.cpp:211-225, 285-287).  A kernel's mask leaves out every bit
+// that its own launch may set, so the recorded cell and the work done do not depend
+// on block order; a kernel that finds such a bit stores ERR_HALT for the later ones
+// that do not test it, which other blocks of its launch may then read: they find
+// the bit as well.
 constexpr int ERR_BITS = 0;
 constexpr int ERR_ID = 1;    // 4 slots
 constexpr int ERR_STEP = 5;  // step counter (Iteration) of the failing pass
