@@ -339,10 +339,13 @@ int xf_ensemble_synchronize(xf_ensemble *ens);
 long long xf_ensemble_cells(const xf_ensemble *ens);
 /* 1 when each ensemble step is one launch per kernel class over the cells of
    every case (the cases agree in species count, scheme, precision, active
-   directions and the limiter, and none is viscous; the tile shapes are the
-   first case's at creation), 0 when each case's stages run on its own
-   stream with one shared chemistry launch. */
+   directions and the limiter, and none is viscous), 0 when each case's stages
+   run on its own stream with one shared chemistry launch. */
 int xf_ensemble_one_launch(const xf_ensemble *ens);
+/* Sweep tile shapes of the one-launch form, fixed at creation: the first case's where
+   xf_set_tile_shape or xf_autotune has chosen one, else the shape that needs the
+   fewest blocks over all cases.  XF_EINVAL without that form. */
+int xf_ensemble_tile_shape(const xf_ensemble *ens, int *shape3);
 void xf_ensemble_destroy(xf_ensemble *ens);
 /* Evaluate the device exp and log (the fixed-sequence FP64 functions every
    kernel uses) on n host values; for bit-level checks against the CPU. */

@@ -166,6 +166,7 @@ _SIGS = {
     "xf_ensemble_synchronize": (C.c_int, [_V]),
     "xf_ensemble_cells": (C.c_longlong, [_V]),
     "xf_ensemble_one_launch": (C.c_int, [_V]),
+    "xf_ensemble_tile_shape": (C.c_int, [_V, C.POINTER(C.c_int)]),
     "xf_ensemble_destroy": (None, [_V]),
 }
 
@@ -567,6 +568,14 @@ class Ensemble:
     def one_launch(self):
         """True when each step is one launch per kernel class over all cases."""
         return lib().xf_ensemble_one_launch(self._h) == 1
+
+    def tile_shape(self):
+        """Sweep tile shape per direction of the one-launch form (xf_ensemble_tile_shape)."""
+        out = np.zeros(3, np.int32)
+        st = lib().xf_ensemble_tile_shape(self._h, _i(out))
+        if st:
+            raise XfError(st, "xf_ensemble_tile_shape")
+        return out
 
     @property
     def cells(self):

@@ -343,7 +343,7 @@ int xf_create(const xf_case_desc *desc, xf_ctx **out)
     g.Yil_limiter = d.Yil_limiter;
     g.Dim_limiter = d.Dim_limiter;
     g.N = c->N;
-    for (int q = 0; q < 3; q++) c->shape[q] = default_tile_shape(g, q);
+    for (int q = 0; q < 3; q++) c->shape[q] = fewest_blocks(q, [&](int s) { return tile_blocks(g, q, s); });
     auto fail = [&](int code) {
         xf_destroy(c);
         return code;
@@ -1052,6 +1052,7 @@ int xf_set_tile_shape(xf_ctx *c, int dir, int shape)
     if (!c || dir < 0 || dir > 2 || shape < 0) return XF_EINVAL;
     const int count = dir == 0 ? SweepShapes<0>::count : SweepShapes<1>::count;
     if (shape >= count) return XF_EINVAL;
+    c->shape_set[dir] = true;
     if (c->shape[dir] != shape) {
         c->shape[dir] = shape;
         // the captured step graph holds the old kernels
@@ -1107,6 +1108,7 @@ int xf_autotune(xf_ctx *c, int reps, int *shape3, double *ms)
                 if (rc == XF_OK && (k == 0 || t < best_ms)) best = k, best_ms = t;
             }
             c->shape[dir] = best;
+            c->shape_set[dir] = true;
         }
     }
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec), c->gexec = nullptr;
@@ -1364,7 +1366,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
         }
     }
     // the one-launch form: cases that agree in everything the launches are
-    // specialised on, with the template case's tile shapes
+    // specialised on, with tile shapes for all of them together
     bool multi = !c0->d.visc && !c0->d.ghost;
     for (int k = 0; k < ncases && multi; k++) {
         const xf_case_desc &d = cases[k]->d, &d0 = c0->d;
@@ -1375,7 +1377,14 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
     }
     if (multi) {
         std::vector<EnsCase> t(ncases);
-        for (int q = 0; q < 3; q++) e->shape[q] = c0->shape[q];
+        for (int q = 0; q < 3; q++) {
+            auto blocks = [&](int s) {
+                long long n = 0;
+                for (int k = 0; k < ncases; k++) n += tile_blocks(cases[k]->g, q, s);
+                return n;
+            };
+            e->shape[q] = c0->shape_set[q] ? c0->shape[q] : fewest_blocks(q, blocks);
+        }
         long long sb = 0, tb[3] = {0, 0, 0};
         for (int k = 0; k < ncases; k++) {
             xf_ctx *c = cases[k];
@@ -1391,7 +1400,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
             r.bcs = bcs | (1 << 28);
             for (int dd = 0; dd < 3; dd++) {
                 unsigned gr[5];
-                sweep_grid(c->g, dd, e->shape[dd], gr);
+                sweep_grid(c->g, dd, e->shape[dd], tile_blocks(c->g, dd, e->shape[dd]), gr);
                 for (int q = 0; q < 5; q++) r.tiles[dd][q] = (int)gr[q];
                 r.tile_off[dd] = tb[dd];
                 tb[dd] += (long long)gr[0] * gr[1] * gr[2];
@@ -1442,6 +1451,13 @@ int xf_ensemble_synchronize(xf_ensemble *e)
 long long xf_ensemble_cells(const xf_ensemble *e) { return e ? e->total : 0; }
 
 int xf_ensemble_one_launch(const xf_ensemble *e) { return e ? (e->multi ? 1 : 0) : XF_EINVAL; }
+
+int xf_ensemble_tile_shape(const xf_ensemble *e, int *shape3)
+{
+    if (!e || !shape3 || !e->multi) return XF_EINVAL;
+    for (int d = 0; d < 3; d++) shape3[d] = e->shape[d];
+    return XF_OK;
+}
 
 void xf_ensemble_destroy(xf_ensemble *e)
 {

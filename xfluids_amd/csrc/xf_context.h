@@ -44,8 +44,8 @@ struct Ops {
     void (*visc_prep)(xf_ctx *, const double *Ug);
     void (*visc_flux)(xf_ctx *, int dir, const double *Ug);
     // one launch over every case of an ensemble (case table on the device;
-    // sel codes pick U, U1 or U2 per case; the scheme, precision and tile
-    // shape are those of the template case c0)
+    // sel codes pick U, U1 or U2 per case; the scheme and precision are those of
+    // the template case c0)
     // fold: some case's blocks are too many for the sweeps to fold
     void (*states_multi)(const xf_ctx *c0, hipStream_t, const EnsCase *, int ncases, long long blocks, int full,
                          int fill, int where, int sel, bool fold);
@@ -96,6 +96,7 @@ struct xf_ctx {
     int mech_spec = -1;
     bool spec_allowed = true;
     int shape[3] = {0, 0, 0}; // sweep tile shape per direction (SweepShape)
+    bool shape_set[3] = {false, false, false}; // chosen by the caller or the autotuner
     hipGraph_t graph = nullptr;
     hipGraphExec_t gexec = nullptr;
     int last_code = 0, last_id = -1;
@@ -120,50 +121,63 @@ namespace xf {
 
 inline unsigned nblk(long long n, int b = 256) { return (unsigned)((n + b - 1) / b); }
 
-// tile grid of a sweep in direction dir with tile shape `shape` (TS faces by
-// TW = 256 / TS pencils, the shapes of SweepShape): x tiles along the sweep
-// axis of x, pencil rows, third axis; then the cells a tile covers along the
-// sweep and (y, z) its columns.  As a rule a direction takes full tiles and a
-// remainder.  Its cells are spread evenly over the same number of tiles instead
-// where that would leave waves with a few active lanes: those run at half speed or
-// less.  Along the sweep when the remainder is at most TS / 16 cells (64 cells in x
-// as 63 + 1 took 129 us at 64^3 and nine species, as 32 + 32 110), and in every
-// launch of under two blocks per CU (one species: 15.2 us at 64^2 and 65^2, 7.8 at
-// 63^2; evenly 7.8 at each).  With fuller remainders even tiles cost 1-2 %, and
-// even columns, whose rows then straddle cache lines, up to 5 %.
-inline void sweep_grid(const Geom &g, int dir, int shape, unsigned out[5])
+// faces along the sweep of a tile of shape `shape` in direction dir (the shapes of
+// SweepShape); it has 256 / that many pencils
+inline int tile_faces(int dir, int shape)
 {
-    const int TS = dir == 0 ? (shape == 0 ? 64 : 32) : (shape == 0 ? 16 : (shape == 1 ? 32 : 8));
-    const int TW = 256 / TS;
+    return dir == 0 ? (shape == 0 ? 64 : 32) : (shape == 0 ? 16 : (shape == 1 ? 32 : 8));
+}
+
+// tile grid of a sweep in direction dir with tile shape `shape` (TS faces by
+// TW = 256 / TS pencils): x tiles along the sweep axis of x, pencil rows, third axis;
+// then the cells a tile covers along the sweep and (y, z) its columns.  launch: the
+// blocks of the launch (tile_blocks).  As a rule
+// a direction takes full tiles and a remainder.  Its cells are spread evenly over the
+// same number of tiles instead where that would leave waves with a few active lanes:
+// those run at half speed or less.  Along the sweep when the remainder is at most
+// TS / 16 cells (64 cells in x as 63 + 1 took 129 us at 64^3 and nine species, as
+// 32 + 32 110), and in every launch of under two blocks per CU (one species: 15.2 us
+// at 64^2 and 65^2, 7.8 at 63^2; evenly 7.8 at each).  With fuller remainders even
+// tiles cost 1-2 %, and even columns, whose rows then straddle cache lines, up to 5 %.
+inline void sweep_grid(const Geom &g, int dir, int shape, long long launch, unsigned out[5])
+{
+    const int TS = tile_faces(dir, shape), TW = 256 / TS;
     auto tiles = [](int n, int most) { return (unsigned)((n + most - 1) / most); };
     const int inner = dir == 0 ? g.X_inner : (dir == 1 ? g.Y_inner : g.Z_inner);
     const unsigned along = tiles(inner, TS - 1), across = tiles(dir == 0 ? g.Y_inner * g.Z_inner : g.X_inner, TW);
     out[0] = dir == 0 ? along : across;
     out[1] = dir == 0 ? across : along;
     out[2] = dir == 0 ? 1 : (unsigned)(dir == 1 ? g.Z_inner : g.Y_inner);
-    const bool small = (long long)out[0] * out[1] * out[2] < 512;
+    const bool small = launch < 512;
     const int rest = inner - (int)(along - 1) * (TS - 1);
     out[3] = small || rest <= TS / 16 ? tiles(inner, (int)along) : TS - 1;
     out[4] = small && dir != 0 ? tiles(g.X_inner, (int)across) : TW;
 }
+// its blocks, which do not depend on the launch's
+inline long long tile_blocks(const Geom &g, int dir, int shape)
+{
+    unsigned gr[5];
+    sweep_grid(g, dir, shape, 0, gr);
+    return (long long)gr[0] * gr[1] * gr[2];
+}
 
-// The tile shape a context starts with (xf_set_tile_shape and xf_autotune change
-// it): the one with the fewest blocks, since every block runs the same instructions
-// whatever part of its lanes has a face; ties take the lower number.  8 x 32 tiles
-// in y and z stage 13 cells for every 7 they finish and must save more than a
-// quarter of the blocks.  Measured at nine species (x 64 x 4 / 32 x 8): 128^3
-// 624 / 544 us with 12288 / 10240 blocks, 64^3 130 / 84 with 2048 / 1536, 100^3 289 /
-// 281 with 5000 each; y (16 x 16 / 32 x 8 / 8 x 32): 128^3 541 / 578 / 852 with 9216 /
-// 10240 / 9728; three species at 97 x 48 x 48 50.8 / 43.7 / 59.6 with 1344 / 1248 /
-// 1344.
-inline int default_tile_shape(const Geom &g, int dir)
+// The tile shape a context or an ensemble starts with (xf_set_tile_shape and
+// xf_autotune change it): the one with the fewest blocks, blocks(shape) those of its
+// launch, since every block runs the same instructions whatever part of its lanes has
+// a face; ties take the lower number.  8 x 32 tiles in y and z stage 13 cells for every
+// 7 they finish and must save more than a quarter of the blocks.  Measured at nine
+// species (x 64 x 4 / 32 x 8): 128^3 624 / 544 us with 12288 / 10240 blocks, 64^3 130 /
+// 84 with 2048 / 1536, 100^3 289 / 281 with 5000 each; y (16 x 16 / 32 x 8 / 8 x 32):
+// 128^3 541 / 578 / 852 with 9216 / 10240 / 9728; three species at 97 x 48 x 48 50.8 /
+// 43.7 / 59.6 with 1344 / 1248 / 1344.  An ensemble of a 64 x 7 and eight 256 x 256
+// channels: 2122 us a step with the shapes of all its cases (x 32 x 8, y 16 x 16), 2284
+// with those of the first one alone (y 8 x 32).
+template <class F> int fewest_blocks(int dir, F blocks)
 {
     double best = 0.0;
     int shape = 0;
     for (int s = 0; s < (dir == 0 ? 2 : 3); s++) {
-        unsigned gr[5];
-        sweep_grid(g, dir, s, gr);
-        const double cost = (double)gr[0] * gr[1] * gr[2] * (s == 2 ? 1.35 : 1.0);
+        const double cost = (double)blocks(s) * (s == 2 ? 1.35 : 1.0);
         if (s == 0 || cost < best) best = cost, shape = s;
     }
     return shape;

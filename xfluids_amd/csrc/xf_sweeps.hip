@@ -12,9 +12,9 @@ template <int NS, bool COP, int SCH> struct SweepKernels {
         constexpr int E = COP ? NS + 4 : 5;
         static_assert(SweepShape<DIR, E, SHAPE>::TS == (DIR == 0 ? (SHAPE == 0 ? 64 : 32)
                                                                  : (SHAPE == 0 ? 16 : (SHAPE == 1 ? 32 : 8))),
-                      "sweep_grid's tile sizes");
+                      "tile_faces");
         unsigned gr[5];
-        sweep_grid(c->g, DIR, SHAPE, gr);
+        sweep_grid(c->g, DIR, SHAPE, tile_blocks(c->g, DIR, SHAPE), gr);
         static const char *names[3] = {"sweep_x", "sweep_y", "sweep_z"};
         ProfScope ps(c, names[DIR]);
         hipLaunchKernelGGL((k_sweep<NS, COP, DIR, SCH, PREC, SHAPE>), dim3(gr[0], gr[1], gr[2]), dim3(256), 0, c->stream,
