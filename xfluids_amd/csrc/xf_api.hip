@@ -1377,6 +1377,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
     }
     if (multi) {
         std::vector<EnsCase> t(ncases);
+        long long full[3];
         for (int q = 0; q < 3; q++) {
             auto blocks = [&](int s) {
                 long long n = 0;
@@ -1384,6 +1385,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
                 return n;
             };
             e->shape[q] = c0->shape_set[q] ? c0->shape[q] : fewest_blocks(q, blocks);
+            full[q] = blocks(e->shape[q]);
         }
         long long sb = 0, tb[3] = {0, 0, 0};
         for (int k = 0; k < ncases; k++) {
@@ -1400,7 +1402,7 @@ int xf_ensemble_create(xf_ctx *const *cases, int ncases, xf_ensemble **out)
             r.bcs = bcs | (1 << 28);
             for (int dd = 0; dd < 3; dd++) {
                 unsigned gr[5];
-                sweep_grid(c->g, dd, e->shape[dd], tile_blocks(c->g, dd, e->shape[dd]), gr);
+                sweep_grid(c->g, dd, e->shape[dd], full[dd], gr);
                 for (int q = 0; q < 5; q++) r.tiles[dd][q] = (int)gr[q];
                 r.tile_off[dd] = tb[dd];
                 tb[dd] += (long long)gr[0] * gr[1] * gr[2];

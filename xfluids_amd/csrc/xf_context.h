@@ -131,7 +131,7 @@ inline int tile_faces(int dir, int shape)
 // tile grid of a sweep in direction dir with tile shape `shape` (TS faces by
 // TW = 256 / TS pencils): x tiles along the sweep axis of x, pencil rows, third axis;
 // then the cells a tile covers along the sweep and (y, z) its columns.  launch: the
-// blocks of the launch (tile_blocks).  As a rule
+// blocks of the whole launch (tile_blocks, over all cases of an ensemble).  As a rule
 // a direction takes full tiles and a remainder.  Its cells are spread evenly over the
 // same number of tiles instead where that would leave waves with a few active lanes:
 // those run at half speed or less.  Along the sweep when the remainder is at most
