@@ -242,53 +242,66 @@ __device__ __forceinline__ void evalcv_energy(const DevThermo *__restrict__ th, 
     q[0] = q0 * _Cv, d[0] = d0 * _Cv;
 }
 
-// evalcv on the fast path: compiled mechanism SPEC, every lane's temperature
-// and pressure where the fast fits and quotients are exact.  Returns false,
-// with nothing of use in q and d, when that does not hold or when a rate is not
+// What evalcv reads of the species at y[0] = T, for waves whose every lane has T and
+// pressure where the fast fits and quotients are exact: enthalpies and Gibbs energies
+// (Ri = 1), the mixture's Cv and the reactions' context; false otherwise.
+template <int NS>
+__device__ __forceinline__ bool evalcv_species(const DevThermo *__restrict__ th, const double *y, double m_p,
+                                               double *h1, double *gk, double &cv, RxnCtx &c)
+{
+    const double m_tmp = y[0];
+    // mix_cv: the species' part inside, with the range's coefficients
+    double _W = 0.0;
+    cv = 0.0;
+    cdouble *Rk = as_const(th->Ri), *iWk = as_const(th->_Wi);
+    auto species = [&](auto fam) {
+        constexpr bool NASA = decltype(fam)::value;
+        return __all(m_tmp >= 0x1p-100 && m_p >= 0x1p-300 && m_p <= 0x1p300) &&
+               fast_fits<NASA>(th, fast_top(th), m_tmp, true, true, [&](cdouble *cf, auto t) {
+                   c.logT = t.lT, c.rT = t.iT;
+                   if (t.cold) c.logT = dlog_pos(m_tmp), c.rT = ddiv_core(1.0, m_tmp);
+#pragma unroll
+                   for (int n = 0; n < NS; n++) {
+                       h1[n] = h_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT, 1.0);
+                       if (t.cold) h1[n] = t.below(h1[n], cp_fast<NASA>(cf + FITC * n, t.T, t.iT, 1.0));
+                       double g = 0.0;
+                       g += s_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT);
+                       g += dquot(-h1[n], m_tmp, c.rT);
+                       gk[n] = g;
+                       cv += y[1 + n] * cp_fast<NASA>(cf + FITC * n, t.T, t.iT, Rk[n]);
+                   }
+               });
+    };
+    if (!(th->thermo ? species(std::true_type{}) : species(std::false_type{}))) return false;
+#pragma unroll
+    for (int n = 0; n < NS; n++) _W += y[1 + n] * iWk[n];
+    cv -= Ru * _W;
+    c.m_tmp = m_tmp, c.logP = dlog_pos(m_p * (1.0 / 101325.0)), c.t_ok = true;
+    c.logStandConc = dlog_pos(ddiv_core(m_p, R0 * m_tmp));
+    return true;
+}
+
+// evalcv on the fast path with compiled mechanism SPEC.  Returns false, with nothing
+// of use in q and d, where evalcv_species does or when a rate is not
 // finite (a non-finite Kf or Kck reaches some species' sum, and with it the
 // temperature's).
 template <int NS, int SPEC>
 __device__ __forceinline__ bool evalcv_fast(const DevThermo *__restrict__ th, const double *y, double *q, double *d,
                                             double m_dens, double _dens, double m_p)
 {
-    const double m_tmp = y[0];
-    double h1[NS], lg[NS], m_cm[NS];
-    const double logP = dlog_pos(m_p * (1.0 / 101325.0));
-    // mix_cv: the species' part inside, with the range's coefficients
-    double cv = 0.0, _W = 0.0;
+    double h1[NS], lg[NS], m_cm[NS], cv;
     RxnCtx c;
-    cdouble *Rk = as_const(th->Ri), *iWk = as_const(th->_Wi);
-    auto species = [&](auto fam) {
-        constexpr bool NASA = decltype(fam)::value;
-        FastT<NASA> ft(th, th->fast, m_tmp);
-        if (!ft.ok || !__all(m_p >= 0x1p-300 && m_p <= 0x1p300)) return false;
-        ft.each(true, [&](cdouble *cf) {
+    cdouble *iWk = as_const(th->_Wi);
+    if (!evalcv_species<NS>(th, y, m_p, h1, lg, cv, c)) return false;
 #pragma unroll
-            for (int n = 0; n < NS; n++) {
-                h1[n] = h_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, ft.lT, 1.0);
-                double g = 0.0;
-                g += s_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, ft.lT);
-                g += dquot(-h1[n], m_tmp, ft.iT);
-                lg[n] = logP - g;
-                cv += y[1 + n] * cp_fast<NASA>(cf + FITC * n, m_tmp, ft.iT, Rk[n]);
-            }
-        });
-        c.logT = ft.lT, c.rT = ft.iT;
-        return true;
-    };
-    if (!(th->thermo ? species(std::true_type{}) : species(std::false_type{}))) return false;
-#pragma unroll
-    for (int n = 0; n < NS; n++) _W += y[1 + n] * iWk[n];
-    cv -= Ru * _W;
-    c.m_tmp = m_tmp, c.logP = logP, c.t_ok = true;
-    c.logStandConc = dlog_pos(ddiv_core(m_p, R0 * m_tmp));
+    for (int n = 0; n < NS; n++) lg[n] = c.logP - lg[n];
 #pragma unroll
     for (int n = 0; n < NS; n++) m_cm[n] = y[1 + n] * iWk[n] * m_dens * 1.0E-3;
     double *qi = q + 1, *pi = d + 1;
 #pragma unroll
     for (int n = 0; n < NS; n++) qi[n] = 0.0, pi[n] = 0.0;
     rxns_fast<NS, SPEC>(std::make_integer_sequence<int, MechSpec<SPEC>::NR>{}, c, lg, m_cm, qi, pi);
-    evalcv_energy<NS>(th, h1, m_tmp, _dens, cv, q, d);
+    evalcv_energy<NS>(th, h1, y[0], _dens, cv, q, d);
     return __all(fabs(q[0]) < __longlong_as_double(0x7ff0000000000000LL) &&
                  fabs(d[0]) < __longlong_as_double(0x7ff0000000000000LL));
 }
@@ -309,30 +322,33 @@ __device__ __forceinline__ void evalcv_dev(const DevThermo *__restrict__ th, con
         if (evalcv_fast<NS, SPEC>(th, y, q, d, m_dens, _dens, m_p)) return;
     }
     // species Gibbs energy and internal-energy ingredients at T (Ri = 1)
-    const TPre t = th->thermo ? tpre<true>(m_tmp, 1) : tpre<true>(m_tmp, 0);
-    double h1[NS], gk[NS];
+    double h1[NS], gk[NS], cv;
+    RxnCtx c;
+    {
+        const TPre t = th->thermo ? tpre<true>(m_tmp, 1) : tpre<true>(m_tmp, 0);
 #pragma unroll
-    for (int n = 0; n < NS; n++) {
-        h1[n] = h_k(th, t, 1.0, n);
-        double temp = 0.0;
-        temp += s_k(th, t, 1.0, n);
-        temp += (-h1[n] / m_tmp);
-        gk[n] = temp;
+        for (int n = 0; n < NS; n++) {
+            h1[n] = h_k(th, t, 1.0, n);
+            double temp = 0.0;
+            temp += s_k(th, t, 1.0, n);
+            temp += (-h1[n] / m_tmp);
+            gk[n] = temp;
+        }
+        cv = mix_cv<NS>(th, y + 1, t);
+        c.m_tmp = m_tmp;
+        // log T: the fit's log max(T, 200) when T >= 200 (the same call on the same value)
+        c.logT = m_tmp >= 200.0 ? t.lT : dlog(m_tmp);
+        c.logP = dlog(m_p * (1.0 / 101325.0));
+        c.logStandConc = dlog(m_p / (R0 * m_tmp));
+        c.rT = 1.0 / m_tmp;
+        c.t_ok = __all(m_tmp >= 0x1p-500 && m_tmp <= 0x1p500);
     }
-    const double logStandConc = dlog(m_p / (R0 * m_tmp));
-    // log T: the fit's log max(T, 200) when T >= 200 (the same call on the same value)
-    const double logT = m_tmp >= 200.0 ? t.lT : dlog(m_tmp);
-    const double logP = dlog(m_p * (1.0 / 101325.0));
     double m_cm[NS];
 #pragma unroll
     for (int n = 0; n < NS; n++) m_cm[n] = y[1 + n] * th->_Wi[n] * m_dens * 1.0E-3;
     double *qi = q + 1, *pi = d + 1;
 #pragma unroll
     for (int n = 0; n < NS; n++) qi[n] = 0.0, pi[n] = 0.0;
-    RxnCtx c;
-    c.m_tmp = m_tmp, c.logT = logT, c.logP = logP, c.logStandConc = logStandConc;
-    c.rT = 1.0 / m_tmp;
-    c.t_ok = __all(m_tmp >= 0x1p-500 && m_tmp <= 0x1p500);
     const int NR = mc->NR;
     for (int r = 0; r < NR; r++) {
         // the uniform record, read in one burst of scalar loads
@@ -340,7 +356,7 @@ __device__ __forceinline__ void evalcv_dev(const DevThermo *__restrict__ th, con
         const double *er = mc->third + r * NS;
         rxn_step<NS>(R, [er](int it) { return er[it]; }, c, gk, m_cm, qi, pi);
     }
-    evalcv_energy<NS>(th, h1, m_tmp, _dens, mix_cv<NS>(th, y + 1, t), q, d);
+    evalcv_energy<NS>(th, h1, m_tmp, _dens, cv, q, d);
 }
 
 // evalcv with the work of one cell spread over the 64 lanes of a wave, every
@@ -696,14 +712,15 @@ __device__ __forceinline__ double mix_e(const DevThermo *__restrict__ th, const 
     cdouble *Rk = as_const(th->Ri);
     auto sum = [&](auto fam) {
         constexpr bool NASA = decltype(fam)::value;
-        FastT<NASA> ft(th, th->fast, T);
-        if (ft.ok) {
-            ft.each(NASA, [&](cdouble *c) {
+        if (fast_fits<NASA>(th, fast_top(th), T, true, NASA, [&](cdouble *c, auto t) {
 #pragma unroll
-                for (int n = 0; n < NS; n++) e += (h_fast<NASA>(c + FITC * n, T, ft.iT, ft.lT, 1.0) - T) * Rk[n] * yi[n];
-            });
+                for (int n = 0; n < NS; n++) {
+                    double h = h_fast<NASA>(c + FITC * n, t.T, t.iT, t.lT, 1.0);
+                    if (t.cold) h = t.below(h, cp_fast<NASA>(c + FITC * n, t.T, t.iT, 1.0));
+                    e += (h - T) * Rk[n] * yi[n];
+                }
+            }))
             return;
-        }
         const TPre t = tpre<NASA>(T, NASA ? 1 : 0);
 #pragma unroll
         for (int n = 0; n < NS; n++) {

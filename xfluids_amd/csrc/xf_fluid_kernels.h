@@ -405,17 +405,14 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
             double cpk[NS], hk[NS];
             auto species = [&](auto fam) {
                 constexpr bool NASA = decltype(fam)::value;
-                FastT<NASA> ft(th, th->fast, T);
                 cdouble *Rk = as_const(th->Ri);
-                if (ft.ok) {
-                    ft.each(NASA, [&](cdouble *cf) {
+                if (!fast_fits<NASA>(th, fast_top(th), T, true, NASA, [&](cdouble *cf, auto t) {
 #pragma unroll
                         for (int n = 0; n < NS; n++) {
-                            cpk[n] = cp_fast<NASA>(cf + FITC * n, T, ft.iT, Rk[n]);
-                            hk[n] = h_fast<NASA>(cf + FITC * n, T, ft.iT, ft.lT, Rk[n]);
+                            cpk[n] = cp_fast<NASA>(cf + FITC * n, t.T, t.iT, Rk[n]);
+                            hk[n] = t.below(h_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT, Rk[n]), cpk[n]);
                         }
-                    });
-                } else {
+                    })) {
                     const TPre t = tpre<NASA>(T, NASA ? 1 : 0);
 #pragma unroll 1
                     for (int n = 0; n < NS; n++) {

@@ -9,6 +9,7 @@
 // once per species (identical values), and loops over species are unrolled
 // for a compile-time species count NS.
 #pragma once
+#include <type_traits>
 #include "xf_internal.h"
 #include "xf_dev_math.h"
 
@@ -138,13 +139,14 @@ __device__ __forceinline__ bool table_fast(const DevThermo *__restrict__ th)
     return *(const int __attribute__((address_space(4))) *)(unsigned long long)&th->fast != 0;
 }
 
-// ---- the fits on a temperature every lane of the wave is known to share a
-// fit range at, 200 K <= T <= 1e5 K (FastT below): the same expressions with the
-// fit family as a constant and one exact shortcut.  -c0 / T takes the corrected
+// ---- the fits on a clamped temperature, 200 K <= T <= 1e5 K on every lane of the
+// wave (FastT below): the same expressions with the fit family as a constant and one
+// exact shortcut.  -c0 / T takes the corrected
 // quotient of the shared reciprocal (DevThermo::fast says that every coefficient
 // is 0 or within [2^-300, 2^300], so nothing leaves the quotient's range; c0 = 0
 // gives a zero, which adds nothing).  No branch on the family, the range or
-// T < 200 is left inside the species loops, so the species' chains overlap: a
+// T < 200 is left inside the species loops (a wave with colder lanes runs a copy of
+// its own, FastT), so the species' chains overlap: a
 // Newton iteration at nine species is one basic block instead of some thirty,
 // and k_states<9> at 8192 cells (a launch as long as its longest Newton chain)
 // went from 44.7 to 24.5 us, on a 128^3 mixing layer from 223 to 181 us.
@@ -169,36 +171,61 @@ __device__ __forceinline__ double s_fast(P c, double T, double iT, double lT)
     return (c[0] * lT + (c[1] + (c[14] + (c[15] + c[16] * T) * T) * T) * T + c[6]);
 }
 
-// The per-temperature values of the fast fits.  ok: the table qualifies and
-// every active lane with run set has 200 K <= T <= 1e5 K.  each(body) runs body(c)
-// with the coefficients of the lane's fit range at c + FITC * species, c the same on
-// every lane that runs it together (scalar loads shared by the wave): once for a wave
-// in one range, once per range for a wave that straddles a limit.
-template <bool NASA> struct FastT {
-    double T, iT, lT;
-    const DevThermo *__restrict__ th;
-    bool ok;
-    // fast_: th_->fast, read once by the caller
-    __device__ __forceinline__ FastT(const DevThermo *__restrict__ th_, int fast_, double T_, bool run = true)
+// The per-temperature values of the fast fits: T = max(T0, 200) and what follows from
+// it.  COLD: some lane of the wave is below 200 K.
+template <bool COLD> struct FastT {
+    static constexpr bool cold = COLD;
+    double T0, T, iT, lT;
+    // a species' enthalpy h at T as that at T0, by the linear extrapolation below 200 K;
+    // Cp its heat capacity at T
+    __device__ __forceinline__ double below(double h, double Cp) const
     {
-        th = th_;
-        T = T_;
-        ok = fast_ && __all(!run || (T >= 200.0 && T <= 1.0e5));
-    }
-    template <class F> __device__ __forceinline__ void each(bool need_log, F body)
-    {
-        iT = ddiv_core(1.0, T);
-        lT = need_log ? dlog_pos(T) : 0.0;
-        // the ranges of tpre at T >= 200
-        const int r = NASA ? (T >= 6000.0 ? 2 : (T >= 1000.0 ? 1 : 0)) : (T > 1000.0 ? 0 : 1);
-#pragma unroll 1
-        for (int q = 0; q < (NASA ? 3 : 2); q++) {
-            int ru = q; // hidden from the compiler, which would put r for q in the address
-            asm volatile("" : "+s"(ru));
-            if (r == q) body(as_const(th->Hf + ru * (MAXNS * FITC)));
-        }
+        return COLD && T0 < 200.0 ? h + Cp * (T0 - 200.0) : h;
     }
 };
+// the highest temperature of the fast fits: 1e5 K, or a NaN, which no temperature is
+// below, where the table does not qualify
+__device__ __forceinline__ double fast_top(const DevThermo *__restrict__ th)
+{
+    return th->fast ? 1.0e5 : __longlong_as_double(0x7ff8000000000000LL);
+}
+template <bool NASA, bool COLD, class F>
+__device__ __forceinline__ void fast_ranges(const DevThermo *__restrict__ th, double T0, bool need_log, F body)
+{
+    FastT<COLD> t;
+    t.T0 = T0;
+    t.T = COLD ? dmax(T0, 200.0) : T0;
+    t.iT = ddiv_core(1.0, t.T);
+    t.lT = need_log ? dlog_pos(t.T) : 0.0;
+    // the ranges of tpre at T >= 200
+    const int r = NASA ? (t.T >= 6000.0 ? 2 : (t.T >= 1000.0 ? 1 : 0)) : (t.T > 1000.0 ? 0 : 1);
+#pragma unroll 1
+    for (int q = 0; q < (NASA ? 3 : 2); q++) {
+        int ru = q; // hidden from the compiler, which would put r for q in the address
+        asm volatile("" : "+s"(ru));
+        if (r == q) body(as_const(th->Hf + ru * (MAXNS * FITC)), t);
+    }
+}
+// body(c, t) with the coefficients of the lane's fit range at c + FITC * species, c the
+// same on every lane that runs it together (scalar loads shared by the wave): once for a
+// wave in one range, once per range for a wave that straddles a limit.  False, with
+// nothing run, unless every active lane with run set has T <= top (fast_top, read once
+// by the caller).  The body is there twice, so that a wave at 200 K and above, the usual
+// one, spends nothing on colder ones.  With a loop over the species and vector loads of
+// the coefficients for the colder ones k_states took 438 us on a stream of 150 K at 64^3
+// and nine species (126 now), and a Reaction of one pass a cell 216 (77 now).
+template <bool NASA, class F>
+__device__ __forceinline__ bool fast_fits(const DevThermo *__restrict__ th, double top, double T, bool run,
+                                          bool need_log, F body)
+{
+    if (__builtin_expect(__all(!run || (T >= 200.0 && T <= top)), 1)) {
+        fast_ranges<NASA, false>(th, T, need_log, body);
+        return true;
+    }
+    if (!__all(!run || T <= top)) return false;
+    fast_ranges<NASA, true>(th, T, need_log, body);
+    return true;
+}
 
 // get_CopR (Mixing_device.h:49-56)
 template <int NS>
@@ -282,15 +309,15 @@ template <int NS> struct NewtonTail {
 };
 // runs the cells of the lanes in `left` (at most CELLS, every lane of the wave active)
 // from iteration it on, until each has converged or one leaves the interval of the
-// straight-line fits; returns the iteration reached
+// straight-line fits or falls below 200 K; returns the iteration reached
 template <int NS, bool NASA>
-__device__ __forceinline__ int newton_tail(const DevThermo *__restrict__ th, const double *yi, double e, double R,
-                                           unsigned long long left, int it, double &T, double &root, bool &run)
+__device__ __forceinline__ int newton_tail(const DevThermo *__restrict__ th, typename NewtonTail<NS>::Shared &sh,
+                                           const double *yi, double e, double R, unsigned long long left, int it,
+                                           double &T, double &root, bool &run)
 {
     using TL = NewtonTail<NS>;
     constexpr int L = TL::L;
     static_assert(NS <= L, "a lane per species");
-    __shared__ typename TL::Shared sh;
     const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3;
     const int rank = __popcll(left & ((1ull << lane) - 1ull)); // of a running lane's cell
     auto order = []() {
@@ -359,29 +386,53 @@ __device__ __forceinline__ int newton_tail(const DevThermo *__restrict__ th, con
 }
 
 template <int NS, bool NASA, bool TAIL>
-__device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, const double *yi, double e, double T0)
+__device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, const double *yi, double e, double T0,
+                                            typename NewtonTail<NS>::Shared *sh)
 {
     double T = T0, root = T0;
     const double R = mix_R<NS>(th, yi);
-    const int fast = th->fast;
+    const double top = fast_top(th);
     cdouble *Rk = as_const(th->Ri);
     bool run = true;
-    for (int it = 1; it < 101; it++) {
-        double h = 0.0;
-        double Cp = 0.0;
-        // a lane that has converged goes on about its root, past the result: with the
-        // last few cells alone active a wave runs at half speed on an otherwise idle
-        // chip
-        FastT<NASA> ft(th, fast, T, run);
-        if (ft.ok) {
-            ft.each(NASA, [&](cdouble *c) {
+    double h, Cp;
+    auto sums = [&](cdouble *c, auto t) {
 #pragma unroll
-                for (int n = 0; n < NS; n++) {
-                    const double Ri = Rk[n];
-                    h += h_fast<NASA>(c + FITC * n, T, ft.iT, ft.lT, Ri) * yi[n];
-                    Cp += yi[n] * cp_fast<NASA>(c + FITC * n, T, ft.iT, Ri);
-                }
-            });
+        for (int n = 0; n < NS; n++) {
+            const double Ri = Rk[n], Cpn = cp_fast<NASA>(c + FITC * n, t.T, t.iT, Ri);
+            h += t.below(h_fast<NASA>(c + FITC * n, t.T, t.iT, t.lT, Ri), Cpn) * yi[n];
+            Cp += yi[n] * Cpn;
+        }
+    };
+    // the step of T from the sums; the lanes that go on
+    auto step = [&]() {
+        const double df = newton_step(h, Cp, R, T, e);
+        T = T - df;
+        root = run ? T : root;
+        run = run && !(fabs(df) <= 1.0e-6);
+        return (unsigned long long)__ballot(run);
+    };
+    // a lane that has converged goes on about its root, past the result: with the last
+    // few cells alone active a wave runs at half speed on an otherwise idle chip
+    int it = 1;
+    for (; it < 101 && __all(!run || (T >= 200.0 && T <= top)); it++) {
+        h = 0.0, Cp = 0.0;
+        fast_ranges<NASA, false>(th, T, NASA, sums);
+        const unsigned long long left = step();
+        if (!left) return root;
+        if constexpr (TAIL) {
+            if (it >= NewtonTail<NS>::FROM && __popcll(left) <= NewtonTail<NS>::CELLS && __ballot(1) == ~0ull &&
+                __all(!run || (T >= 200.0 && T <= top))) {
+                it = newton_tail<NS, NASA>(th, *sh, yi, e, R, left, it + 1, T, root, run) - 1;
+                if (!__any(run)) return root;
+            }
+        }
+    }
+    // a loop of its own from the first lane below 200 K (or above the fits' interval) on,
+    // so that the usual waves' stays short
+    for (; it < 101; it++) {
+        h = 0.0, Cp = 0.0;
+        if (__all(!run || T <= top)) {
+            fast_ranges<NASA, true>(th, T, NASA, sums);
         } else {
             const TPre t = tpre<NASA>(T, NASA ? 1 : 0);
 #pragma unroll 1
@@ -393,26 +444,19 @@ __device__ __forceinline__ double get_T_fam(const DevThermo *__restrict__ th, co
                 Cp += y * cp_k(th, t, th->Ri[n], n);
             }
         }
-        const double df = newton_step(h, Cp, R, T, e);
-        T = T - df;
-        root = run ? T : root;
-        run = run && !(fabs(df) <= 1.0e-6);
-        const unsigned long long left = __ballot(run);
-        if (!left) break;
-        if constexpr (TAIL) {
-            if (it >= NewtonTail<NS>::FROM && fast && __popcll(left) <= NewtonTail<NS>::CELLS &&
-                __ballot(1) == ~0ull && __all(!run || (T >= 200.0 && T <= 1.0e5))) {
-                it = newton_tail<NS, NASA>(th, yi, e, R, left, it + 1, T, root, run) - 1;
-                if (!__any(run)) break;
-            }
-        }
+        if (!step()) break;
     }
     return root;
 }
 template <int NS, bool TAIL>
 __device__ __forceinline__ double get_T(const DevThermo *__restrict__ th, const double *yi, double e, double T0)
 {
-    return th->thermo ? get_T_fam<NS, true, TAIL>(th, yi, e, T0) : get_T_fam<NS, false, TAIL>(th, yi, e, T0);
+    typename NewtonTail<NS>::Shared *sh = nullptr;
+    if constexpr (TAIL) {
+        __shared__ typename NewtonTail<NS>::Shared s;
+        sh = &s;
+    }
+    return th->thermo ? get_T_fam<NS, true, TAIL>(th, yi, e, T0, sh) : get_T_fam<NS, false, TAIL>(th, yi, e, T0, sh);
 }
 
 } // namespace xf
