@@ -750,13 +750,21 @@ int xf_download_maxima(xf_ctx *c, double *eigen_block, double *uvw_c_max)
 {
     if (!c) return XF_EINVAL;
     double red[RED_SIZE];
-    // the CFL maxima of the last pass, which a step's own kernels may have folded
-    // for themselves
-    hipLaunchKernelGGL(k_states_fold, dim3(12), dim3(1024), 0, c->stream, c->f.spart, state_blocks(c->g), c->f.red,
-                       c->f.err);
-    if (int e = check_launch()) return e;
     XF_HIP(hipStreamSynchronize(c->stream));
     XF_HIP(hipMemcpy(red, c->f.red, sizeof(red), hipMemcpyDeviceToHost));
+    // the CFL maxima of the last pass: up to FOLD_BLOCKS blocks the step's own kernels
+    // fold them for themselves, and so does this one, without a launch that would write
+    // the slots (an ensemble's steps may be under way on another stream)
+    const int nb = state_blocks(c->g);
+    if (uvw_c_max && nb <= FOLD_BLOCKS) {
+        double part[3 * FOLD_BLOCKS];
+        XF_HIP(hipMemcpy(part, c->f.spart + 9 * (long long)nb, 3 * (size_t)nb * sizeof(double), hipMemcpyDeviceToHost));
+        for (int d = 0; d < 3; d++) {
+            red[RED_DT + d] = 0.0;
+            for (int b = 0; b < nb; b++)
+                if (part[d * nb + b] > red[RED_DT + d]) red[RED_DT + d] = part[d * nb + b];
+        }
+    }
     const int E = c->E;
     if (eigen_block)
         for (int d = 0; d < 3; d++)

@@ -227,8 +227,8 @@ static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__r
 //
 // Up to FOLD_BLOCKS blocks the kernels that use the values (the sweeps, k_dt) fold
 // the planes themselves, each wave on its own while its first loads are in flight;
-// k_states_fold then runs only where the host reads the slots.  A launch costs 4.5 us
-// here however little it does: a 64 x 64 vortex step takes 72.2 us
+// k_states_fold then does not run (xf_download_maxima folds them on the host).  A launch
+// costs 4.5 us here however little it does: a 64 x 64 vortex step takes 72.2 us
 // instead of 76.6, 253 x 190 (202 blocks) 74.5 instead of 79.8.  At 468 blocks a sweep
 // takes 1.3 us longer for it, which is where the line lies: a step 106.7 instead of
 // 107.5.
