@@ -9,6 +9,7 @@
 #include <map>
 #include <string>
 #include <memory>
+#include <new>
 #include <vector>
 
 using namespace xf;
@@ -993,20 +994,22 @@ namespace {
 struct RedGuard {
     xf_ctx *c;
     double h[RED_SIZE];
-    std::vector<double> part;
+    const size_t bytes;
+    std::unique_ptr<char[]> part; // null, and ok false, without memory for it
     bool ok;
-    explicit RedGuard(xf_ctx *c_) : c(c_), part((size_t)state_blocks(c_->g) * 12)
+    explicit RedGuard(xf_ctx *c_)
+        : c(c_), bytes((size_t)state_blocks(c_->g) * 12 * sizeof(double)), part(new (std::nothrow) char[bytes])
     {
-        ok = hipMemcpyAsync(h, c->f.red, sizeof(h), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
-             hipMemcpyAsync(part.data(), c->f.spart, part.size() * sizeof(double), hipMemcpyDeviceToHost,
-                            c->stream) == hipSuccess &&
-             hipStreamSynchronize(c->stream) == hipSuccess;
+        ok = part && hipMemcpyAsync(h, c->f.red, sizeof(h), hipMemcpyDeviceToHost, c->stream) == hipSuccess &&
+             hipMemcpyAsync(part.get(), c->f.spart, bytes, hipMemcpyDeviceToHost, c->stream) == hipSuccess;
+        // also after a failure: the first copy may be under way
+        ok = hipStreamSynchronize(c->stream) == hipSuccess && ok;
     }
     ~RedGuard()
     {
         if (ok) {
             (void)hipMemcpyAsync(c->f.red, h, sizeof(h), hipMemcpyHostToDevice, c->stream);
-            (void)hipMemcpyAsync(c->f.spart, part.data(), part.size() * sizeof(double), hipMemcpyHostToDevice, c->stream);
+            (void)hipMemcpyAsync(c->f.spart, part.get(), bytes, hipMemcpyHostToDevice, c->stream);
             (void)hipStreamSynchronize(c->stream);
         }
     }
