@@ -642,7 +642,17 @@ static int exchange_buffer(xf_ctx *c, long long &cells)
     return XF_OK;
 }
 
-// E planes of N cells to the host's AoS order, after the work on the stream.
+// The copies to and from the caller's memory end before a call returns, also where a
+// later piece fails.
+static int exchange_end(xf_ctx *c, int status)
+{
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess && status == XF_OK) fprintf(stderr, "xfluids_amd: state exchange: %s\n", hipGetErrorString(e));
+    return status ? status : (e != hipSuccess ? XF_EHIP : XF_OK);
+}
+
+// E planes of N cells to the host's AoS order, after the work on the stream
+// (exchange_end after it).
 // 136^3 cells of 13 components (262 MB): 82 ms before, 29 ms now, bound by the
 // copy into the caller's pageable memory (fresh pages here); the upload, which also
 // wrote the state three times over the bus, 110 ms before, 11 ms now.  A 72^2 state:
@@ -662,38 +672,41 @@ static int exchange_out(xf_ctx *c, const double *planes, double *aos)
     return XF_OK;
 }
 
+static int exchange_in(xf_ctx *c, int which, const double *U_aos)
+{
+    // initial state: U1 = U as the reference's initial-condition kernels
+    // set it (e.g. 2D-EulerVortex/ini_sample.hpp:84-88); ghost cells of
+    // an Inflow boundary keep these values for the whole run
+    double *p1 = which == 0 ? c->f.U1 : nullptr, *p2 = which == 0 ? c->U2 : nullptr;
+    long long cells = 0;
+    if (int e = exchange_buffer(c, cells)) return e;
+    for (long long c0 = 0; c0 < c->N; c0 += cells) {
+        const long long n = std::min(cells, c->N - c0);
+        XF_HIP(hipMemcpyAsync(c->xbuf, U_aos + (size_t)c0 * c->E, (size_t)n * c->E * sizeof(double),
+                              hipMemcpyHostToDevice, c->stream));
+        hipLaunchKernelGGL(k_aos_to_planes, dim3(nblk(n)), dim3(256), 256 * (c->E | 1) * sizeof(double), c->stream,
+                           c->xbuf, c->N, c0, n, c->E, which_ptr(c, which), p1, p2);
+        if (int e = check_launch()) return e;
+    }
+    return XF_OK;
+}
+
 int xf_upload_state(xf_ctx *c, int which, const double *U_aos, const double *T)
 {
     if (!c || which < 0 || which > 2) return XF_EINVAL;
-    if (U_aos) {
-        // initial state: U1 = U as the reference's initial-condition kernels
-        // set it (e.g. 2D-EulerVortex/ini_sample.hpp:84-88); ghost cells of
-        // an Inflow boundary keep these values for the whole run
-        double *p1 = which == 0 ? c->f.U1 : nullptr, *p2 = which == 0 ? c->U2 : nullptr;
-        long long cells = 0;
-        if (int e = exchange_buffer(c, cells)) return e;
-        for (long long c0 = 0; c0 < c->N; c0 += cells) {
-            const long long n = std::min(cells, c->N - c0);
-            XF_HIP(hipMemcpyAsync(c->xbuf, U_aos + (size_t)c0 * c->E, (size_t)n * c->E * sizeof(double),
-                                  hipMemcpyHostToDevice, c->stream));
-            hipLaunchKernelGGL(k_aos_to_planes, dim3(nblk(n)), dim3(256), 256 * (c->E | 1) * sizeof(double), c->stream,
-                               c->xbuf, c->N, c0, n, c->E, which_ptr(c, which), p1, p2);
-            if (int e = check_launch()) return e;
-        }
-    }
-    if (T) XF_HIP(hipMemcpyAsync(c->f.T, T, (size_t)c->N * sizeof(double), hipMemcpyHostToDevice, c->stream));
-    XF_HIP(hipStreamSynchronize(c->stream));
-    return XF_OK;
+    int e = U_aos ? exchange_in(c, which, U_aos) : XF_OK;
+    if (!e && T && hipMemcpyAsync(c->f.T, T, (size_t)c->N * sizeof(double), hipMemcpyHostToDevice, c->stream))
+        e = XF_EHIP;
+    return exchange_end(c, e);
 }
 
 int xf_download_state(xf_ctx *c, int which, double *U_aos, double *T)
 {
     if (!c || which < 0 || which > 2) return XF_EINVAL;
-    if (U_aos)
-        if (int e = exchange_out(c, which_ptr(c, which), U_aos)) return e;
-    if (T) XF_HIP(hipMemcpyAsync(T, c->f.T, (size_t)c->N * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    XF_HIP(hipStreamSynchronize(c->stream));
-    return XF_OK;
+    int e = U_aos ? exchange_out(c, which_ptr(c, which), U_aos) : XF_OK;
+    if (!e && T && hipMemcpyAsync(T, c->f.T, (size_t)c->N * sizeof(double), hipMemcpyDeviceToHost, c->stream))
+        e = XF_EHIP;
+    return exchange_end(c, e);
 }
 
 int xf_download_prims(xf_ctx *c, double *rho, double *p, double *u, double *v, double *w, double *H, double *cc,
@@ -742,9 +755,7 @@ int xf_download_prims(xf_ctx *c, double *rho, double *p, double *u, double *v, d
 int xf_download_lu(xf_ctx *c, double *LU_aos)
 {
     if (!c || !LU_aos) return XF_EINVAL;
-    if (int e = exchange_out(c, c->f.LU, LU_aos)) return e;
-    XF_HIP(hipStreamSynchronize(c->stream));
-    return XF_OK;
+    return exchange_end(c, exchange_out(c, c->f.LU, LU_aos));
 }
 
 int xf_download_maxima(xf_ctx *c, double *eigen_block, double *uvw_c_max)
