@@ -185,16 +185,15 @@ int take_error(xf_ctx *c)
     return code;
 }
 
-// FluidBoundaryCondition: all ghost cells in one launch; reset_red also
-// zeroes the per-pass maxima for the UpdateStates pass that follows
-void boundary_async(xf_ctx *c, double *U, int reset_red)
+// FluidBoundaryCondition: all ghost cells in one launch
+void boundary_async(xf_ctx *c, double *U)
 {
     ProfScope ps(c, "boundary");
     const Geom &g = c->g;
     const long long n = (g.DimZ ? 2LL * g.Bz * g.Ymax * g.Xmax : 0) + (g.DimY ? 2LL * g.By * g.Xmax * g.Z_inner : 0) +
                         (g.DimX ? 2LL * g.Bx * g.Y_inner * g.Z_inner : 0);
     hipLaunchKernelGGL(k_boundary_all, dim3(std::max(1u, nblk(n))), dim3(256), 0, c->stream, g, U, c->E, c->d.BC[0],
-                       c->d.BC[1], c->d.BC[2], c->d.BC[3], c->d.BC[4], c->d.BC[5], c->f.red, reset_red);
+                       c->d.BC[1], c->d.BC[2], c->d.BC[3], c->d.BC[4], c->d.BC[5]);
 }
 
 // UpdateStates (the pass's GLF and CFL maxima replace the stored ones);
@@ -231,8 +230,6 @@ void lu_async(xf_ctx *c, const double *Ug, int rk_stage, const double *Ua, const
         c->ops.sweep(c, dirs[q], Ug, mode, rk_stage, Ua, Ub, Uo);
     }
 }
-
-void reaction_prep_async(xf_ctx *c);
 
 // XFLUIDS::Reaction before its chemistry launch: UpdateStates(U) (the step's
 // k_dt has set the chemistry step)
@@ -791,7 +788,7 @@ int xf_download_maxima(xf_ctx *c, double *eigen_block, double *uvw_c_max)
 int xf_boundary(xf_ctx *c, int which)
 {
     if (!c || which < 0 || which > 2) return XF_EINVAL;
-    boundary_async(c, which_ptr(c, which), 0);
+    boundary_async(c, which_ptr(c, which));
     if (int e = check_launch()) return e;
     XF_HIP(hipStreamSynchronize(c->stream));
     return XF_OK;

@@ -148,8 +148,6 @@ __device__ __forceinline__ void bc_apply(double *__restrict__ U, long long N, in
 // cell's value with the momentum sign flips of every map applied.  Sources
 // are interior cells or Inflow ghosts (which no pass writes), so no thread
 // reads a cell another thread writes.  Copies and negations are exact.
-// Thread 0 also zeroes the per-pass reduction slots for the following
-// UpdateStates pass when reset_red is set.
 __device__ __forceinline__ void bc_axis(int bc, int &s, int B, int inner, int Lmax, int mom, int &flip)
 {
     if (s >= B && s < Lmax - B) return;
@@ -161,12 +159,8 @@ __device__ __forceinline__ void bc_axis(int bc, int &s, int B, int inner, int Lm
 }
 
 static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__restrict__ U, int E, int bx0, int bx1, int by0,
-                                                      int by1, int bz0, int bz1, double *red, int reset_red)
+                                                      int by1, int bz0, int bz1)
 {
-    if (reset_red && blockIdx.x == 0 && threadIdx.x < 12) {
-        if (threadIdx.x < 9) red[RED_GLFP + threadIdx.x] = 0.0;
-        else red[RED_DT + threadIdx.x - 9] = 0.0;
-    }
     long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     // enumerate the ghost shell: z slabs, then y slabs inside interior z,
     // then x slabs inside interior y and z
