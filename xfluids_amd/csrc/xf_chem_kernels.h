@@ -50,10 +50,10 @@ struct RxnCtx {
 };
 
 // One reaction's contribution to the production and loss rates (evalcore,
-// ProductionRates.h:117-176).  The record R and the third-body efficiencies
-// eff(s) come either from the device tables (generic loop) or from
-// compile-time constants (a specialisation of a shipped mechanism): the code
-// is this one function in both cases, so the results are the same bits.
+// ProductionRates.h:117-176), from its record R and third-body efficiencies
+// eff(s) in the device tables: the general form, whose values rxn_fast (a compiled
+// mechanism, a lane per cell) and wave_rates (a cell per wave) reproduce bit for bit
+// within their ranges.
 // Species loops run over compile-time n and test the record's masks, which
 // skips exactly the zero-coefficient terms (each adds +0 or multiplies by 1 in
 // the reference, so skipping changes no bit).
@@ -139,9 +139,9 @@ __device__ __forceinline__ void rxn_step(const DevRxn R, Eff eff, const RxnCtx &
 // The rate evaluation is bound by FP64 issue at two waves per SIMD (one lane per
 // cell, ~4250 instructions per pass and cell before, 97 KB of code against the 64
 // KB instruction cache): the fast path below drops what a compiled mechanism and
-// an ordinary state make exact no-ops, and needs no scratch memory.  k_chem at
-// 128^3 went from 1417 to 997 us, k_chem_queue on a 256^2 channel from 149 to
-// 106 us.
+// an ordinary state make exact no-ops, and needs no scratch memory.  k_chem on a
+// 128^3 mixing layer past its start-up went from 1417 to 997 us, k_chem_queue on a
+// 256^2 channel from 149 to 106 us.
 //
 // Reaction r of compiled mechanism K on the fast path of evalcv_dev: rxn_step's
 // values with every test on the record resolved at compile time.  lg = log p - g
@@ -442,8 +442,9 @@ __device__ __forceinline__ double alpha_of(double r)
 // negative, and in_range bounds all of them.  A dividend so small that the remainder
 // underflows leaves a quotient below 2^-890, whose last bits reach nothing: it is only
 // ever added to ymin or more, or competes with eps >= 1e-10.  The temperature's rates
-// may have either sign, and it keeps the IEEE division.  k_chem at 128^3 and one pass
-// per cell went from 997 to 947 us, k_chem_queue on a 256^2 channel from 106 to 102.
+// may have either sign, and it keeps the IEEE division.  k_chem on the 128^3 mixing
+// layer went on from 997 to 947 us, k_chem_queue on the channel from 106 to 102; at one
+// pass a cell a launch on 128^3 takes 480 us now, 771 before both.
 //
 // a non-negative number up to 2^160: its upper word is at most this one
 constexpr unsigned CHEM_IN_RANGE = (1023u + 160u) << 20;

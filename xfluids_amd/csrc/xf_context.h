@@ -169,7 +169,10 @@ inline long long tile_blocks(const Geom &g, int dir, int shape)
 // species (x 64 x 4 / 32 x 8): 128^3 624 / 544 us with 12288 / 10240 blocks, 64^3 130 /
 // 84 with 2048 / 1536, 100^3 289 / 281 with 5000 each; y (16 x 16 / 32 x 8 / 8 x 32):
 // 128^3 541 / 578 / 852 with 9216 / 10240 / 9728; three species at 97 x 48 x 48 50.8 /
-// 43.7 / 59.6 with 1344 / 1248 / 1344.  An ensemble of a 64 x 7 and eight 256 x 256
+// 43.7 / 59.6 with 1344 / 1248 / 1344.  Where 8 x 32 tiles save a quarter (64 cases of
+// 128 x 16, y 16 x 16 / 8 x 32, microseconds a step): one species 289 / 285, three 427 /
+// 406, nine 1089 / 1104; where they save nothing (nine cases of 256 x 256) 377 / 386, 651 /
+// 655 and 2122 / 2298.  An ensemble of a 64 x 7 and eight 256 x 256
 // channels: 2122 us a step with the shapes of all its cases (x 32 x 8, y 16 x 16), 2284
 // with those of the first one alone (y 8 x 32).
 template <class F> int fewest_blocks(int dir, F blocks)

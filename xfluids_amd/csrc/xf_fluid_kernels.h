@@ -222,16 +222,19 @@ static __global__ void __launch_bounds__(256) k_boundary_all(Geom g, double *__r
 // Up to FOLD_BLOCKS blocks the kernels that use the values (the sweeps, k_dt) fold
 // the planes themselves, each wave on its own while its first loads are in flight;
 // k_states_fold then does not run (xf_download_maxima folds them on the host).  A launch
-// costs 4.5 us here however little it does: a 64 x 64 vortex step takes 72.2 us
-// instead of 76.6, 253 x 190 (202 blocks) 74.5 instead of 79.8.  At 468 blocks a sweep
-// takes 1.3 us longer for it, which is where the line lies: a step 106.7 instead of
-// 107.5.
+// costs 4.5 us here however little it does, but the fold takes a sweep longer the more
+// blocks there are.  Microseconds a step with the launch / without: one species 76.8 /
+// 72.0 at 50 blocks, 81 / 76 at 200, 103.0 / 102.8 at 400, 122.5 / 124.4 at 512, 126.4 /
+// 132.3 at 598; three species 139.8 / 132.9, 150 / 142, 181.2 / 178.2, 190.8 / 188.0,
+// 227.9 / 232.8; five in 3-D 385 / 378 at 191, 492.7 / 492.1 at 500, 526.8 / 531.0 at 579.
 constexpr int FOLD_BLOCKS = 512;
 // Up to this many blocks (four on each CU) a states launch is resident at once and
 // lasts as long as its longest Newton chain; above it the registers of newton_tail
-// cost a wave per SIMD and its shorter chains gain nothing (three species at 2096
-// blocks 31.8 us with it, 29.0 without; at 711 blocks and five species 45.5 instead
-// of 54.3, at 33 and nine 16.7 instead of 20.0).
+// cost a wave per SIMD, which short chains do not make up for.  Microseconds a launch
+// without / with it: three species 17.8 / 17.9 at 700 blocks, 19.4 / 18.9 at 1024,
+// 20.9 / 23.2 at 1201, 34.7 / 36.7 at 2996; nine species 20.0 / 16.7 at 33 (a tube),
+// 26.9 / 27.7 at 900, 31.8 / 33.1 at 1199; five species behind a shock, whose chains
+// are long, 60.2 / 48.2 at 873 and still 70.5 / 55.7 at 1175, 119.5 / 97.8 at 2937.
 constexpr long long STATES_TAIL = 1024;
 __host__ __device__ inline int state_blocks(const Geom &g) { return (int)((g.N + 255) / 256); }
 
@@ -488,7 +491,7 @@ __device__ __forceinline__ void states_block(const Geom &g, const DevThermo *__r
             dtm[d] = fabs(uu) + cl;
         }
     }
-    // block reduction: wave butterfly, then one lane per wave folds into LDS
+    // block reduction: each wave's maxima (wave_fold), then the four waves' in LDS
     __shared__ double sred[4][12];
     __shared__ int serr;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;

@@ -247,8 +247,7 @@ __device__ __forceinline__ bool lane_halted(int *err, int mask)
     return (b | h) != 0;
 }
 
-// One scalar load per cache line of a kernel's arguments (or of an ensemble's case),
-// all in flight together.  The compiler loads the arguments where they are first used,
+// One scalar load per cache line of a kernel's arguments, all in flight together.  The compiler loads the arguments where they are first used,
 // in groups that each wait for the one before, with a cold cache at every launch.
 // With the late test above it takes 0.4 us off k_states and a sweep: a step at
 // 253 x 190 73.8 us instead of 75.2, at 350 x 330 104.3 instead of 107.7.

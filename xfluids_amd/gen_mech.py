@@ -8,10 +8,10 @@ evaluation reads (A, B, Ea*4.184/Ru, masks and packed coefficients, exactly as
 xf_set_mechanism builds them, see csrc/xf_api.hip) and the third-body table, as
 constexpr functions.  The chemistry kernels instantiate one rate evaluation per
 record set with these values known at compile time: the mask tests, scalar
-loads and coefficient decoding of the generic loop fold away, and the compiler
-can schedule the nineteen reactions' exponentials together.  The arithmetic is
-the generic loop's own code (rxn_step in csrc/xf_chem_kernels.h), so results
-are bit-identical.
+loads and coefficient decoding of the generic loop fold away, and terms with a
+zero factor are left out.  rxn_fast in csrc/xf_chem_kernels.h computes the values
+of the generic loop's rxn_step in its order, so results are bit-identical; waves
+whose temperatures or rates are out of its range take rxn_step itself.
 
 A context uses a specialisation only when the records it was given compare
 equal field by field (xf_mech_spec_find); any other mechanism runs the generic
