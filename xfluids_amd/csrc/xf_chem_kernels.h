@@ -243,40 +243,53 @@ __device__ __forceinline__ void evalcv_energy(const DevThermo *__restrict__ th, 
 }
 
 // What evalcv reads of the species at y[0] = T, for waves whose every lane has T and
-// pressure where the fast fits and quotients are exact: enthalpies and Gibbs energies
-// (Ri = 1), the mixture's Cv and the reactions' context; false otherwise.
-template <int NS>
+// pressure where the fast fits and quotients are exact: enthalpies and Gibbs energies g
+// (Ri = 1; LG: log p - g in their place), the mixture's Cv and the reactions' context;
+// false otherwise.
+template <int NS, bool LG>
 __device__ __forceinline__ bool evalcv_species(const DevThermo *__restrict__ th, const double *y, double m_p,
                                                double *h1, double *gk, double &cv, RxnCtx &c)
 {
     const double m_tmp = y[0];
+    const double logP = dlog_pos(m_p * (1.0 / 101325.0));
     // mix_cv: the species' part inside, with the range's coefficients
     double _W = 0.0;
     cv = 0.0;
     cdouble *Rk = as_const(th->Ri), *iWk = as_const(th->_Wi);
     auto species = [&](auto fam) {
         constexpr bool NASA = decltype(fam)::value;
-        return __all(m_tmp >= 0x1p-100 && m_p >= 0x1p-300 && m_p <= 0x1p300) &&
-               fast_fits<NASA>(th, fast_top(th), m_tmp, true, true, [&](cdouble *cf, auto t) {
-                   c.logT = t.lT, c.rT = t.iT;
-                   if (t.cold) c.logT = dlog_pos(m_tmp), c.rT = ddiv_core(1.0, m_tmp);
+        const bool p_ok = m_p >= 0x1p-300 && m_p <= 0x1p300;
+        const double top = fast_top(th);
+        auto values = [&](cdouble *cf, auto t) {
+            c.logT = t.lT, c.rT = t.iT;
+            if (t.cold) c.logT = dlog_pos(m_tmp), c.rT = ddiv_core(1.0, m_tmp);
 #pragma unroll
-                   for (int n = 0; n < NS; n++) {
-                       h1[n] = h_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT, 1.0);
-                       if (t.cold) h1[n] = t.below(h1[n], cp_fast<NASA>(cf + FITC * n, t.T, t.iT, 1.0));
-                       double g = 0.0;
-                       g += s_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT);
-                       g += dquot(-h1[n], m_tmp, c.rT);
-                       gk[n] = g;
-                       cv += y[1 + n] * cp_fast<NASA>(cf + FITC * n, t.T, t.iT, Rk[n]);
-                   }
-               });
+            for (int n = 0; n < NS; n++) {
+                h1[n] = h_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT, 1.0);
+                if (t.cold) h1[n] = t.below(h1[n], cp_fast<NASA>(cf + FITC * n, t.T, t.iT, 1.0));
+                double g = 0.0;
+                g += s_fast<NASA>(cf + FITC * n, t.T, t.iT, t.lT);
+                g += dquot(-h1[n], m_tmp, c.rT);
+                gk[n] = LG ? logP - g : g;
+                cv += y[1 + n] * cp_fast<NASA>(cf + FITC * n, t.T, t.iT, Rk[n]);
+            }
+        };
+        // the usual waves by one vote, and the colder ones' copy behind it: with a vote of
+        // its own for each condition a step of a 256^2 channel, one lane per cell, takes
+        // 505 us instead of 497
+        if (__builtin_expect(__all(m_tmp >= 200.0 && m_tmp <= top && p_ok), 1)) {
+            fast_ranges<NASA, false>(th, m_tmp, true, values);
+            return true;
+        }
+        if (!__all(m_tmp >= 0x1p-100 && m_tmp <= top && p_ok)) return false;
+        fast_ranges<NASA, true>(th, m_tmp, true, values);
+        return true;
     };
     if (!(th->thermo ? species(std::true_type{}) : species(std::false_type{}))) return false;
 #pragma unroll
     for (int n = 0; n < NS; n++) _W += y[1 + n] * iWk[n];
     cv -= Ru * _W;
-    c.m_tmp = m_tmp, c.logP = dlog_pos(m_p * (1.0 / 101325.0)), c.t_ok = true;
+    c.m_tmp = m_tmp, c.logP = logP, c.t_ok = true;
     c.logStandConc = dlog_pos(ddiv_core(m_p, R0 * m_tmp));
     return true;
 }
@@ -292,9 +305,7 @@ __device__ __forceinline__ bool evalcv_fast(const DevThermo *__restrict__ th, co
     double h1[NS], lg[NS], m_cm[NS], cv;
     RxnCtx c;
     cdouble *iWk = as_const(th->_Wi);
-    if (!evalcv_species<NS>(th, y, m_p, h1, lg, cv, c)) return false;
-#pragma unroll
-    for (int n = 0; n < NS; n++) lg[n] = c.logP - lg[n];
+    if (!evalcv_species<NS, true>(th, y, m_p, h1, lg, cv, c)) return false;
 #pragma unroll
     for (int n = 0; n < NS; n++) m_cm[n] = y[1 + n] * iWk[n] * m_dens * 1.0E-3;
     double *qi = q + 1, *pi = d + 1;
@@ -326,7 +337,7 @@ __device__ __forceinline__ void evalcv_dev(const DevThermo *__restrict__ th, con
     // species Gibbs energy and internal-energy ingredients at T (Ri = 1)
     double h1[NS], gk[NS], cv;
     RxnCtx c;
-    if (SPEC >= 0 || !evalcv_species<NS>(th, y, m_p, h1, gk, cv, c)) {
+    if (SPEC >= 0 || !evalcv_species<NS, false>(th, y, m_p, h1, gk, cv, c)) {
         const TPre t = th->thermo ? tpre<true>(m_tmp, 1) : tpre<true>(m_tmp, 0);
 #pragma unroll
         for (int n = 0; n < NS; n++) {
@@ -715,15 +726,15 @@ __device__ __forceinline__ double mix_e(const DevThermo *__restrict__ th, const 
     cdouble *Rk = as_const(th->Ri);
     auto sum = [&](auto fam) {
         constexpr bool NASA = decltype(fam)::value;
-        if (fast_fits<NASA>(th, fast_top(th), T, true, NASA, [&](cdouble *c, auto t) {
+        // (twice a cell: the general form below serves the colder waves)
+        if (__all(T >= 200.0 && T <= fast_top(th))) {
+            fast_ranges<NASA, false>(th, T, NASA, [&](cdouble *c, auto t) {
 #pragma unroll
-                for (int n = 0; n < NS; n++) {
-                    double h = h_fast<NASA>(c + FITC * n, t.T, t.iT, t.lT, 1.0);
-                    if (t.cold) h = t.below(h, cp_fast<NASA>(c + FITC * n, t.T, t.iT, 1.0));
-                    e += (h - T) * Rk[n] * yi[n];
-                }
-            }))
+                for (int n = 0; n < NS; n++)
+                    e += (h_fast<NASA>(c + FITC * n, t.T, t.iT, t.lT, 1.0) - T) * Rk[n] * yi[n];
+            });
             return;
+        }
         const TPre t = tpre<NASA>(T, NASA ? 1 : 0);
 #pragma unroll
         for (int n = 0; n < NS; n++) {

@@ -213,7 +213,7 @@ __device__ __forceinline__ void fast_ranges(const DevThermo *__restrict__ th, do
 // by the caller).  The body is there twice, so that a wave at 200 K and above, the usual
 // one, spends nothing on colder ones.  With a loop over the species and vector loads of
 // the coefficients for the colder ones k_states took 438 us on a stream of 150 K at 64^3
-// and nine species (126 now), and a Reaction of one pass a cell 216 (77 now).
+// and nine species (126 now), and a Reaction of one pass a cell 216 (89 now).
 template <bool NASA, class F>
 __device__ __forceinline__ bool fast_fits(const DevThermo *__restrict__ th, double top, double T, bool run,
                                           bool need_log, F body)
