@@ -142,7 +142,8 @@ inline int tile_faces(int dir, int shape)
 inline void sweep_grid(const Geom &g, int dir, int shape, long long launch, unsigned out[5])
 {
     const int TS = tile_faces(dir, shape), TW = 256 / TS;
-    auto tiles = [](int n, int most) { return (unsigned)((n + most - 1) / most); };
+    // (0 tiles of no cells, where a direction has none: the launch then fails)
+    auto tiles = [](int n, int most) { return most > 0 ? (unsigned)((n + most - 1) / most) : 0u; };
     const int inner = dir == 0 ? g.X_inner : (dir == 1 ? g.Y_inner : g.Z_inner);
     const unsigned along = tiles(inner, TS - 1), across = tiles(dir == 0 ? g.Y_inner * g.Z_inner : g.X_inner, TW);
     out[0] = dir == 0 ? along : across;
